@@ -9,7 +9,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIBPATH = os.path.join(_HERE, 'libmi355df.so')
-ABI_VERSION = 12
+ABI_VERSION = 13
 DTYPE_F64, DTYPE_F32 = 0, 1
 PREC_FP64 = 0
 PREC_FP32 = 1
@@ -31,6 +31,10 @@ _SIGS = {
     'mdf_get_j_noalloc': (I, [P, I, L, L, L, P, I, L, P, L, P, L, I, P]),
     'mdf_get_k_workspace': (SZ, [L, I, I, I, I, L]),
     'mdf_get_k': (I, [P, I, L, L, L, P, I, P, P, I, L, I, P, L, I, P, SZ, P]),
+    'mdf_pair_tiles_bytes': (SZ, [I]),
+    'mdf_build_pair_tiles': (I, [P, I, I, P, P, SZ, P]),
+    'mdf_get_k_tiles_workspace': (SZ, [L, I, I, I, I, L]),
+    'mdf_get_k_tiles': (I, [P, I, L, L, L, P, P, I, P, P, I, L, I, P, L, I, P, SZ, P]),
     'mdf_pack_dm': (I, [P, I, I, L, P, L, I, P, L, P]),
     'mdf_unpack_pairs': (I, [P, I, L, P, L, I, P, L, P]),
     'mdf_build_pair_map': (I, [P, L, I, P, P]),

@@ -29,8 +29,8 @@ class JKItem(ctypes.Structure):
     _fields_ = [('cderi', P), ('ld', ctypes.c_long), ('naux', ctypes.c_long),
                 ('npairs', ctypes.c_long), ('nao', ctypes.c_int), ('pair_map', P),
                 ('n_dm', ctypes.c_int), ('dm_pairs', P), ('rho', P), ('vj_pairs', P),
-                ('fl', P), ('fr', P), ('nocc', ctypes.c_int), ('vk', P), ('cderi_dtype', ctypes.c_int)]
-
+                ('fl', P), ('fr', P), ('nocc', ctypes.c_int), ('vk', P), ('cderi_dtype', ctypes.c_int),
+                ('pair_tiles', P)]
 
 
 class Entry:
@@ -43,12 +43,13 @@ class Entry:
     are allocated here unless given.
     """
 
-    def __init__(self, cderi, nao, n_dm, nocc, dm_pairs=None, fl=None, fr=None, pair_map=None):
+    def __init__(self, cderi, nao, n_dm, nocc, dm_pairs=None, fl=None, fr=None, pair_map=None, pair_tiles=None):
         t = _dev.torch()
         dev = cderi.device
         self.cderi, self.nao, self.n_dm, self.nocc = cderi, nao, n_dm, nocc
         self.naux, self.npairs = cderi.shape
         self.pair_map = pair_map
+        self.pair_tiles = pair_tiles      # the map's tiles (fastdf._PairLayout.tiles()), else made by the first plan
         self.dm_pairs = dm_pairs if dm_pairs is not None else \
             t.zeros((n_dm, self.npairs), dtype=t.float64, device=dev)
         self.fl = fl if fl is not None else t.zeros((n_dm, nao, nocc), dtype=t.float64, device=dev)
@@ -57,11 +58,19 @@ class Entry:
         self.vj_pairs = t.empty((n_dm, self.npairs), dtype=t.float64, device=dev)
         self.vk = t.empty((n_dm, nao, nao), dtype=t.float64, device=dev)
 
-    def item(self):
+    def tiles(self):
+        """The pair map's tiles, given or made here: the same ones a single
+        call's layout makes, so an item's K is the same alone."""
+        if self.pair_tiles is None and self.pair_map is not None:
+            self.pair_tiles = fastdf.PairTiles(self.pair_map, self.nao, self.npairs).buf
+        return self.pair_tiles
+
+    def item(self, with_k=True):
         p = lambda x: None if x is None else x.data_ptr()
         return JKItem(self.cderi.data_ptr(), self.cderi.stride(0), self.naux, self.npairs, self.nao,
                       p(self.pair_map), self.n_dm, p(self.dm_pairs), p(self.rho), p(self.vj_pairs),
-                      p(self.fl), p(self.fr), self.nocc, p(self.vk), fastdf._dtype_code(self.cderi))
+                      p(self.fl), p(self.fr), self.nocc, p(self.vk), fastdf._dtype_code(self.cderi),
+                      p(self.tiles()) if with_k else None)
 
     def signature(self):
         return (self.nao, self.naux, self.npairs, self.n_dm, self.nocc, self.fr is not None)
@@ -84,7 +93,7 @@ class GroupedJK:
         self.with_j, self.with_k = with_j, with_k
         self.precision = precision
         self.prec = fastdf.PRECISIONS[precision]
-        arr = (JKItem * max(len(self.entries), 1))(*[e.item() for e in self.entries])
+        arr = (JKItem * max(len(self.entries), 1))(*[e.item(with_k) for e in self.entries])
         self._arr = arr
         sig = (tuple(sorted(e.signature() for e in self.entries)), with_j, with_k, precision)
         if bn is None:
@@ -188,7 +197,7 @@ def batched_get_jk(dfobjs, dms_list, hermi=1, precision='fp64', work_limit=0):
         dms3 = _dev.to_device(dms).reshape(-1, nao, nao)
         fl, fr = fastdf.factorize_dm(dms, hermi)
         d = fastdf._sparse_dm(dms3, lay, hermi)
-        e = Entry(cderi, nao, dms3.shape[0], fl.shape[-1], dm_pairs=d, fl=fl, fr=fr, pair_map=lay.map)
+        e = Entry(cderi, nao, dms3.shape[0], fl.shape[-1], dm_pairs=d, fl=fl, fr=fr, pair_map=lay.map, pair_tiles=lay.tiles())
         e.layout = lay
         entries.append(e)
         shapes.append(tuple(np.shape(dms)))

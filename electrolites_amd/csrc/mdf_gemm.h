@@ -3,7 +3,7 @@
 // One workgroup (256 threads = 4 wavefronts as 2 x 2) computes a BM x BN
 // tile of C = sum_k A[m, k] B[k, n] over nk K-steps of BK = 16.  Operands are
 // staged through double-buffered LDS (A as As[k][m], B as Bs[k][n]) with the
-// next K-step's global loads held in registers while the current step's MFMAs
+// K-step after the next held in registers while the current step's MFMAs
 // run, so there is one barrier per K-step.  Loaders decide where a tile comes
 // from (packed triangle, row-major matrix, transformed block ...) and convert
 // to the engine's element type T on the way into LDS:
@@ -12,6 +12,7 @@
 //     using reg_t = ...;                      // register type (the source type)
 //     static constexpr int N;                 // elements per thread per K-step
 //     void load(int kt, reg_t (&r)[N]);       // global -> registers
+//     static constexpr int SWZ;               // swizzle of its LDS rows
 //     void store(const reg_t (&r)[N], T *lds, int pitch);   // convert -> LDS
 //   };
 //
@@ -60,6 +61,17 @@ struct Mfma<float> {
 
 __device__ __forceinline__ double4_t mfma16(double a, double b, double4_t c) { return Mfma<double>::mma(a, b, c); }
 
+// Row k of an operand's LDS tile may hold its elements permuted, element m at
+// m ^ swizzle<SWZ>(k), so that the stores of a loader whose lanes run along k
+// spread over the banks (the pitch, 32 banks modulo 64, keeps the reads free
+// of conflicts either way).  SWZ, the loader's: 0 none; 1 lanes of 16 single
+// k by 4 rows; 2 of 8 k pairs (16 bytes of double) by 8 rows; 3 of 4 k
+// quadruples (16 bytes of float) by 16 rows.
+template <int SWZ>
+__device__ __forceinline__ constexpr int swizzle(int k) {
+    return SWZ == 1 ? ((k >> 1) & 3) << 2 : SWZ == 2 ? ((k >> 1) & 3) << 3 : SWZ == 3 ? ((k >> 2) & 3) << 4 : 0;
+}
+
 // A workgroup of WGM x WGN wavefronts (64 WGM WGN threads) computes a
 // BM x BN tile; wavefront w owns sub-tile (w % WGM, w / WGM).
 template <int BM, int BN, int WGM = 2, int WGN = 2>
@@ -92,50 +104,77 @@ __device__ __forceinline__ void gemm_mainloop(LA &la, LB &lb, int nk, T *lds,
                                      Acc<TileShape<BM, BN, WGM, WGN>::MI, TileShape<BM, BN, WGM, WGN>::NI, T> &acc) {
     using S = TileShape<BM, BN, WGM, WGN>;
     constexpr int SA = G_BK * S::PA, SB = G_BK * S::PB;
+    static_assert(LA::SWZ < 2 || (S::MI & (S::MI - 1)) == 0, "a swizzled operand has 2^n blocks a wavefront");
+    static_assert(LB::SWZ < 2 || (S::NI & (S::NI - 1)) == 0, "a swizzled operand has 2^n blocks a wavefront");
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int wm = wave % WGM, wn = wave / WGM;
     T *const Bbase = lds + 2 * SA;
-    const MDF_LDS T *Ar = (const MDF_LDS T *)(lds + wm * S::WM + (lane & 15));
-    const MDF_LDS T *Br = (const MDF_LDS T *)(Bbase + wn * S::WN + (lane & 15));
+    const MDF_LDS T *const Ar = (const MDF_LDS T *)lds, *const Br = (const MDF_LDS T *)Bbase;
+    const int q4 = lane >> 4;
+    const int la15 = (lane & 15) ^ swizzle<LA::SWZ>(q4), lb15 = (lane & 15) ^ swizzle<LB::SWZ>(q4);
     typename LA::reg_t ra[LA::N];
     typename LB::reg_t rb[LB::N];
     if (nk <= 0) return;
+    T a[2][S::MI], b[2][S::NI];
+    auto read = [&](int buf, int kq, int s) {
+        // the swizzle of k = 4 kq + q4 is that of q4 (lane bits) and of 4 kq
+        // (a constant here: lane bits below 16, MFMA blocks above)
+        const int kk = kq * 4 + q4, xa = swizzle<LA::SWZ>(kq * 4), xb = swizzle<LB::SWZ>(kq * 4);
+        const int ba = xa >> 4, bb = xb >> 4;
+        const MDF_LDS T *A = Ar + buf * SA + kk * S::PA + (wm ^ (ba / S::MI)) * S::WM + (la15 ^ (xa & 15));
+        const MDF_LDS T *B = Br + buf * SB + kk * S::PB + (wn ^ (bb / S::NI)) * S::WN + (lb15 ^ (xb & 15));
+#pragma unroll
+        for (int mi = 0; mi < S::MI; mi++) a[s][mi] = A[(ba ? mi ^ (ba % S::MI) : mi) * 16];
+#pragma unroll
+        for (int ni = 0; ni < S::NI; ni++) b[s][ni] = B[(bb ? ni ^ (bb % S::NI) : ni) * 16];
+    };
     la.load(0, ra);
     lb.load(0, rb);
     la.store(ra, lds, S::PA);
     lb.store(rb, Bbase, S::PB);
+    if (nk > 1) {
+        la.load(1, ra);
+        lb.load(1, rb);
+    }
     __syncthreads();
+    read(0, 0, 0);
     for (int kt = 0; kt < nk; kt++) {
         const int cur = kt & 1;
         const bool more = kt + 1 < nk;
-        if (more) {
-            la.load(kt + 1, ra);
-            lb.load(kt + 1, rb);
-        }
-        const MDF_LDS T *A = Ar + cur * SA;
-        const MDF_LDS T *B = Br + cur * SB;
 #pragma unroll
         for (int kq = 0; kq < G_BK / 4; kq++) {
-            const int kk = kq * 4 + (lane >> 4);
-            T a[S::MI], b[S::NI];
-#pragma unroll
-            for (int mi = 0; mi < S::MI; mi++) a[mi] = A[kk * S::PA + mi * 16];
-#pragma unroll
-            for (int ni = 0; ni < S::NI; ni++) b[ni] = B[kk * S::PB + ni * 16];
+            // the operands of the next MFMA group are read before this
+            // group's MFMAs issue, so they arrive under them; the step's
+            // barrier stands before its last group, whose operands are in
+            // registers: the next step's first reads run under that group
+            if (kq < G_BK / 4 - 1) {
+                read(cur, kq + 1, (kq + 1) & 1);
+            } else if (more) {
+                __syncthreads();
+                read(cur ^ 1, 0, (kq + 1) & 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int mi = 0; mi < S::MI; mi++)
 #pragma unroll
-                for (int ni = 0; ni < S::NI; ni++) acc.v[mi][ni] = Mfma<T>::mma(a[mi], b[ni], acc.v[mi][ni]);
-            // the next K-step's tile goes into the other buffer (read by no
-            // wave since the last barrier) halfway through this step's MFMAs,
-            // so the stores overlap the matrix pipe instead of following it
+                for (int ni = 0; ni < S::NI; ni++)
+                    acc.v[mi][ni] = Mfma<T>::mma(a[kq & 1][mi], b[kq & 1][ni], acc.v[mi][ni]);
+            __builtin_amdgcn_sched_barrier(0);
+            // halfway through a step's MFMAs the next step's tile goes into
+            // the other buffer (read by no wave since the last barrier) and
+            // the loads of the step after it start: they have a whole step,
+            // from here to the next one's middle, to arrive
             if (kq == G_BK / 8 - 1 && more) {
                 la.store(ra, lds + (cur ^ 1) * SA, S::PA);
                 lb.store(rb, Bbase + (cur ^ 1) * SB, S::PB);
+                if (kt + 2 < nk) {
+                    la.load(kt + 2, ra);
+                    lb.load(kt + 2, rb);
+                }
             }
         }
-        __syncthreads();
     }
+    __syncthreads();        // the LDS may be reused by the caller
 }
 
 // Visits every accumulator element with its tile-local (row, col); the
@@ -165,87 +204,104 @@ __device__ __forceinline__ void gemm_epilogue(const Acc<TileShape<BM, BN>::MI, T
 }
 
 // ---------------------------------------------------------------- loaders
-// Row-major matrix M[row][k] (k contiguous, element type S) as the A or B
-// operand: tile rows r0 .. r0+R-1, K-step kt covers k = kt*BK .. +BK-1.
-// Out-of-range reads 0.
+// Two or four neighbouring elements loaded at once, at the alignment of one.
+template <typename S, int N>
+struct alignas(sizeof(S)) Piece {
+    S v[N];
+};
+
+// Row-major matrix M[row][k] (k contiguous, element type Src) as the A or B
+// operand: tile rows r0 .. r0+R-1, K-step kt covers k = kt*BK .. +BK-1, out of
+// range k read 0.  Eight lanes take the 16 k of one row in pairs, so a load
+// instruction reads whole 128-byte rows (a thread per 8 k of a row touched
+// every line four times: 3.2 times the cache accesses in K's step 2).
+// Rows past the last repeat it (their results are not used).
 template <int R, typename T = double, typename Src = double, int THREADS = G_THREADS>
 struct RowsLoader {
     using reg_t = Src;
-    static constexpr int N = R * G_BK / THREADS;
-    static_assert(N >= 1 && G_BK % N == 0 && (THREADS / (G_BK / N)) == R, "RowsLoader shape");
-    const Src *base;      // &M[0][0]
-    long ld;              // row stride
-    int r0, nrows, k0, kmax;
-    __device__ __forceinline__ void load(int kt, Src (&r)[N]) const {
-        const int t = threadIdx.x;
-        const int row = r0 + t / (G_BK / N);
-        const int kb = k0 + kt * G_BK + (t % (G_BK / N)) * N;
-        if (row < nrows && kb + N <= kmax) {
-            // the whole chunk is in range: plain loads, no per-element select
-            const Src *src = base + (long)row * ld + kb;
+    static constexpr int N = R * G_BK / THREADS, Q = N / 2;
+    static constexpr int RPP = THREADS / 8;              // rows per piece
+    static constexpr int SWZ = 2;
+    static_assert(Q >= 1 && Q * RPP == R, "RowsLoader shape");
+    const Src *p[Q];          // this thread's rows, at k0
+    int nk;                   // k in range from there
+    __device__ __forceinline__ RowsLoader(const Src *base, long ld, int r0, int nrows, int k0, int kmax) {
 #pragma unroll
-            for (int v = 0; v < N; v++) r[v] = src[v];
+        for (int q = 0; q < Q; q++)
+            p[q] = base + (long)min(r0 + (int)(threadIdx.x >> 3) + q * RPP, nrows - 1) * ld + k0;
+        nk = kmax - k0;
+    }
+    __device__ __forceinline__ void load(int kt, Src (&r)[N]) const {
+        const int k = kt * G_BK + 2 * (int)(threadIdx.x & 7);
+        if ((kt + 1) * G_BK <= nk) {
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                const Piece<Src, 2> x = *(const Piece<Src, 2> *)(p[q] + k);
+                r[2 * q] = x.v[0];
+                r[2 * q + 1] = x.v[1];
+            }
             return;
         }
-        // edge: unconditional loads at clamped (in-bounds) addresses, the
-        // out-of-range elements selected to zero
-        const Src *src = base + (long)min(row, nrows - 1) * ld;
 #pragma unroll
-        for (int v = 0; v < N; v++) {
-            const Src x = src[min(kb + v, kmax - 1)];
-            r[v] = (row < nrows && kb + v < kmax) ? x : (Src)0;
-        }
+        for (int q = 0; q < Q; q++)
+#pragma unroll
+            for (int v = 0; v < 2; v++) {
+                const Src x = p[q][min(k + v, nk - 1)];
+                r[2 * q + v] = k + v < nk ? x : (Src)0;
+            }
     }
     __device__ __forceinline__ void store(const Src (&r)[N], T *lds, int pitch) const {
-        const int t = threadIdx.x;
-        const int row = t / (G_BK / N);
-        const int kb = (t % (G_BK / N)) * N;
+        const int k = 2 * (threadIdx.x & 7);
+        T *d = lds + k * pitch + ((int)(threadIdx.x >> 3) ^ swizzle<SWZ>(k));
 #pragma unroll
-        for (int v = 0; v < N; v++) lds[(kb + v) * pitch + row] = (T)r[v];
+        for (int q = 0; q < Q; q++) {
+            d[q * RPP] = (T)r[2 * q];
+            d[q * RPP + pitch] = (T)r[2 * q + 1];
+        }
     }
 };
 
 // Row-major matrix M[k][col] (col contiguous) as the B operand: tile columns
-// c0 .. c0+C-1.
+// c0 .. c0+C-1.  The lanes of a k row take column pairs at a stride of the
+// whole row of lanes, so loads and LDS stores run along rows.  Columns past
+// the last repeat one in range (their results are not used).
 template <int C, typename T = double, typename Src = double, int THREADS = G_THREADS>
 struct ColsLoader {
     using reg_t = Src;
-    static constexpr int N = C * G_BK / THREADS;
-    const Src *base;
+    static constexpr int N = C * G_BK / THREADS, Q = N / 2;
+    static constexpr int TPR = THREADS / G_BK;           // threads per k row
+    static constexpr int SWZ = 0;
+    static_assert(Q >= 1 && Q * 2 * TPR == C, "ColsLoader shape");
+    const Src *base;          // row k0
     long ld;
-    int c0, ncols, k0, kmax;
+    int c, ncols, nk;
+    __device__ __forceinline__ ColsLoader(const Src *b, long ld_, int c0, int ncols_, int k0, int kmax)
+        : base(b + (long)k0 * ld_), ld(ld_), c(c0 + 2 * (int)(threadIdx.x % TPR)), ncols(ncols_), nk(kmax - k0) {}
     __device__ __forceinline__ void load(int kt, Src (&r)[N]) const {
-        const int t = threadIdx.x;
-        // each thread takes N consecutive columns of one k row
-        constexpr int TPR = C / N;              // threads per k row
-        const int kk = t / TPR;
-        const int cb = c0 + (t % TPR) * N;
-        const int k = k0 + kt * G_BK + kk;
-        if (kk < G_BK && k < kmax && cb + N <= ncols) {
-            // the whole chunk is in range: plain loads, no per-element select
-            const Src *src = base + (long)k * ld + cb;
+        const int k = kt * G_BK + (int)(threadIdx.x / TPR);
+        const int cl = c - 2 * (int)(threadIdx.x % TPR);          // the tile's first column
+        if ((kt + 1) * G_BK <= nk && cl + C <= ncols) {
+            const Src *src = base + (long)k * ld + c;
 #pragma unroll
-            for (int v = 0; v < N; v++) r[v] = src[v];
+            for (int q = 0; q < Q; q++) {
+                const Piece<Src, 2> x = *(const Piece<Src, 2> *)(src + q * 2 * TPR);
+                r[2 * q] = x.v[0];
+                r[2 * q + 1] = x.v[1];
+            }
             return;
         }
-        // edge: unconditional loads at clamped (in-bounds) addresses, the
-        // out-of-range elements selected to zero
-        const Src *src = base + (long)min(k, kmax - 1) * ld;
+        const Src *src = base + (long)min(k, nk - 1) * ld;
 #pragma unroll
-        for (int v = 0; v < N; v++) {
-            const Src x = src[min(cb + v, ncols - 1)];
-            r[v] = (kk < G_BK && k < kmax && cb + v < ncols) ? x : (Src)0;
+        for (int e = 0; e < N; e++) {
+            const Src x = src[min(c + (e >> 1) * 2 * TPR + (e & 1), ncols - 1)];
+            r[e] = k < nk ? x : (Src)0;
         }
     }
     __device__ __forceinline__ void store(const Src (&r)[N], T *lds, int pitch) const {
-        const int t = threadIdx.x;
-        constexpr int TPR = C / N;
-        const int kk = t / TPR;
-        const int cb = (t % TPR) * N;
-        if (kk < G_BK) {
+        struct alignas(2 * sizeof(T)) Pair { T x, y; };
+        T *d = lds + (threadIdx.x / TPR) * pitch + 2 * (threadIdx.x % TPR);
 #pragma unroll
-            for (int v = 0; v < N; v++) lds[kk * pitch + cb + v] = (T)r[v];
-        }
+        for (int q = 0; q < Q; q++) *(Pair *)(d + q * 2 * TPR) = Pair{(T)r[2 * q], (T)r[2 * q + 1]};
     }
 };
 

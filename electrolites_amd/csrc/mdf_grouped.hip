@@ -61,22 +61,27 @@ struct GKItem {
     void *rl, *rr;          // transformed blocks (T), nL aux rows each
     double *part;           // ksplit x nao x nao
     long nL;                // aux rows per pass
-    int nao, nocc, ksplit, ntile, vec;
+    int nao, nocc, ksplit, ntile;
     // split-BF16 (prec 2): workspace offsets of [side][FT hi, FT lo, R hi, R lo]
     void *b3[2][4];
     long ldr, ldft;         // R row stride (FP64/FP32: kcore::r_ld; split-BF16: a multiple of 32), FT row stride
     int bn3;                // split-BF16 step-1 tile width (kb3::pick_bn(ldr))
     int bn1;                // FP64/FP32 step-1 tile width (the plan's bn, or kcore::pick_bn(nocc))
+    const void *tiles;      // FP64/FP32: the pair map's tiles, or NULL
+    void *fp[2];            // and the packed factors (rows of ldp)
+    long ldp;
+    size_t packb;           // bytes of one packed factor (host)
 };
 
 struct Tile {
     int item, a, b, c;
 };
 
-// A launch of the K sequence: kind 0 = factor split (prec 2), 1 = step 1,
-// 2 = step 2, 3 = finalize, over tiles [start, start + count) of that kind's
-// table.  Split-BF16 step-1 launches hold items of one tile width `bn` and
-// one `mapped` flag each.
+// A launch of the K sequence: kind 0 = factor split (prec 2) or packing (items
+// with pair tiles), 1 = step 1, 2 = step 2, 3 = finalize, over tiles [start,
+// start + count) of that kind's table.  Step-1 launches hold items of one tile
+// width `bn` and one `mapped` flag each (split-BF16: a pair map; else: pair
+// tiles).
 struct Phase {
     int kind;
     long start, count;
@@ -196,6 +201,39 @@ __global__ __launch_bounds__(kcore::Step1Shape<BN>::THREADS) void gk_step1(const
     }
 }
 
+// Step 1 of the items with pair tiles.
+template <int BN, typename T, typename Src>
+__global__ __launch_bounds__(kcore::Step1Shape<BN>::THREADS, 2) void gk_step1_pairs(const GKItem *items,
+                                                                                const Tile *tab, long n,
+                                                                                char *work) {
+    __shared__ T lds[kcore::Step1Shape<BN>::S::LDS_ELEMS];
+    XCD_RUN_LOOP(t, n) {
+        const Tile e = tab[t];              // (item, first of 8 aux rows, group, k-tile | right-factor flag << 16)
+        const GKItem &it = items[e.item];
+        const int side = e.c >> 16, ktile = e.c & 0xffff;
+        const long lb = e.a % it.nL;        // row within the pass
+        const long end = min(e.a - lb + it.nL, it.naux);
+        T *R = (T *)(work + (size_t)(side ? it.rr : it.rl)) + lb * it.nao * it.ldr;
+        kcore::step1_pairs_tile<BN, T, Src, false>((const Src *)it.cderi + (long)e.a * it.ld, it.ld,
+                                                   (int)min((long)tiles::NL, end - e.a),
+                                                   tiles::view(it.tiles, it.nao), e.b,
+                                                   (const T *)(work + (size_t)it.fp[side]), (unsigned)it.ldp, it.nocc,
+                                                   R, it.ldr, (long)it.nao * it.ldr, ktile * BN, lds);
+        __syncthreads();
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void gk_pack_factor(const GKItem *items, const Tile *tab, long n, char *work) {
+    for (long t = blockIdx.x; t < n; t += gridDim.x) {
+        const Tile e = tab[t];              // (item, chunk, side)
+        const GKItem &it = items[e.item];
+        const long e0 = (long)e.a * 1024, e1 = min(e0 + 1024, (long)(it.nao + 1) * it.ldp);
+        tiles::pack_factor_range(e.b ? it.fr : it.fl, it.nocc, it.nao, it.nocc, (T *)(work + (size_t)it.fp[e.b]),
+                                 it.ldp, e0, e1);
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(G_THREADS, 2) void gk_step2(const GKItem *items, const Tile *tiles, long n,
                                                          char *work) {
@@ -218,12 +256,8 @@ __global__ __launch_bounds__(G_THREADS, 2) void gk_step2(const GKItem *items, co
         const T *rl = (const T *)(work + (size_t)it.rl);
         const T *rr = it.fr ? (const T *)(work + (size_t)it.rr) : rl;
         double *o = (double *)(work + (size_t)it.part) + (long)e.b * it.nao * it.nao;
-        if (it.vec)
-            kcore::step2_tile<true, T>(rl, rr, it.nao, it.nocc, it.ldr, (long)it.nao * it.ldr, ti * kcore::S2_B,
-                                       tj * kcore::S2_B, s0, s1, o, e.c > 0, lds);
-        else
-            kcore::step2_tile<false, T>(rl, rr, it.nao, it.nocc, it.ldr, (long)it.nao * it.ldr, ti * kcore::S2_B,
-                                        tj * kcore::S2_B, s0, s1, o, e.c > 0, lds);
+        kcore::step2_tile<T>(rl, rr, it.nao, it.nocc, it.ldr, (long)it.nao * it.ldr, ti * kcore::S2_B,
+                             tj * kcore::S2_B, s0, s1, o, e.c > 0, lds);
         __syncthreads();
     }
 }
@@ -395,7 +429,17 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
                 g.nao = x.nao; g.nocc = x.nocc; g.ksplit = kp.ksplit; g.ntile = kp.ntile;
                 g.nL = kp.nL;
                 g.bn1 = bn ? bn : kcore::pick_bn(x.nocc);
-                g.vec = 1;             // R rows padded to whole 16-byte vectors (kcore::r_ld)
+                if (!b3 && x.pair_tiles) {
+                    if (x.nao > tiles::MAX_NAO || x.npairs >= (1L << 29)) {
+                        set_error("mdf_grouped_plan_create: item %d is beyond what pair tiles hold", m);
+                        delete p;
+                        return MDF_EINVAL;
+                    }
+                    g.tiles = x.pair_tiles;
+                    kp.bn = g.bn1;
+                    g.ldp = kcore::pack_ld(kp, x.nocc);
+                    g.packb = align_up(kcore::pack_words(kp, x.nao, x.nocc) * elem, 256);
+                }
                 // workspace offsets are assigned per wave below; keep the sizes
                 if (b3) {
                     const kcore::kb3::Layout y = kcore::kb3::layout(x.nao, x.nocc, kp.nL, kp.ksplit, two);
@@ -423,7 +467,7 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
         size_t used = 0, w1 = w0;
         while (w1 < p->hk.size()) {
             const GKItem &g = p->hk[w1];
-            const size_t need = (g.fr ? 2 : 1) * (size_t)g.rl + (size_t)g.part;
+            const size_t need = (g.fr ? 2 : 1) * ((size_t)g.rl + g.packb) + (size_t)g.part;
             if (w1 > w0 && used + need > work_limit) break;
             used += need;
             w1++;
@@ -445,6 +489,10 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
                 g.rl = (void *)o; o += rb;
                 if (g.fr) { g.rr = (void *)o; o += rb; }
                 g.part = (double *)o; o += pb;
+                for (int side = 0; side < (g.fr ? 2 : 1); side++) {
+                    g.fp[side] = (void *)o;
+                    o += g.packb;
+                }
             }
             maxpass = std::max(maxpass, cdiv(g.naux, g.nL));
         }
@@ -459,22 +507,42 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
             p->kphases.push_back({0, s0, (long)k0.size() - s0, 0, 0});
         }
         const bool b3 = prec == MDF_PREC_BF16X3;
+        if (!b3) {
+            const long s0 = k0.size();
+            for (size_t i = w0; i < w1; i++) {
+                const GKItem &g = p->hk[i];
+                if (!g.tiles) continue;
+                for (int side = 0; side < (g.fr ? 2 : 1); side++)
+                    for (long e = 0; e < cdiv((long)(g.nao + 1) * g.ldp, 1024L); e++)
+                        k0.push_back({(int)i, (int)e, side, 0});
+            }
+            p->kphases.push_back({0, s0, (long)k0.size() - s0, 0, 0});
+        }
         for (long b = 0; b < maxpass; b++) {
-          // one step-1 launch per tile width (and, for split-BF16, per pair-map flag)
-          for (int cls = 0; cls < (b3 ? 8 : 6); cls++) {
+          // one step-1 launch per tile width and per pair-map (split-BF16) or
+          // pair-tiles flag
+          for (int cls = 0; cls < (b3 ? 8 : 12); cls++) {
             static const int kBN3[4] = {128, 192, 256, 320};
             static const int kBN1[6] = {64, 128, 160, 192, 256, 320};
-            const int mp = b3 ? cls / 4 : 0, cbn = b3 ? kBN3[cls % 4] : kBN1[cls];
+            const int mp = cls / (b3 ? 4 : 6), cbn = b3 ? kBN3[cls % 4] : kBN1[cls % 6];
             const long s1 = k1.size();
             for (size_t i = w0; i < w1; i++) {
                 const GKItem &g = p->hk[i];
                 const long L0 = b * g.nL;
                 if (L0 >= g.naux) continue;
                 if (b3 && ((g.pmap != nullptr) != (mp == 1) || g.bn3 != cbn)) continue;
-                if (!b3 && g.bn1 != cbn) continue;
+                if (!b3 && ((g.tiles != nullptr) != (mp == 1) || g.bn1 != cbn)) continue;
                 const long L1 = std::min(L0 + g.nL, g.naux);
                 const int nkt = b3 ? (int)cdiv(g.ldr, (long)cbn) : (int)cdiv(g.nocc, cbn);
                 const int nit = (int)cdiv(g.nao, 128);
+                if (!b3 && mp) {
+                    // the groups of one aux block together, the longest first
+                    for (int side = 0; side < (g.fr ? 2 : 1); side++)
+                        for (long L = L0; L < L1; L += tiles::NL)
+                            for (int it = tiles::groups(g.nao) - 1; it >= 0; it--)
+                                for (int kt = 0; kt < nkt; kt++) k1.push_back({(int)i, (int)L, it, kt | (side << 16)});
+                    continue;
+                }
                 for (int side = 0; side < (g.fr ? 2 : 1); side++)
                     for (long L = L0; L < L1; L++)
                         for (int it = 0; it < nit; it++)
@@ -613,21 +681,25 @@ static void launch_gj(int c, int dtype, const GJItem *items, const Tile *tiles, 
 }
 
 template <int BN, typename Src>
-static void launch_gk1_s(const mdf_grouped_plan *p, const Tile *tiles, long n, char *w, hipStream_t st) {
+static void launch_gk1_s(const mdf_grouped_plan *p, const Tile *tiles, long n, int pairs, char *w, hipStream_t st) {
     const int g = persistent_grid(n, BN >= 192 ? 1 : 2);
     const dim3 b(kcore::Step1Shape<BN>::THREADS);
-    if (p->prec == MDF_PREC_FP32)
+    if (pairs && p->prec == MDF_PREC_FP32)
+        hipLaunchKernelGGL((gk_step1_pairs<BN, float, Src>), dim3(g), b, 0, st, p->kitems, tiles, n, w);
+    else if (pairs)
+        hipLaunchKernelGGL((gk_step1_pairs<BN, double, Src>), dim3(g), b, 0, st, p->kitems, tiles, n, w);
+    else if (p->prec == MDF_PREC_FP32)
         hipLaunchKernelGGL((gk_step1<BN, float, Src>), dim3(g), b, 0, st, p->kitems, tiles, n, w);
     else
         hipLaunchKernelGGL((gk_step1<BN, double, Src>), dim3(g), b, 0, st, p->kitems, tiles, n, w);
 }
 
 template <int BN>
-static void launch_gk1(const mdf_grouped_plan *p, const Tile *tiles, long n, char *w, hipStream_t st) {
+static void launch_gk1(const mdf_grouped_plan *p, const Tile *tiles, long n, int pairs, char *w, hipStream_t st) {
     if (p->dtype == MDF_DTYPE_F32)
-        launch_gk1_s<BN, float>(p, tiles, n, w, st);
+        launch_gk1_s<BN, float>(p, tiles, n, pairs, w, st);
     else
-        launch_gk1_s<BN, double>(p, tiles, n, w, st);
+        launch_gk1_s<BN, double>(p, tiles, n, pairs, w, st);
 }
 
 template <bool MAPPED, int BN>
@@ -673,7 +745,16 @@ extern "C" int mdf_grouped_jk(const mdf_grouped_plan *p, void *work, size_t work
         const bool b3 = p->prec == MDF_PREC_BF16X3;
         for (const Phase &ph : p->kphases) {
             if (ph.count == 0) continue;
-            if (ph.kind == 0) {
+            if (ph.kind == 0 && !b3) {
+                const dim3 g0(persistent_grid(ph.count, 4));
+                if (p->prec == MDF_PREC_FP32)
+                    hipLaunchKernelGGL(gk_pack_factor<float>, g0, dim3(256), 0, st, p->kitems, p->k0 + ph.start,
+                                       ph.count, w);
+                else
+                    hipLaunchKernelGGL(gk_pack_factor<double>, g0, dim3(256), 0, st, p->kitems, p->k0 + ph.start,
+                                       ph.count, w);
+                MDF_LAUNCHED("gk_pack_factor");
+            } else if (ph.kind == 0) {
                 hipLaunchKernelGGL(gk_split_ft, dim3(persistent_grid(ph.count, 4)), dim3(256), 0, st, p->kitems,
                                    p->k0 + ph.start, ph.count, w);
                 MDF_LAUNCHED("gk_split_ft");
@@ -697,12 +778,12 @@ extern "C" int mdf_grouped_jk(const mdf_grouped_plan *p, void *work, size_t work
             } else if (ph.kind == 1) {
                 const Tile *t = p->k1 + ph.start;
                 switch (ph.bn) {
-                case 320: launch_gk1<320>(p, t, ph.count, w, st); break;
-                case 256: launch_gk1<256>(p, t, ph.count, w, st); break;
-                case 192: launch_gk1<192>(p, t, ph.count, w, st); break;
-                case 160: launch_gk1<160>(p, t, ph.count, w, st); break;
-                case 128: launch_gk1<128>(p, t, ph.count, w, st); break;
-                default: launch_gk1<64>(p, t, ph.count, w, st); break;
+                case 320: launch_gk1<320>(p, t, ph.count, ph.mapped, w, st); break;
+                case 256: launch_gk1<256>(p, t, ph.count, ph.mapped, w, st); break;
+                case 192: launch_gk1<192>(p, t, ph.count, ph.mapped, w, st); break;
+                case 160: launch_gk1<160>(p, t, ph.count, ph.mapped, w, st); break;
+                case 128: launch_gk1<128>(p, t, ph.count, ph.mapped, w, st); break;
+                default: launch_gk1<64>(p, t, ph.count, ph.mapped, w, st); break;
                 }
                 MDF_LAUNCHED("gk_step1");
             } else if (ph.kind == 2) {

@@ -47,8 +47,34 @@ __global__ __launch_bounds__(Step1Shape<BN>::THREADS) void k_step1(
                                         kt * BN, lds);
 }
 
+// The pair-tile step 1: 1-D grid of round_xcd(nkt * ngroup * blocks of 8 aux
+// rows) workgroups in XCD order, k-tile fastest, then group (the longest, the
+// last placed, first), then aux rows: the groups of one aux block read the
+// same cderi rows.
+template <int BN, typename T, typename Src, bool HALVES>
+__global__ __launch_bounds__(Step1Shape<BN>::THREADS, 2) void k_step1_pairs(
+    const Src *__restrict__ cderi, long ld, int nL, tiles::View tv, const T *__restrict__ fp, unsigned ldp, int nocc,
+    T *__restrict__ R, long ldr, long strideL, int nkt, long ntiles) {
+    __shared__ T lds[Step1Shape<BN>::S::LDS_ELEMS];
+    const long x = xcd_tile(blockIdx.x, gridDim.x);
+    if (x >= ntiles) return;
+    const int kt = (int)(x % nkt);
+    const long y = x / nkt;
+    const int g = tv.ngroup - 1 - (int)(y % tv.ngroup);
+    const long L = y / tv.ngroup * tiles::NL;
+    step1_pairs_tile<BN, T, Src, HALVES>(cderi + L * ld, ld, (int)min((long)tiles::NL, nL - L), tv, g, fp, ldp, nocc,
+                                         R + L * strideL, ldr, strideL, kt * BN, lds);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_pack_factor(const double *__restrict__ F, long ldf, int nao, int nocc,
+                                                     T *__restrict__ fp, long ldp) {
+    const long e0 = (long)blockIdx.x * 1024;
+    tiles::pack_factor_range(F, ldf, nao, nocc, fp, ldp, e0, min(e0 + 1024, (long)(nao + 1) * ldp));
+}
+
 // 1-D grid of ntiles_grid * ksplit workgroups, (tile, split) by step2_coords.
-template <bool SYM, bool VEC, typename T>
+template <bool SYM, typename T>
 __global__ __launch_bounds__(G_THREADS, 2) void k_step2(
     const T *__restrict__ Rl, const T *__restrict__ Rr, int nao, int nocc,
     long ldr, long strideL, int nL, int ntile, int ntiles_grid, int ksplit, double *__restrict__ part,
@@ -65,7 +91,7 @@ __global__ __launch_bounds__(G_THREADS, 2) void k_step2(
     const int kchunks = (nocc + G_BK - 1) / G_BK;
     const long nsteps = (long)nL * kchunks;
     const long s0 = nsteps * split / ksplit, s1 = nsteps * (split + 1) / ksplit;
-    step2_tile<VEC, T>(Rl, Rr, nao, nocc, ldr, strideL, ti * S2_B, tj * S2_B, s0, s1,
+    step2_tile<T>(Rl, Rr, nao, nocc, ldr, strideL, ti * S2_B, tj * S2_B, s0, s1,
                        part + (long)split * part_stride, beta, lds);
 }
 
@@ -162,45 +188,84 @@ int step1(const KPlan &p, int nL, hipStream_t st, const Src *blk, long ld, const
     return MDF_OK;
 }
 
+template <int BN, typename T, typename Src, bool HALVES>
+void launch_step1_pairs(int nL, hipStream_t st, const Src *blk, long ld, const tiles::View &tv, const T *fp,
+                        unsigned ldp, int nocc, T *r, long ldr, long strideL) {
+    const int nkt = (int)cdiv(nocc, BN);
+    const long ntiles = (long)nkt * tv.ngroup * cdiv(nL, tiles::NL);
+    hipLaunchKernelGGL((k_step1_pairs<BN, T, Src, HALVES>), dim3((unsigned)round_xcd(ntiles)),
+                       dim3(Step1Shape<BN>::THREADS), 0, st, blk, ld, nL, tv, fp, ldp, nocc, r, ldr, strideL, nkt,
+                       ntiles);
+}
+
+template <typename T, typename Src, bool HALVES = false>
+int step1_pairs(const KPlan &p, int nL, hipStream_t st, const Src *blk, long ld, const tiles::View &tv, const T *fp,
+                int nocc, T *r, long ldr, long strideL) {
+    const unsigned ldp = pack_ld(p, nocc);
+    switch (p.bn) {
+    case 320: launch_step1_pairs<320, T, Src, HALVES>(nL, st, blk, ld, tv, fp, ldp, nocc, r, ldr, strideL); break;
+    case 256: launch_step1_pairs<256, T, Src, HALVES>(nL, st, blk, ld, tv, fp, ldp, nocc, r, ldr, strideL); break;
+    case 192: launch_step1_pairs<192, T, Src, HALVES>(nL, st, blk, ld, tv, fp, ldp, nocc, r, ldr, strideL); break;
+    case 160: launch_step1_pairs<160, T, Src, HALVES>(nL, st, blk, ld, tv, fp, ldp, nocc, r, ldr, strideL); break;
+    case 128: launch_step1_pairs<128, T, Src, HALVES>(nL, st, blk, ld, tv, fp, ldp, nocc, r, ldr, strideL); break;
+    default: launch_step1_pairs<64, T, Src, HALVES>(nL, st, blk, ld, tv, fp, ldp, nocc, r, ldr, strideL); break;
+    }
+    MDF_LAUNCHED("k_step1_pairs");
+    return MDF_OK;
+}
+
+template <typename T>
+int pack_factor(const KPlan &p, hipStream_t st, const double *f, long ldf, int nao, int nocc, T *fp) {
+    const long n = (long)pack_words(p, nao, nocc);
+    hipLaunchKernelGGL(k_pack_factor<T>, dim3((unsigned)cdiv(n, 1024L)), dim3(256), 0, st, f, ldf, nao, nocc, fp,
+                       (long)pack_ld(p, nocc));
+    MDF_LAUNCHED("k_pack_factor");
+    return MDF_OK;
+}
+
 template <typename T>
 int step2(const KPlan &p, int nL, bool two, hipStream_t st, const T *rl, const T *rr, int nao, int nocc,
           long ldr, long strideL, double *part, long part_stride, int beta) {
     const dim3 g2((unsigned)((long)p.ntiles_grid * p.ksplit));
-    const bool vec = (ldr % (16 / (long)sizeof(T)) == 0) && ((uintptr_t)rl % 16 == 0) && ((uintptr_t)rr % 16 == 0);
-    if (two && vec)
-        hipLaunchKernelGGL((k_step2<false, true, T>), g2, dim3(G_THREADS), 0, st, rl, rr, nao, nocc, ldr,
-                           strideL, nL, p.ntile, p.ntiles_grid, p.ksplit, part, part_stride, beta);
-    else if (two)
-        hipLaunchKernelGGL((k_step2<false, false, T>), g2, dim3(G_THREADS), 0, st, rl, rr, nao, nocc, ldr,
-                           strideL, nL, p.ntile, p.ntiles_grid, p.ksplit, part, part_stride, beta);
-    else if (vec)
-        hipLaunchKernelGGL((k_step2<true, true, T>), g2, dim3(G_THREADS), 0, st, rl, rl, nao, nocc, ldr,
-                           strideL, nL, p.ntile, p.ntiles_grid, p.ksplit, part, part_stride, beta);
+    if (two)
+        hipLaunchKernelGGL((k_step2<false, T>), g2, dim3(G_THREADS), 0, st, rl, rr, nao, nocc, ldr, strideL, nL,
+                           p.ntile, p.ntiles_grid, p.ksplit, part, part_stride, beta);
     else
-        hipLaunchKernelGGL((k_step2<true, false, T>), g2, dim3(G_THREADS), 0, st, rl, rl, nao, nocc, ldr,
-                           strideL, nL, p.ntile, p.ntiles_grid, p.ksplit, part, part_stride, beta);
+        hipLaunchKernelGGL((k_step2<true, T>), g2, dim3(G_THREADS), 0, st, rl, rl, nao, nocc, ldr, strideL, nL,
+                           p.ntile, p.ntiles_grid, p.ksplit, part, part_stride, beta);
     MDF_LAUNCHED("k_step2");
     return MDF_OK;
 }
 
-// The block loop of mdf_get_k for element type T.
+// The block loop of mdf_get_k for element type T.  Step 1 runs on the pair
+// tiles where the caller has them, else from the pair map or the packed
+// triangle.
 template <typename T, typename Src>
-int run_k(const KPlan &p, const Src *cderi, long naux, long ld, const int *pair_map, int nao,
+int run_k(const KPlan &p, const Src *cderi, long naux, long ld, const int *pair_map, const void *pair_tiles, int nao,
           const double *fl, const double *fr, int nocc, long ldf, double *vk, long ldvk, int accumulate,
           void *work, hipStream_t st) {
     const bool two = fr != nullptr;
     double *part = (double *)work;
     T *rl = (T *)(part + align_up(p.part_words, 64));
     T *rr = two ? rl + align_up(p.r_words, 64) : rl;
+    T *fp[2];
+    fp[0] = rr + align_up(p.r_words, 64);
+    fp[1] = fp[0] + align_up(pack_words(p, nao, nocc), 64);
+    if (pair_tiles)
+        for (int side = 0; side < (two ? 2 : 1); side++)
+            if (int rc = pack_factor<T>(p, st, side ? fr : fl, ldf, nao, nocc, fp[side])) return rc;
     const long ldr = r_ld(nocc, sizeof(T)), strideL = (long)nao * ldr;
     const long part_stride = (long)nao * nao;
     for (long L0 = 0; L0 < naux; L0 += p.nL) {
         const int nL = (int)(naux - L0 < p.nL ? naux - L0 : p.nL);
         const Src *blk = cderi + L0 * ld;
-        int rc = step1<T, Src>(p, nL, st, blk, ld, pair_map, nao, fl, ldf, nocc, rl, ldr, strideL);
-        if (rc) return rc;
-        if (two) {
-            rc = step1<T, Src>(p, nL, st, blk, ld, pair_map, nao, fr, ldf, nocc, rr, ldr, strideL);
+        int rc;
+        for (int side = 0; side < (two ? 2 : 1); side++) {
+            T *r = side ? rr : rl;
+            rc = pair_tiles ? step1_pairs<T, Src>(p, nL, st, blk, ld, tiles::view(pair_tiles, nao), fp[side], nocc, r,
+                                                  ldr, strideL)
+                            : step1<T, Src>(p, nL, st, blk, ld, pair_map, nao, side ? fr : fl, ldf, nocc, r, ldr,
+                                            strideL);
             if (rc) return rc;
         }
         rc = step2<T>(p, nL, two, st, rl, rr, nao, nocc, ldr, strideL, part, part_stride, L0 > 0);
@@ -274,8 +339,9 @@ int run_k_b3(const KPlan &p, const Src *cderi, long naux, long ld, const int *pa
 
 }  // namespace
 
-static size_t k_workspace(const KPlan &p, bool two, size_t elem) {
-    return align_up(p.part_words, 64) * sizeof(double) + (two ? 2 : 1) * align_up(p.r_words, 64) * elem;
+static size_t k_workspace(const KPlan &p, bool two, size_t elem, size_t pack) {
+    return align_up(p.part_words, 64) * sizeof(double) +
+           (two ? 2 : 1) * (align_up(p.r_words, 64) + align_up(pack, 64)) * elem;
 }
 
 // Aux rows per pass and workspace of one call for any precision.
@@ -283,23 +349,41 @@ static long k_rows_rule(long naux, int nao, int nocc, bool two, int prec) {
     if (prec == MDF_PREC_BF16X3) return block_rows(naux, nao, (int)kb3::pad32(nocc), two, 4);
     return block_rows(naux, nao, nocc, two, prec == MDF_PREC_FP32 ? sizeof(float) : sizeof(double));
 }
-static size_t k_bytes(long naux, int nao, int nocc, bool two, int prec, long rows) {
+static size_t k_bytes(long naux, int nao, int nocc, bool two, int prec, long rows, bool pairs) {
     KPlan p = plan_k(naux, nao, nocc, two, rows, prec == MDF_PREC_FP32 ? sizeof(float) : sizeof(double));
     if (prec == MDF_PREC_BF16X3) return kb3::layout(nao, nocc, p.nL, p.ksplit, two).total;
-    return k_workspace(p, two, prec == MDF_PREC_FP32 ? sizeof(float) : sizeof(double));
+    return k_workspace(p, two, prec == MDF_PREC_FP32 ? sizeof(float) : sizeof(double),
+                       pairs ? pack_words(p, nao, nocc) : 0);
+}
+
+static size_t k_workspace_rule(long naux, int nao, int nocc, bool two, int prec, long max_block_rows, bool pairs) {
+    long rows = k_rows_rule(naux, nao, nocc, two, prec);
+    if (max_block_rows > 0 && max_block_rows < rows) rows = max_block_rows;
+    return k_bytes(naux, nao, nocc, two, prec, rows, pairs);
 }
 
 extern "C" size_t mdf_get_k_workspace(long naux, int nao, int nocc, int two_factors, int prec,
                                       long max_block_rows) {
-    long rows = k_rows_rule(naux, nao, nocc, two_factors != 0, prec);
-    if (max_block_rows > 0 && max_block_rows < rows) rows = max_block_rows;
-    return k_bytes(naux, nao, nocc, two_factors != 0, prec, rows);
+    return k_workspace_rule(naux, nao, nocc, two_factors != 0, prec, max_block_rows, false);
+}
+
+extern "C" size_t mdf_get_k_tiles_workspace(long naux, int nao, int nocc, int two_factors, int prec,
+                                            long max_block_rows) {
+    return k_workspace_rule(naux, nao, nocc, two_factors != 0, prec, max_block_rows, true);
 }
 
 extern "C" int mdf_get_k(const void *cderi, int cderi_dtype, long naux, long npairs, long ld, const int *pair_map,
                          int nao, const double *fl, const double *fr, int nocc, long ldf, int prec,
                          double *vk, long ldvk, int accumulate, void *work, size_t work_bytes,
                          void *stream) {
+    return mdf_get_k_tiles(cderi, cderi_dtype, naux, npairs, ld, pair_map, nullptr, nao, fl, fr, nocc, ldf, prec, vk,
+                           ldvk, accumulate, work, work_bytes, stream);
+}
+
+extern "C" int mdf_get_k_tiles(const void *cderi, int cderi_dtype, long naux, long npairs, long ld,
+                               const int *pair_map, const void *pair_tiles, int nao, const double *fl,
+                               const double *fr, int nocc, long ldf, int prec, double *vk, long ldvk, int accumulate,
+                               void *work, size_t work_bytes, void *stream) {
     MDF_CHECK_ARG(naux >= 0 && nao >= 0 && nocc >= 0, "mdf_get_k: bad sizes");
     MDF_CHECK_ARG(cderi && fl && vk, "mdf_get_k: null pointer");
     MDF_CHECK_ARG(ld >= npairs && ldf >= nocc && ldvk >= nao, "mdf_get_k: leading dimension too small");
@@ -310,16 +394,19 @@ extern "C" int mdf_get_k(const void *cderi, int cderi_dtype, long naux, long npa
     MDF_CHECK_ARG(pair_map || npairs == (long)nao * (nao + 1) / 2,
                   "mdf_get_k: without a pair map the cderi must hold the full packed triangle "
                   "(npairs=%ld, nao=%d)", npairs, nao);
+    MDF_CHECK_ARG(!pair_tiles || (nao <= tiles::MAX_NAO && npairs < (1L << 29)),
+                  "mdf_get_k: pair tiles hold up to %d functions and 2^29 pairs (nao=%d, npairs=%ld)", tiles::MAX_NAO,
+                  nao, npairs);
     hipStream_t st = as_stream(stream);
     if (nao == 0) return MDF_OK;
-    const bool two = fr != nullptr;
+    const bool two = fr != nullptr, pairs = pair_tiles != nullptr;
     if (nocc == 0 || naux == 0) {
         if (!accumulate)
             for (int i = 0; i < nao; i++) MDF_HIP(hipMemsetAsync(vk + (long)i * ldvk, 0, nao * sizeof(double), st));
         return MDF_OK;
     }
     MDF_CHECK_ARG(work != nullptr, "mdf_get_k: workspace is null");
-    size_t need1 = k_bytes(naux, nao, nocc, two, prec, 1);
+    size_t need1 = k_bytes(naux, nao, nocc, two, prec, 1, pairs);
     if (work_bytes < need1) {
         set_error("mdf_get_k: workspace %zu bytes < %zu required", work_bytes, need1);
         return MDF_EWORKSPACE;
@@ -327,11 +414,11 @@ extern "C" int mdf_get_k(const void *cderi, int cderi_dtype, long naux, long npa
     // passes of the shape rule's aux rows (the grouped launch cuts the same
     // way); shorter when the workspace is smaller
     long rows = k_rows_rule(naux, nao, nocc, two, prec);
-    if (k_bytes(naux, nao, nocc, two, prec, rows) > work_bytes) {
+    if (k_bytes(naux, nao, nocc, two, prec, rows, pairs) > work_bytes) {
         long lo = 1, hi = rows;          // largest rows that fit
         while (lo < hi) {
             const long mid = (lo + hi + 1) / 2;
-            if (k_bytes(naux, nao, nocc, two, prec, mid) <= work_bytes) lo = mid; else hi = mid - 1;
+            if (k_bytes(naux, nao, nocc, two, prec, mid, pairs) <= work_bytes) lo = mid; else hi = mid - 1;
         }
         rows = lo;
     }
@@ -341,15 +428,19 @@ extern "C" int mdf_get_k(const void *cderi, int cderi_dtype, long naux, long npa
         if (prec == MDF_PREC_BF16X3)
             return run_k_b3(p, c, naux, ld, pair_map, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate, work, st);
         if (prec == MDF_PREC_FP32)
-            return run_k<float>(p, c, naux, ld, pair_map, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate, work, st);
-        return run_k<double>(p, c, naux, ld, pair_map, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate, work, st);
+            return run_k<float>(p, c, naux, ld, pair_map, pair_tiles, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate,
+                                 work, st);
+        return run_k<double>(p, c, naux, ld, pair_map, pair_tiles, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate,
+                                 work, st);
     }
     const double *c = (const double *)cderi;
     if (prec == MDF_PREC_BF16X3)
         return run_k_b3(p, c, naux, ld, pair_map, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate, work, st);
     if (prec == MDF_PREC_FP32)
-        return run_k<float>(p, c, naux, ld, pair_map, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate, work, st);
-    return run_k<double>(p, c, naux, ld, pair_map, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate, work, st);
+        return run_k<float>(p, c, naux, ld, pair_map, pair_tiles, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate,
+                                 work, st);
+    return run_k<double>(p, c, naux, ld, pair_map, pair_tiles, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate,
+                                 work, st);
 }
 
 // The first step of mdf_get_k alone, FP64: R[L] = A_L F for the nL aux rows

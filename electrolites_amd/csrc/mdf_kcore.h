@@ -11,6 +11,7 @@
 #include "mdf_common.h"
 #include "mdf_gemm.h"
 #include "mdf_b3.h"
+#include "mdf_tiles.h"
 
 namespace mdf {
 namespace kcore {
@@ -25,6 +26,7 @@ template <bool MAPPED, typename T = double, typename Src = double, int THREADS =
 struct PackedALoader {
     using reg_t = Src;                                   // the cderi storage type
     static constexpr int N = 128 * G_BK / THREADS;       // 8 (256 threads) or 4 (512)
+    static constexpr int SWZ = 0;
     static constexpr int TPJ = THREADS / G_BK;           // threads per j row (upper)
     static constexpr int TPR = G_BK / N;                 // threads per i row (lower)
     const Src *row;      // cderi row L
@@ -169,49 +171,97 @@ __device__ __forceinline__ void step1_tile(const Src *__restrict__ row, const in
     gemm_epilogue_layout<128, BN, T, decltype(acc), decltype(emit) &, 2, C::WGN>(acc, emit);
 }
 
+// The step-1 tile of one group of pair tiles: its 16 AO rows of the nl (1..8)
+// aux rows at c, occupied columns k0..k0+BN-1, into the R blocks of those aux
+// rows.  `fp` is the packed factor (tiles::pack_factor_range, row stride ldp).
+template <int BN, typename T, typename Src, bool HALVES>
+__device__ __forceinline__ void step1_pairs_tile(const Src *__restrict__ c, long ld, int nl, const tiles::View &tv, int g,
+                                        const T *__restrict__ fp, unsigned ldp, int nocc, T *__restrict__ R, long ldr,
+                                        long strideL, int k0, T *lds) {
+    using C = Step1Shape<BN>;
+    using S = typename C::S;
+    tiles::ALoader<T, Src, C::THREADS, HALVES> la;
+    tiles::BLoader<BN, T, C::THREADS> lb;
+    la.init(c, ld, nl, tv.map + (long)g * tv.ccap * tiles::RB);
+    lb.init(fp, ldp, k0, tv.cols + (long)g * tv.ccap);
+    Acc<S::MI, S::NI, T> acc;
+    acc.zero();
+    gemm_mainloop<128, BN, decltype(la), decltype(lb), T, 2, C::WGN>(la, lb, tv.nstep[g], lds, acc);
+    // a wavefront's 16-row MFMA blocks are whole aux rows
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int l0 = (wave % 2) * S::MI, c0 = k0 + (wave / 2) * S::WN + (lane & 15);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int i = tv.rows[g * tiles::RB + Mfma<T>::row(lane, v)];
+        if (i < 0) continue;
+        T *Ri = R + (long)i * ldr + c0;
+#pragma unroll
+        for (int mi = 0; mi < S::MI; mi++)
+            if (l0 + mi < nl) {
+                T *Rl = Ri + (l0 + mi) * strideL;
+#pragma unroll
+                for (int ni = 0; ni < S::NI; ni++)
+                    if (c0 + ni * 16 < nocc) Rl[ni * 16] = acc.v[mi][ni][v];
+            }
+    }
+}
+
 // ---------------------------------------------------------------- step 2
 // Rows r0..r0+127 of R[L] (k contiguous); K-step kt of this split is
-// (L, kc) = divmod(s0 + kt, kchunks), columns kc*16 .. kc*16 + 15.
-template <bool VEC, typename T>
+// (L, kc) = divmod(s0 + kt, kchunks), columns kc*16 .. kc*16 + 15.  Rows of R
+// are whole 16-byte pieces (r_ld); the lanes of a row take its pieces, as in
+// RowsLoader.
+template <typename T>
 struct TransformedLoader {
     using reg_t = T;
     static constexpr int N = 128 * G_BK / G_THREADS;     // 8
-    static constexpr int EPV = 16 / (int)sizeof(T);       // elements per 16-byte load
-    using V = typename std::conditional<sizeof(T) == 8, double2, float4>::type;
+    static constexpr int EPV = 16 / (int)sizeof(T);      // elements per 16-byte piece
+    static constexpr int Q = N / EPV, LPR = G_BK / EPV, RPP = G_THREADS / LPR;
+    static constexpr int SWZ = sizeof(T) == 8 ? 2 : 3;
     const T *R;
-    long strideL, ldr;
-    int r0, nao, nocc, kchunks;
+    long strideL;
+    int nocc, kchunks;
+    unsigned off[Q];     // this thread's rows
+    int last;            // its column in a row's last, ragged chunk
     long L;              // current aux row of the next load()
     int kc;              // current k chunk of the next load()
-    // thread t owns row t % 128 and k half t / 128, so a wavefront's LDS
-    // stores cover 64 consecutive rows of one k (no bank conflicts)
+    int left;            // columns in range of the loaded chunk
+    __device__ __forceinline__ TransformedLoader(const T *R_, long strideL_, long ldr, int r0, int nao, int nocc_,
+                                                 int kchunks_, long L_, int kc_)
+        : R(R_), strideL(strideL_), nocc(nocc_), kchunks(kchunks_), L(L_), kc(kc_) {
+        const int c = (int)(threadIdx.x % LPR) * EPV;
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+            off[q] = (unsigned)((long)min(r0 + (int)(threadIdx.x / LPR) + q * RPP, nao - 1) * ldr) + c;
+        last = min((kchunks - 1) * G_BK + c, (int)ldr - EPV) - c;
+    }
     __device__ __forceinline__ void load(int, T (&r)[N]) {
         // called for kt = 0, 1, 2, ... in order: advance (L, kc) in place
-        const int t = threadIdx.x;
-        const int kb = kc * G_BK + (t >> 7) * N;
-        const int row = r0 + (t & 127);
-        const T *src = R + L * strideL + (long)row * ldr + kb;
-        if (VEC && row < nao && kb + N <= nocc) {
+        const bool ragged = (kc + 1) * G_BK > nocc;
+        const T *src = R + L * strideL + (ragged ? last : kc * G_BK);
 #pragma unroll
-            for (int v = 0; v < N; v += EPV) {
-                const V x = *reinterpret_cast<const V *>(src + v);
-                const T *xe = reinterpret_cast<const T *>(&x);
+        for (int q = 0; q < Q; q++) {
+            const Piece<T, EPV> x = *(const Piece<T, EPV> *)(src + off[q]);
 #pragma unroll
-                for (int e = 0; e < EPV; e++) r[v + e] = xe[e];
-            }
-        } else {
-#pragma unroll
-            for (int v = 0; v < N; v++) r[v] = (row < nao && kb + v < nocc) ? src[v] : (T)0;
+            for (int e = 0; e < EPV; e++) r[q * EPV + e] = x.v[e];
         }
+        left = nocc - kc * G_BK;
         if (++kc == kchunks) {
             kc = 0;
             ++L;
         }
     }
-    __device__ __forceinline__ void store(const T (&r)[N], T *lds, int pitch) const {
-        const int t = threadIdx.x, ii = t & 127, kb = (t >> 7) * N;
+    __device__ __forceinline__ void store(T (&r)[N], T *lds, int pitch) const {
+        const int k = (int)(threadIdx.x % LPR) * EPV;
+        if (left < G_BK) {
+            // columns nocc.. are not written: zero, whatever they hold
 #pragma unroll
-        for (int v = 0; v < N; v++) lds[(kb + v) * pitch + ii] = r[v];
+            for (int e = 0; e < N; e++)
+                if (k + e % EPV >= left) r[e] = (T)0;
+        }
+        T *d = lds + k * pitch + ((int)(threadIdx.x / LPR) ^ swizzle<SWZ>(k));
+#pragma unroll
+        for (int e = 0; e < N; e++) d[(e % EPV) * pitch + e / EPV * RPP] = r[e];
     }
 };
 
@@ -223,7 +273,7 @@ constexpr int S2_FLUSH = 32;
 
 // One 128 x 128 output tile (i0, j0) of step 2 over the K-steps [s0, s1) of
 // the (L, k-chunk) reduction; writes (beta = 0) or adds (beta = 1) into o.
-template <bool VEC, typename T>
+template <typename T>
 __device__ __forceinline__ void step2_tile(const T *__restrict__ Rl, const T *__restrict__ Rr, int nao, int nocc, long ldr,
                                   long strideL, int i0, int j0, long s0, long s1, double *__restrict__ o, int beta,
                                   T *lds) {
@@ -231,8 +281,8 @@ __device__ __forceinline__ void step2_tile(const T *__restrict__ Rl, const T *__
     const int kchunks = (nocc + G_BK - 1) / G_BK;
     const long Ls = s0 / kchunks;
     const int kcs = (int)(s0 - Ls * kchunks);
-    TransformedLoader<VEC, T> la{Rl, strideL, ldr, i0, nao, nocc, kchunks, Ls, kcs};
-    TransformedLoader<VEC, T> lb{Rr, strideL, ldr, j0, nao, nocc, kchunks, Ls, kcs};
+    TransformedLoader<T> la{Rl, strideL, ldr, i0, nao, nocc, kchunks, Ls, kcs};
+    TransformedLoader<T> lb{Rr, strideL, ldr, j0, nao, nocc, kchunks, Ls, kcs};
     Acc<S::MI, S::NI, T> acc;
     auto emit = [&](int r, int c, double v) {
         const int i = i0 + r, j = j0 + c;
@@ -404,6 +454,10 @@ inline KPlan plan_k(long naux, int nao, int nocc, bool two, long max_rows, size_
     p.part_words = (size_t)p.ksplit * nao * nao;
     return p;
 }
+
+// Packed factor of the pair-tile step 1: nao + 1 rows of whole tile widths.
+inline unsigned pack_ld(const KPlan &p, int nocc) { return (unsigned)((nocc + p.bn - 1) / p.bn * p.bn); }
+inline size_t pack_words(const KPlan &p, int nao, int nocc) { return (size_t)(nao + 1) * pack_ld(p, nocc); }
 
 // ------------------------------------------------- split-BF16 (prec 2)
 // The same two steps on the three-term split-BF16 engine (mdf_b3.h).  The

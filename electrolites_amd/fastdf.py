@@ -29,6 +29,7 @@ values are widened to FP64 before arithmetic.
 """
 import ctypes
 import os
+import threading
 import weakref
 
 import numpy as np
@@ -207,6 +208,59 @@ class _PairLayout:
             self.map = t.empty(nao * nao, dtype=t.int32, device=_dev.device())
             _lib.call('mdf_build_pair_map', _dev.ptr(addr), npairs, nao,
                       _dev.ptr(self.map), _dev.stream_ptr())
+        self._tiles = {}
+        self._tiles_lock = threading.Lock()
+
+    def tiles(self, lower=False):
+        """The pair tiles of this layout's map (K's step 1 skips the pairs
+        not stored), built at the first exchange; None for a full triangle
+        or sizes they do not hold.  ``lower``: the triangular half's.  Another
+        stream than the building one waits for it."""
+        if self.map is None:
+            return None
+        with self._tiles_lock:
+            got = self._tiles.get(lower)
+            if got is None:
+                got = self._tiles[lower] = PairTiles(
+                    self.map, self.nao, self.npairs, lower,
+                    self._tiles[False].buf if lower and False in self._tiles else None)
+        return got.on_stream()
+
+
+#: K's step 1 runs on pair tiles from this many functions: below it they
+#: gain nothing (a whole get_jk at nao 72: 257 us with them, 253 without; at
+#: 120: 342 and 352; at 192: 534 and 607) and the first call pays for them
+TILES_MIN_NAO = 112
+
+
+class PairTiles:
+    """``mdf_build_pair_tiles`` of a pair map, with the stream it was built
+    on (``buf`` None: sizes the tiles do not hold or do not help)."""
+
+    def __init__(self, pair_map, nao, npairs, lower=False, order_of=None):
+        t = _dev.torch()
+        self.buf = None
+        nbytes = _lib.query('mdf_pair_tiles_bytes', nao) if nao >= TILES_MIN_NAO and npairs < 1 << 29 else 0
+        if not nbytes:
+            return
+        self.buf = t.empty(nbytes, dtype=t.uint8, device=pair_map.device)
+        _lib.call('mdf_build_pair_tiles', _dev.ptr(pair_map), nao, int(lower), _dev.ptr(order_of),
+                  _dev.ptr(self.buf), nbytes, _dev.stream_ptr())
+        self.stream = t.cuda.current_stream()
+        self.done = t.cuda.Event()
+        self.done.record(self.stream)
+
+    def on_stream(self):
+        """The buffer, ordered before the current stream's next work and kept
+        for it."""
+        if self.buf is None:
+            return None
+        cur = _dev.torch().cuda.current_stream()
+        if cur != self.stream:
+            if not self.done.query():
+                cur.wait_event(self.done)
+            self.buf.record_stream(cur)
+        return self.buf
 
 
 def _layout(dfobj, cderi, nao):
@@ -412,6 +466,10 @@ def _dtype_code(cderi):
     raise ValueError(f'cderi dtype {cderi.dtype}')
 
 
+def _k_workspace(tiles):
+    return 'mdf_get_k_workspace' if tiles is None else 'mdf_get_k_tiles_workspace'
+
+
 def _vk(cderi, lay, fl, fr, precision='fp64'):
     """``vk[n] = sum_L (A_L fl[n])(A_L fr[n])^T`` on the HIP path.
     ``precision`` 'fp64', 'fp32' (FP32 MFMA for both steps) or 'bf16x3'
@@ -427,12 +485,13 @@ def _vk(cderi, lay, fl, fr, precision='fp64'):
     rows = max(1, min(naux, K_WORKSPACE_BYTES // max(per_row, 1)))
     # the library cuts naux into passes by shape (the grouped launch cuts the
     # same way); K_WORKSPACE_BYTES can only shorten them
-    nbytes = _lib.query('mdf_get_k_workspace', naux, nao, nocc, int(two), prec, rows)
+    tiles = lay.tiles()
+    nbytes = _lib.query(_k_workspace(tiles), naux, nao, nocc, int(two), prec, rows)
     work = _dev.WORKSPACE.get(nbytes)
     for i in range(n):
         STATS['k_calls'] += 1
-        _lib.call('mdf_get_k', _dev.ptr(cderi), _dtype_code(cderi), naux, npairs, cderi.stride(0),
-                  _dev.ptr(lay.map), nao, _dev.ptr(fl[i]),
+        _lib.call('mdf_get_k_tiles', _dev.ptr(cderi), _dtype_code(cderi), naux, npairs, cderi.stride(0),
+                  _dev.ptr(lay.map), _dev.ptr(tiles), nao, _dev.ptr(fl[i]),
                   _dev.ptr(fr[i]) if two else None, nocc, nocc, prec,
                   _dev.ptr(vk[i]), nao, 0, _dev.ptr(work), nbytes,
                   _dev.stream_ptr())
@@ -459,12 +518,13 @@ def _jk_blocked(dfobj, cderi, lay, dms3, hermi, with_j, fl, fr, precision, block
     blk_rows = blk_rows or dfstore.block_rows(npairs, elem, naux)
     with_k = fl is not None
     jbytes = _lib.query('mdf_get_j_workspace', blk_rows, npairs, n) if with_j else 0
-    kbytes, prec, two, nocc = 0, PRECISIONS[precision], False, 0
+    kbytes, prec, two, nocc, tiles = 0, PRECISIONS[precision], False, 0, None
     if with_k:
+        tiles = lay.tiles()
         nocc, two = fl.shape[-1], fr is not None
         per_row = nao * nocc * (8 if prec == 0 else 4) * (2 if two else 1)
         rows = max(1, min(blk_rows, K_WORKSPACE_BYTES // max(per_row, 1)))
-        kbytes = _lib.query('mdf_get_k_workspace', blk_rows, nao, nocc, int(two), prec, rows)
+        kbytes = _lib.query(_k_workspace(tiles), blk_rows, nao, nocc, int(two), prec, rows)
     nbytes = max(jbytes, kbytes)
     if blocks is None:
         # what this call allocates beside the prefix: two streamed blocks,
@@ -495,8 +555,8 @@ def _jk_blocked(dfobj, cderi, lay, dms3, hermi, with_j, fl, fr, precision, block
         if with_k:
             for i in range(n):
                 STATS['k_calls'] += 1
-                _lib.call('mdf_get_k', _dev.ptr(blk), dt, nL, npairs, ld, _dev.ptr(lay.map), nao,
-                          _dev.ptr(fl[i]), _dev.ptr(fr[i]) if two else None, nocc, nocc, prec,
+                _lib.call('mdf_get_k_tiles', _dev.ptr(blk), dt, nL, npairs, ld, _dev.ptr(lay.map),
+                          _dev.ptr(tiles), nao, _dev.ptr(fl[i]), _dev.ptr(fr[i]) if two else None, nocc, nocc, prec,
                           _dev.ptr(vk[i]), nao, 1, _dev.ptr(work), nbytes, _dev.stream_ptr())
     vj = None
     if with_j:

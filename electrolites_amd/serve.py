@@ -141,7 +141,7 @@ class _Slot:
         self.cderi = fastdf._cderi_of(dfobj)
         nao = req.mol.nao
         self.lay = fastdf._layout(dfobj, self.cderi, nao)
-        self.entry = batch.Entry(self.cderi, nao, 1, self.scf.nocc, pair_map=self.lay.map)
+        self.entry = batch.Entry(self.cderi, nao, 1, self.scf.nocc, pair_map=self.lay.map, pair_tiles=self.lay.tiles())
         self.entry.layout = self.lay
         self.nao = nao
         self._vj = t.empty((1, nao, nao), dtype=t.float64, device=self.cderi.device)

@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define MDF_ABI_VERSION 12
+#define MDF_ABI_VERSION 13
 
 /* arithmetic precision of a contraction */
 #define MDF_PREC_FP64 0
@@ -114,6 +114,29 @@ int mdf_get_k(const void *cderi, int cderi_dtype, long naux, long npairs, long l
               double *vk, long ldvk, int accumulate, void *work, size_t work_bytes,
               void *stream);
 
+/* ---- pair tiles: a screened cderi's pairs in blocks ---------------------
+ * No counterpart in the reference (its block-sparse step 1 works on fixed
+ * 128-wide tiles, electrolites/fastdf.py:566-574).  mdf_build_pair_tiles turns
+ * a pair map into groups of 16 AO rows with compacted column lists (one device
+ * buffer of mdf_pair_tiles_bytes(nao) bytes, 0 when nao is out of range; built
+ * on the stream, nothing returns to the host).  It depends on the pair map
+ * only and serves every later call over the same cderi.  lower != 0: the
+ * triangular half T with A = T + T^T (columns of a row's own and earlier
+ * groups, own-group pairs halved), for mdf_k_step1_tiles; order_of, another
+ * buffer of the same map or NULL, gives the row order.
+ * mdf_get_k_tiles is mdf_get_k with step 1 on the tiles (pair_tiles NULL:
+ * mdf_get_k itself; MDF_PREC_BF16X3 uses the pair map either way); npairs <
+ * 2^29.  Its workspace also holds the packed factors. */
+size_t mdf_pair_tiles_bytes(int nao);
+int mdf_build_pair_tiles(const int *pair_map, int nao, int lower, const void *order_of, void *tiles,
+                         size_t tiles_bytes, void *stream);
+size_t mdf_get_k_tiles_workspace(long naux, int nao, int nocc, int two_factors, int prec,
+                                 long max_block_rows);
+int mdf_get_k_tiles(const void *cderi, int cderi_dtype, long naux, long npairs, long ld, const int *pair_map,
+                    const void *pair_tiles, int nao, const double *fl, const double *fr, int nocc, long ldf,
+                    int prec, double *vk, long ldvk, int accumulate, void *work, size_t work_bytes,
+                    void *stream);
+
 /* ---- grouped J/K over many (molecule, density) items -------------------
  * No counterpart in the reference (each get_jk call there contracts one
  * molecule, electrolites/fastdf.py:805-1026); this batches many.  One item
@@ -149,6 +172,7 @@ typedef struct {
     int nocc;
     double *vk;
     int cderi_dtype;      /* MDF_DTYPE_F64 or _F32; one storage type per plan */
+    const void *pair_tiles;   /* the pair map's tiles (mdf_build_pair_tiles) or NULL */
 } mdf_jk_item;
 
 typedef struct mdf_grouped_plan mdf_grouped_plan;

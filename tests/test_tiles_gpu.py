@@ -1,0 +1,155 @@
+"""K's step 1 on pair tiles against the pair-map path and a plain FP64 sum,
+at the sizes where it can go wrong: AO counts off the 16-row groups, aux rows
+off the blocks of 8, occupied counts at the edges of the tile widths, AOs with
+no stored pair, one and two factors, one storage or arithmetic type at a time."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def pair_list(rng, nao, fill, empty=()):
+    """A screened pair list: each pair with probability ``fill`` (rows of
+    their own densities), none for the AOs in ``empty``."""
+    rows, cols = np.tril_indices(nao)
+    p = np.clip(fill * (.2 + 1.6 * rng.random(nao)), 0, 1)
+    keep = rng.random(len(rows)) < np.sqrt(p[rows] * p[cols])
+    for i in empty:
+        keep &= (rows != i) & (cols != i)
+    return rows[keep], cols[keep]
+
+
+def exact_k(cderi, rows, cols, nao, fl, fr):
+    import torch
+    a = torch.zeros((len(cderi), nao, nao), dtype=torch.float64, device='cuda')
+    a[:, rows, cols] = cderi.double()
+    a[:, cols, rows] = cderi.double()
+    rl = (a.reshape(-1, nao) @ fl).reshape(len(cderi), nao, -1).transpose(0, 1).reshape(nao, -1)
+    rr = rl if fr is None else (a.reshape(-1, nao) @ fr).reshape(len(cderi), nao, -1).transpose(0, 1).reshape(nao, -1)
+    return rl @ rr.T.contiguous()
+
+
+def inputs(nao, naux, nocc, two, storage='float64', seed=0, empty=()):
+    import torch
+    rng = np.random.default_rng(seed + 7 * nao + naux + 31 * nocc)
+    rows, cols = pair_list(rng, nao, .4, empty)
+    dt = getattr(torch, storage)
+    cderi = torch.from_numpy(rng.standard_normal((naux, len(rows)))).cuda().to(dt)
+    f = [torch.from_numpy(rng.standard_normal((nao, nocc))).cuda() for _ in range(1 + two)]
+    addr = torch.from_numpy((rows * nao + cols).astype(np.int32)).cuda()
+    return cderi, torch.from_numpy(rows).cuda(), torch.from_numpy(cols).cuda(), addr, f[0], f[1] if two else None
+
+
+def make_tiles(addr, nao, lower=0, order_of=None):
+    import torch
+    from electrolites_amd import _dev, _lib
+    pmap = torch.empty(nao * nao, dtype=torch.int32, device='cuda')
+    _lib.call('mdf_build_pair_map', _dev.ptr(addr), len(addr), nao, _dev.ptr(pmap), _dev.stream_ptr())
+    nb = _lib.query('mdf_pair_tiles_bytes', nao)
+    buf = torch.full((nb,), 0x5a, dtype=torch.uint8, device='cuda')
+    _lib.call('mdf_build_pair_tiles', _dev.ptr(pmap), nao, lower, _dev.ptr(order_of), _dev.ptr(buf), nb,
+              _dev.stream_ptr())
+    return pmap, buf
+
+
+def get_k(cderi, pmap, tiles, nao, fl, fr, prec, rows=0):
+    import torch
+    from electrolites_amd import _dev, _lib, fastdf
+    naux, npairs = cderi.shape
+    nocc = fl.shape[1]
+    q = 'mdf_get_k_workspace' if tiles is None else 'mdf_get_k_tiles_workspace'
+    nb = _lib.query(q, naux, nao, nocc, int(fr is not None), prec, rows)
+    # NaN workspace: every value that is used has to have been written
+    work = torch.full((nb // 8 + 1,), float('nan'), dtype=torch.float64, device='cuda')
+    vk = torch.full((nao, nao), float('nan'), dtype=torch.float64, device='cuda')
+    _lib.call('mdf_get_k_tiles', _dev.ptr(cderi), fastdf._dtype_code(cderi), naux, npairs, cderi.stride(0),
+              _dev.ptr(pmap), _dev.ptr(tiles), nao, _dev.ptr(fl), _dev.ptr(fr), nocc, nocc, prec, _dev.ptr(vk), nao,
+              0, _dev.ptr(work), nb, _dev.stream_ptr())
+    return vk
+
+
+def rel(a, b):
+    return float((a - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize('nao,naux,nocc', [
+    (1, 1, 1), (16, 8, 16), (17, 9, 17), (31, 7, 63), (33, 15, 64), (112, 16, 65), (129, 17, 129), (130, 3, 161),
+    (145, 8, 193), (131, 5, 257), (128, 2, 321)])
+@pytest.mark.parametrize('two', [False, True])
+def test_k_tiles_fp64(nao, naux, nocc, two):
+    print(f'k tiles nao {nao} naux {naux} nocc {nocc} two {two}', flush=True)
+    empty = (0, nao - 1, nao // 2) if nao > 16 else ()
+    cderi, rows, cols, addr, fl, fr = inputs(nao, naux, nocc, two, empty=empty)
+    if not len(addr):
+        pytest.skip('no pair drawn')
+    pmap, buf = make_tiles(addr, nao)
+    vk = get_k(cderi, pmap, buf, nao, fl, fr, 0)
+    # a product of n terms in any order is within n eps of the exact one
+    tol = 2.3e-16 * (nao + naux * nocc)
+    assert rel(vk, exact_k(cderi, rows, cols, nao, fl, fr)) < tol
+    assert rel(vk, get_k(cderi, pmap, None, nao, fl, fr, 0)) < 2 * tol
+
+
+@pytest.mark.parametrize('storage,prec', [('float32', 0), ('float32', 1), ('float64', 1)])
+@pytest.mark.parametrize('nao,naux,nocc', [(33, 9, 17), (130, 12, 161), (150, 5, 320)])
+def test_k_tiles_types(storage, prec, nao, naux, nocc):
+    print(f'k tiles {storage} prec {prec} nao {nao} naux {naux} nocc {nocc}', flush=True)
+    cderi, rows, cols, addr, fl, _ = inputs(nao, naux, nocc, False, storage)
+    pmap, buf = make_tiles(addr, nao)
+    vk = get_k(cderi, pmap, buf, nao, fl, None, prec)
+    tol = (2.3e-16 if prec == 0 else 1.2e-7) * (nao + naux * nocc) ** (1 if prec == 0 else .5)
+    assert rel(vk, exact_k(cderi, rows, cols, nao, fl, None)) < tol
+
+
+def test_k_tiles_passes():
+    """Passes of fewer aux rows than a block of 8, and of several blocks."""
+    cderi, rows, cols, addr, fl, _ = inputs(60, 37, 20, False)
+    pmap, buf = make_tiles(addr, 60)
+    ref = exact_k(cderi, rows, cols, 60, fl, None)
+    for nrow in (1, 5, 8, 13):
+        print(f'k tiles passes of {nrow}', flush=True)
+        assert rel(get_k(cderi, pmap, buf, 60, fl, None, 0, nrow), ref) < 2.3e-16 * (60 + 37 * 20)
+
+
+@pytest.mark.parametrize('nao', [5, 16, 47, 130, 600, 2060])
+def test_tiles_hold_every_pair_once(nao):
+    """Rows are a permutation; the map holds each stored pair in both orders,
+    and its lower half each off-group pair once and each in-group pair twice
+    with the factor 1/2."""
+    import torch
+    print(f'tiles nao {nao}', flush=True)
+    rng = np.random.default_rng(nao)
+    rows, cols = pair_list(rng, nao, .1 if nao > 500 else .4, (nao // 3,))
+    addr = torch.from_numpy((rows * nao + cols).astype(np.int32)).cuda()
+    _, buf = make_tiles(addr, nao)
+    _, low = make_tiles(addr, nao, 1, buf)
+    G, C = (nao + 15) // 16, (nao + 31) // 32 * 32 + 32
+    half = 1 << 30
+    for which, b in (('full', buf), ('lower', low)):
+        w = b.cpu().numpy()[:(len(b) // 4) * 4].view(np.int32)
+        r = w[:16 * G].reshape(G, 16)
+        nstep = w[16 * G:17 * G]
+        o = (17 * G + 63) // 64 * 64
+        cc = w[o:o + G * C].reshape(G, C)
+        o = (o + G * C + 63) // 64 * 64
+        m = w[o:o + G * C * 16].reshape(G, C // 16, 16, 16)
+        assert sorted(r[r >= 0]) == list(range(nao)) and np.all(r.reshape(-1)[nao:] == -1)
+        got = np.zeros((nao, nao))
+        for g in range(G):
+            n = nstep[g] * 16
+            c = cc[g]
+            real = c[c < nao]
+            assert np.all(c[len(real):] == nao) and np.all(np.diff(real) > 0) and n == -(-len(real) // 16) * 16
+            mm = m[g].transpose(1, 0, 2).reshape(16, C)
+            assert np.all(mm[:, len(real):] == -1)
+            ii, kk = np.nonzero(mm >= 0)
+            e = mm[ii, kk]
+            i, j = r[g][ii], c[kk]
+            p = e & (half - 1)
+            assert np.all(rows[p] == np.maximum(i, j)) and np.all(cols[p] == np.minimum(i, j))
+            np.add.at(got, (i, j), np.where(e & half, .5, 1.))
+        want = np.zeros((nao, nao))
+        want[rows, cols] = want[cols, rows] = 1.
+        if which == 'lower':
+            got = got + got.T
+        assert np.array_equal(got, want)
