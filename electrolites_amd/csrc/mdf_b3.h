@@ -10,8 +10,9 @@
 // LDS holds each operand tile as two planes (hi, lo) of [row][k] bfloat16
 // with k contiguous and a row pitch of PK = 40 elements (80 bytes): a lane's
 // eight k values are one 16-byte ds_read, and eight consecutive rows start in
-// distinct bank groups.  Double-buffered; the next K-step's global loads are
-// held in registers (in the source type) while the current step's MFMAs run.
+// distinct bank groups.  Double-buffered; the global loads of the K-step after
+// the next are held in registers (in the source type) from one step's middle
+// to the next one's.
 //
 // MFMA lane layouts (measured with one-hot probes): lane l holds
 // A[m = l % 16][k = 8 (l / 16) + s] and B[k = 8 (l / 16) + s][n = l % 16]
@@ -39,6 +40,16 @@ __device__ __forceinline__ float bf16_f(u16 h) { return __uint_as_float((unsigne
 __device__ __forceinline__ void split(float x, u16 &hi, u16 &lo) {
     hi = bf16_rne(x);
     lo = bf16_rne(x - bf16_f(hi));
+}
+
+// Two values at once on the packed conversion (the same rounding): hi and lo
+// pairs, the first value in the low half.
+__device__ __forceinline__ void split2(float x0, float x1, unsigned &hi, unsigned &lo) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    hi = __builtin_bit_cast(unsigned, __builtin_convertvector((f2{x0, x1}), b2));
+    lo = __builtin_bit_cast(unsigned, __builtin_convertvector(
+        (f2{x0 - __uint_as_float(hi << 16), x1 - __uint_as_float(hi & 0xffff0000u)}), b2));
 }
 
 // A workgroup of WGM x WGN wavefronts computes a BM x BN tile; each
@@ -80,14 +91,13 @@ __device__ __forceinline__ void mainloop(LA &la, LB &lb, int nk, u16 *lds,
     lb.load(0, rb);
     la.store(ra, lds, lds + S::A_PLANE);
     lb.store(rb, lds + 2 * S::A_PLANE, lds + 2 * S::A_PLANE + S::B_PLANE);
+    if (nk > 1) {
+        la.load(1, ra);
+        lb.load(1, rb);
+    }
     __syncthreads();
     for (int kt = 0; kt < nk; kt++) {
         const int cur = kt & 1;
-        const bool more = kt + 1 < nk;
-        if (more) {
-            la.load(kt + 1, ra);
-            lb.load(kt + 1, rb);
-        }
         const MDF_LDS u16 *base = (const MDF_LDS u16 *)(lds + cur * S::STAGE);
         bf16x8_t ahi[S::MI], alo[S::MI], bhi[S::NI], blo[S::NI];
 #pragma unroll
@@ -101,17 +111,25 @@ __device__ __forceinline__ void mainloop(LA &la, LB &lb, int nk, u16 *lds,
             blo[ni] = *(const MDF_LDS bf16x8_t *)(base + boff + ni * 16 * PK + S::B_PLANE);
         }
 #pragma unroll
-        for (int mi = 0; mi < S::MI; mi++)
+        for (int mi = 0; mi < S::MI; mi++) {
+            // halfway through the MFMAs: the next step's tile into the other
+            // buffer, and the loads of the step after it, which have a whole
+            // step to arrive
+            if (mi == S::MI / 2 && kt + 1 < nk) {
+                u16 *nxt = lds + (cur ^ 1) * S::STAGE;
+                la.store(ra, nxt, nxt + S::A_PLANE);
+                lb.store(rb, nxt + 2 * S::A_PLANE, nxt + 2 * S::A_PLANE + S::B_PLANE);
+                if (kt + 2 < nk) {
+                    la.load(kt + 2, ra);
+                    lb.load(kt + 2, rb);
+                }
+            }
 #pragma unroll
             for (int ni = 0; ni < S::NI; ni++) {
                 acc.v[mi][ni] = mma(alo[mi], bhi[ni], acc.v[mi][ni]);
                 acc.v[mi][ni] = mma(ahi[mi], blo[ni], acc.v[mi][ni]);
                 acc.v[mi][ni] = mma(ahi[mi], bhi[ni], acc.v[mi][ni]);
             }
-        if (more) {
-            u16 *nxt = lds + (cur ^ 1) * S::STAGE;
-            la.store(ra, nxt, nxt + S::A_PLANE);
-            lb.store(rb, nxt + 2 * S::A_PLANE, nxt + 2 * S::A_PLANE + S::B_PLANE);
         }
         __syncthreads();
     }

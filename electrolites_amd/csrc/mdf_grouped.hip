@@ -80,8 +80,7 @@ struct Tile {
 // A launch of the K sequence: kind 0 = factor split (prec 2) or packing (items
 // with pair tiles), 1 = step 1, 2 = step 2, 3 = finalize, over tiles [start,
 // start + count) of that kind's table.  Step-1 launches hold items of one tile
-// width `bn` and one `mapped` flag each (split-BF16: a pair map; else: pair
-// tiles).
+// width `bn` and one form of the pairs (`mapped`) each.
 struct Phase {
     int kind;
     long start, count;
@@ -268,7 +267,14 @@ __global__ __launch_bounds__(256) void gk_split_ft(const GKItem *items, const Ti
         const Tile e = tiles[t];            // (item, chunk, side)
         const GKItem &it = items[e.item];
         using kcore::kb3::u16;
-        const long e0 = (long)e.a * 1024, e1 = min(e0 + 1024, (long)it.nocc * it.ldft);
+        const long e0 = (long)e.a * 1024;
+        if (it.tiles) {
+            kcore::kb3::pack_split_range(e.b ? it.fr : it.fl, it.nocc, it.nao, it.nocc,
+                                         (unsigned *)(work + (size_t)it.b3[e.b][0]), it.ldp, e0,
+                                         min(e0 + 1024, (long)(it.nao + 1) * it.ldp));
+            continue;
+        }
+        const long e1 = min(e0 + 1024, (long)it.nocc * it.ldft);
         kcore::kb3::split_ft_range(e.b ? it.fr : it.fl, it.nocc, it.nao, it.nocc,
                                    (u16 *)(work + (size_t)it.b3[e.b][0]), (u16 *)(work + (size_t)it.b3[e.b][1]),
                                    it.ldft, e0, e1);
@@ -296,6 +302,27 @@ __global__ __launch_bounds__(kcore::kb3::Step1Cfg<BN>::THREADS) void gk_step1_b3
         // each keeps the register budget of the single-item kernel)
         kcore::kb3::step1_tile<MAPPED, BN, Src>(row, it.pmap, it.nao, fthi, ftlo, it.ldft, it.nocc, rhi, rlo, it.ldr,
                                            e.b * kcore::kb3::BM, ktile * BN, lds);
+        __syncthreads();
+    }
+}
+
+template <int BN, typename Src>
+__global__ __launch_bounds__(kcore::kb3::Step1Cfg<BN>::THREADS) void gk_step1_pairs_b3(const GKItem *items,
+                                                                                       const Tile *tab, long n,
+                                                                                       char *work) {
+    using kcore::kb3::u16;
+    __shared__ u16 lds[kcore::kb3::Step1Cfg<BN>::S::LDS_ELEMS];
+    XCD_RUN_LOOP(t, n) {
+        const Tile e = tab[t];              // (item, first of 8 aux rows, group, k-tile | side << 16)
+        const GKItem &it = items[e.item];
+        const int side = e.c >> 16, ktile = e.c & 0xffff;
+        const long lb = e.a % it.nL, end = min(e.a - lb + it.nL, it.naux), stride = it.nao * it.ldr;
+        kcore::kb3::step1_pairs_tile<BN, Src>((const Src *)it.cderi + (long)e.a * it.ld, it.ld,
+                                              (int)min((long)tiles::NL, end - e.a), tiles::view(it.tiles, it.nao), e.b,
+                                              (const unsigned *)(work + (size_t)it.b3[side][0]), (unsigned)it.ldp,
+                                              (u16 *)(work + (size_t)it.b3[side][2]) + lb * stride,
+                                              (u16 *)(work + (size_t)it.b3[side][3]) + lb * stride, it.ldr, stride,
+                                              ktile * BN, lds);
         __syncthreads();
     }
 }
@@ -429,7 +456,7 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
                 g.nao = x.nao; g.nocc = x.nocc; g.ksplit = kp.ksplit; g.ntile = kp.ntile;
                 g.nL = kp.nL;
                 g.bn1 = bn ? bn : kcore::pick_bn(x.nocc);
-                if (!b3 && x.pair_tiles) {
+                if (x.pair_tiles) {
                     if (x.nao > tiles::MAX_NAO || x.npairs >= (1L << 29)) {
                         set_error("mdf_grouped_plan_create: item %d is beyond what pair tiles hold", m);
                         delete p;
@@ -438,13 +465,14 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
                     g.tiles = x.pair_tiles;
                     kp.bn = g.bn1;
                     g.ldp = kcore::pack_ld(kp, x.nocc);
-                    g.packb = align_up(kcore::pack_words(kp, x.nao, x.nocc) * elem, 256);
+                    g.packb = b3 ? 0 : align_up(kcore::pack_words(kp, x.nao, x.nocc) * elem, 256);
                 }
                 // workspace offsets are assigned per wave below; keep the sizes
                 if (b3) {
-                    const kcore::kb3::Layout y = kcore::kb3::layout(x.nao, x.nocc, kp.nL, kp.ksplit, two);
+                    const kcore::kb3::Layout y = kcore::kb3::layout(x.nao, x.nocc, kp.nL, kp.ksplit, two, g.tiles != nullptr);
                     g.ldr = y.ldr;
                     g.ldft = y.ldft;
+                    g.ldp = y.ldp;
                     g.bn3 = kcore::kb3::pick_bn(y.ldr);
                     g.rl = (void *)0;
                     g.part = (double *)y.total;
@@ -477,7 +505,8 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
         for (size_t i = w0; i < w1; i++) {
             GKItem &g = p->hk[i];
             if (prec == MDF_PREC_BF16X3) {
-                const kcore::kb3::Layout y = kcore::kb3::layout(g.nao, g.nocc, g.nL, g.ksplit, g.fr != nullptr);
+                const kcore::kb3::Layout y = kcore::kb3::layout(g.nao, g.nocc, g.nL, g.ksplit, g.fr != nullptr,
+                                                                    g.tiles != nullptr);
                 for (int side = 0; side < 2; side++) {
                     const kcore::kb3::Side q = kcore::kb3::side_ptrs((char *)o, y, g.fr ? side : 0);
                     g.b3[side][0] = q.fthi; g.b3[side][1] = q.ftlo; g.b3[side][2] = q.rhi; g.b3[side][3] = q.rlo;
@@ -501,8 +530,9 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
             const long s0 = k0.size();
             for (size_t i = w0; i < w1; i++) {
                 const GKItem &g = p->hk[i];
+                const long n0 = g.tiles ? (long)(g.nao + 1) * g.ldp : (long)g.nocc * g.ldft;
                 for (int side = 0; side < (g.fr ? 2 : 1); side++)
-                    for (long e = 0; e < cdiv((long)g.nocc * g.ldft, 1024L); e++) k0.push_back({(int)i, (int)e, side, 0});
+                    for (long e = 0; e < cdiv(n0, 1024L); e++) k0.push_back({(int)i, (int)e, side, 0});
             }
             p->kphases.push_back({0, s0, (long)k0.size() - s0, 0, 0});
         }
@@ -519,9 +549,10 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
             p->kphases.push_back({0, s0, (long)k0.size() - s0, 0, 0});
         }
         for (long b = 0; b < maxpass; b++) {
-          // one step-1 launch per tile width and per pair-map (split-BF16) or
-          // pair-tiles flag
-          for (int cls = 0; cls < (b3 ? 8 : 12); cls++) {
+          // one step-1 launch per tile width and per form of the pairs (0 the
+          // full triangle, or for FP64/FP32 a pair map too; 1 a pair map
+          // (split-BF16) or pair tiles; 2 pair tiles (split-BF16))
+          for (int cls = 0; cls < 12; cls++) {
             static const int kBN3[4] = {128, 192, 256, 320};
             static const int kBN1[6] = {64, 128, 160, 192, 256, 320};
             const int mp = cls / (b3 ? 4 : 6), cbn = b3 ? kBN3[cls % 4] : kBN1[cls % 6];
@@ -530,12 +561,12 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
                 const GKItem &g = p->hk[i];
                 const long L0 = b * g.nL;
                 if (L0 >= g.naux) continue;
-                if (b3 && ((g.pmap != nullptr) != (mp == 1) || g.bn3 != cbn)) continue;
+                if (b3 && ((g.tiles ? 2 : g.pmap ? 1 : 0) != mp || g.bn3 != cbn)) continue;
                 if (!b3 && ((g.tiles != nullptr) != (mp == 1) || g.bn1 != cbn)) continue;
                 const long L1 = std::min(L0 + g.nL, g.naux);
                 const int nkt = b3 ? (int)cdiv(g.ldr, (long)cbn) : (int)cdiv(g.nocc, cbn);
                 const int nit = (int)cdiv(g.nao, 128);
-                if (!b3 && mp) {
+                if (g.tiles) {
                     // the groups of one aux block together, the longest first
                     for (int side = 0; side < (g.fr ? 2 : 1); side++)
                         for (long L = L0; L < L1; L += tiles::NL)
@@ -713,6 +744,15 @@ static void launch_gk1_b3(const mdf_grouped_plan *p, const Tile *tiles, long n, 
         hipLaunchKernelGGL((gk_step1_b3<MAPPED, BN, double>), g, b, 0, st, p->kitems, tiles, n, w);
 }
 
+template <int BN>
+static void launch_gk1_pairs_b3(const mdf_grouped_plan *p, const Tile *tab, long n, char *w, hipStream_t st) {
+    const dim3 g(persistent_grid(n, BN == 128 ? 2 : 1)), b(kcore::kb3::Step1Cfg<BN>::THREADS);
+    if (p->dtype == MDF_DTYPE_F32)
+        hipLaunchKernelGGL((gk_step1_pairs_b3<BN, float>), g, b, 0, st, p->kitems, tab, n, w);
+    else
+        hipLaunchKernelGGL((gk_step1_pairs_b3<BN, double>), g, b, 0, st, p->kitems, tab, n, w);
+}
+
 extern "C" int mdf_grouped_jk(const mdf_grouped_plan *p, void *work, size_t work_bytes, void *stream) {
     MDF_CHECK_ARG(p && (work || p->work_bytes <= 256), "mdf_grouped_jk: null argument");
     if (work_bytes < p->work_bytes) {
@@ -760,7 +800,14 @@ extern "C" int mdf_grouped_jk(const mdf_grouped_plan *p, void *work, size_t work
                 MDF_LAUNCHED("gk_split_ft");
             } else if (ph.kind == 1 && b3) {
                 const Tile *t1 = p->k1 + ph.start;
-                switch (ph.bn * 2 + ph.mapped) {
+                if (ph.mapped == 2) {
+                    switch (ph.bn) {
+                    case 320: launch_gk1_pairs_b3<320>(p, t1, ph.count, w, st); break;
+                    case 256: launch_gk1_pairs_b3<256>(p, t1, ph.count, w, st); break;
+                    case 192: launch_gk1_pairs_b3<192>(p, t1, ph.count, w, st); break;
+                    default: launch_gk1_pairs_b3<128>(p, t1, ph.count, w, st); break;
+                    }
+                } else switch (ph.bn * 2 + ph.mapped) {
                 case 640: launch_gk1_b3<false, 320>(p, t1, ph.count, w, st); break;
                 case 641: launch_gk1_b3<true, 320>(p, t1, ph.count, w, st); break;
                 case 512: launch_gk1_b3<false, 256>(p, t1, ph.count, w, st); break;

@@ -124,6 +124,38 @@ __global__ __launch_bounds__(kb3::Step1Cfg<BN>::THREADS) void k_step1_b3(
                                 Rlo + z * strideL, ldr, it * kb3::BM, kt * BN, lds);
 }
 
+// The pair-tile step 1, tiles ordered as k_step1_pairs.
+template <int BN, typename Src>
+__global__ __launch_bounds__(kb3::Step1Cfg<BN>::THREADS) void k_step1_pairs_b3(
+    const Src *__restrict__ cderi, long ld, int nL, tiles::View tv, const unsigned *__restrict__ fp, unsigned ldp,
+    b3::u16 *Rhi, b3::u16 *Rlo, long ldr, long strideL, int nkt, long ntiles) {
+    __shared__ b3::u16 lds[kb3::Step1Cfg<BN>::S::LDS_ELEMS];
+    const long x = xcd_tile(blockIdx.x, gridDim.x);
+    if (x >= ntiles) return;
+    const int kt = (int)(x % nkt);
+    const long y = x / nkt;
+    const int g = tv.ngroup - 1 - (int)(y % tv.ngroup);
+    const long L = y / tv.ngroup * tiles::NL;
+    kb3::step1_pairs_tile<BN, Src>(cderi + L * ld, ld, (int)min((long)tiles::NL, nL - L), tv, g, fp, ldp,
+                                   Rhi + L * strideL, Rlo + L * strideL, ldr, strideL, kt * BN, lds);
+}
+
+__global__ __launch_bounds__(256) void k_pack_split(const double *__restrict__ F, long ldf, int nao, int nocc,
+                                                    unsigned *fp, long ldp) {
+    const long e0 = (long)blockIdx.x * 1024;
+    kb3::pack_split_range(F, ldf, nao, nocc, fp, ldp, e0, min(e0 + 1024, (long)(nao + 1) * ldp));
+}
+
+template <int BN, typename Src>
+void launch_step1_pairs_b3(int nL, hipStream_t st, const Src *blk, long ld, const tiles::View &tv, const kb3::Side &q,
+                           const kb3::Layout &y, long strideL) {
+    const int nkt = (int)(y.ldp / BN);
+    const long ntiles = (long)nkt * tv.ngroup * cdiv(nL, tiles::NL);
+    hipLaunchKernelGGL((k_step1_pairs_b3<BN, Src>), dim3((unsigned)round_xcd(ntiles)),
+                       dim3(kb3::Step1Cfg<BN>::THREADS), 0, st, blk, ld, nL, tv, (const unsigned *)q.fthi,
+                       (unsigned)y.ldp, q.rhi, q.rlo, y.ldr, strideL, nkt, ntiles);
+}
+
 template <int BN, typename Src>
 void launch_step1_b3(int nL, hipStream_t st, const Src *blk, long ld, const int *pmap, int nao,
                      const b3::u16 *fthi, const b3::u16 *ftlo, long ldft, int nocc, b3::u16 *rhi, b3::u16 *rlo,
@@ -280,43 +312,41 @@ int run_k(const KPlan &p, const Src *cderi, long naux, long ld, const int *pair_
 
 // The block loop of mdf_get_k on the split-BF16 engine.
 template <typename Src>
-int run_k_b3(const KPlan &p, const Src *cderi, long naux, long ld, const int *pair_map, int nao,
+int run_k_b3(const KPlan &p, const Src *cderi, long naux, long ld, const int *pair_map, const void *pair_tiles, int nao,
              const double *fl, const double *fr, int nocc, long ldf, double *vk, long ldvk, int accumulate,
              void *work, hipStream_t st) {
     const bool two = fr != nullptr;
-    const kb3::Layout y = kb3::layout(nao, nocc, p.nL, p.ksplit, two);
+    const kb3::Layout y = kb3::layout(nao, nocc, p.nL, p.ksplit, two, pair_tiles != nullptr);
     double *part = (double *)work;
     kb3::Side sd[2] = {kb3::side_ptrs((char *)work, y, 0), kb3::side_ptrs((char *)work, y, two ? 1 : 0)};
     const long strideL = (long)nao * y.ldr, part_stride = (long)nao * nao;
-    const long nft = (long)nocc * y.ldft;
+    const long nft = pair_tiles ? (long)(nao + 1) * y.ldp : (long)nocc * y.ldft;
     for (int side = 0; side < (two ? 2 : 1); side++) {
-        hipLaunchKernelGGL(k_split_ft, dim3((unsigned)cdiv(nft, 1024L)), dim3(256), 0, st, side ? fr : fl, ldf, nao,
-                           nocc, sd[side].fthi, sd[side].ftlo, y.ldft);
+        if (pair_tiles)
+            hipLaunchKernelGGL(k_pack_split, dim3((unsigned)cdiv(nft, 1024L)), dim3(256), 0, st, side ? fr : fl, ldf,
+                               nao, nocc, (unsigned *)sd[side].fthi, y.ldp);
+        else
+            hipLaunchKernelGGL(k_split_ft, dim3((unsigned)cdiv(nft, 1024L)), dim3(256), 0, st, side ? fr : fl, ldf,
+                               nao, nocc, sd[side].fthi, sd[side].ftlo, y.ldft);
         MDF_LAUNCHED("k_split_ft");
     }
+    auto step1 = [&](auto width, int nL, const Src *blk, const kb3::Side &q) {
+        constexpr int BN = decltype(width)::value;
+        if (pair_tiles)
+            launch_step1_pairs_b3<BN>(nL, st, blk, ld, tiles::view(pair_tiles, nao), q, y, strideL);
+        else
+            launch_step1_b3<BN>(nL, st, blk, ld, pair_map, nao, q.fthi, q.ftlo, y.ldft, nocc, q.rhi, q.rlo, y.ldr,
+                                strideL);
+    };
     for (long L0 = 0; L0 < naux; L0 += p.nL) {
         const int nL = (int)(naux - L0 < p.nL ? naux - L0 : p.nL);
         const Src *blk = cderi + L0 * ld;
-        const int bn = kb3::pick_bn(y.ldr);
         for (int side = 0; side < (two ? 2 : 1); side++) {
-            const kb3::Side &q = sd[side];
-            switch (bn) {
-            case 320:
-                launch_step1_b3<320>(nL, st, blk, ld, pair_map, nao, q.fthi, q.ftlo, y.ldft, nocc, q.rhi, q.rlo,
-                                     y.ldr, strideL);
-                break;
-            case 256:
-                launch_step1_b3<256>(nL, st, blk, ld, pair_map, nao, q.fthi, q.ftlo, y.ldft, nocc, q.rhi, q.rlo,
-                                     y.ldr, strideL);
-                break;
-            case 192:
-                launch_step1_b3<192>(nL, st, blk, ld, pair_map, nao, q.fthi, q.ftlo, y.ldft, nocc, q.rhi, q.rlo,
-                                     y.ldr, strideL);
-                break;
-            default:
-                launch_step1_b3<128>(nL, st, blk, ld, pair_map, nao, q.fthi, q.ftlo, y.ldft, nocc, q.rhi, q.rlo,
-                                     y.ldr, strideL);
-                break;
+            switch (kb3::pick_bn(y.ldr)) {
+            case 320: step1(std::integral_constant<int, 320>{}, nL, blk, sd[side]); break;
+            case 256: step1(std::integral_constant<int, 256>{}, nL, blk, sd[side]); break;
+            case 192: step1(std::integral_constant<int, 192>{}, nL, blk, sd[side]); break;
+            default: step1(std::integral_constant<int, 128>{}, nL, blk, sd[side]); break;
             }
             MDF_LAUNCHED("k_step1_b3");
         }
@@ -351,7 +381,7 @@ static long k_rows_rule(long naux, int nao, int nocc, bool two, int prec) {
 }
 static size_t k_bytes(long naux, int nao, int nocc, bool two, int prec, long rows, bool pairs) {
     KPlan p = plan_k(naux, nao, nocc, two, rows, prec == MDF_PREC_FP32 ? sizeof(float) : sizeof(double));
-    if (prec == MDF_PREC_BF16X3) return kb3::layout(nao, nocc, p.nL, p.ksplit, two).total;
+    if (prec == MDF_PREC_BF16X3) return kb3::layout(nao, nocc, p.nL, p.ksplit, two, pairs).total;
     return k_workspace(p, two, prec == MDF_PREC_FP32 ? sizeof(float) : sizeof(double),
                        pairs ? pack_words(p, nao, nocc) : 0);
 }
@@ -426,7 +456,8 @@ extern "C" int mdf_get_k_tiles(const void *cderi, int cderi_dtype, long naux, lo
     if (cderi_dtype == MDF_DTYPE_F32) {
         const float *c = (const float *)cderi;
         if (prec == MDF_PREC_BF16X3)
-            return run_k_b3(p, c, naux, ld, pair_map, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate, work, st);
+            return run_k_b3(p, c, naux, ld, pair_map, pair_tiles, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate, work,
+                            st);
         if (prec == MDF_PREC_FP32)
             return run_k<float>(p, c, naux, ld, pair_map, pair_tiles, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate,
                                  work, st);
@@ -435,7 +466,8 @@ extern "C" int mdf_get_k_tiles(const void *cderi, int cderi_dtype, long naux, lo
     }
     const double *c = (const double *)cderi;
     if (prec == MDF_PREC_BF16X3)
-        return run_k_b3(p, c, naux, ld, pair_map, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate, work, st);
+        return run_k_b3(p, c, naux, ld, pair_map, pair_tiles, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate, work,
+                            st);
     if (prec == MDF_PREC_FP32)
         return run_k<float>(p, c, naux, ld, pair_map, pair_tiles, nao, fl, fr, nocc, ldf, vk, ldvk, accumulate,
                                  work, st);

@@ -624,6 +624,36 @@ inline int pick_bn(long ldr) {
     return best;
 }
 
+// Writes one plane at a time: the split 128 x BN tile through LDS (freed by
+// the mainloop's last barrier), then whole 16-byte runs of 8 columns at
+// dst(row) + chunk-major offset of (AO row, column).
+template <int BN, class AccT, class Row>
+__device__ __forceinline__ void put_split_tile(const AccT &acc, u16 *Rhi, u16 *Rlo, int nao, long ldr, int k0, u16 *lds,
+                                               Row &&row) {
+    using C = Step1Cfg<BN>;
+    constexpr int P = BN + 8;                  // row pitch (u16), 16-byte multiple
+    constexpr int CH = BN / 8;                 // 16-byte runs per row
+    static_assert(BM * P <= C::S::LDS_ELEMS, "one output plane must fit the tile's LDS");
+    for (int plane = 0; plane < 2; plane++) {
+        u16 *R = plane ? Rlo : Rhi;
+        b3::epilogue<BM, BN, 2, C::WGN>(acc, [&](int r, int c, float v) {
+            u16 h, l;
+            b3::split(v, h, l);
+            lds[r * P + c] = plane ? l : h;
+        });
+        __syncthreads();
+        // ldr and k0 are multiples of 32: a run lies inside or outside ldr
+        for (int u = threadIdx.x; u < BM * CH; u += C::THREADS) {
+            const int r = u / CH, c = (u % CH) * 8, k = k0 + c;
+            long off;
+            const int i = row(r, off);
+            if (i >= 0 && k < ldr)
+                *reinterpret_cast<uint4 *>(R + off + r_index(nao, i, k)) = *reinterpret_cast<const uint4 *>(lds + r * P + c);
+        }
+        __syncthreads();
+    }
+}
+
 // One 128 x BN tile of step 1 for the cderi row `row`: rows i0.., columns
 // k0.. of the split R planes (row stride ldr; columns nocc..ldr-1 get zeros).
 template <bool MAPPED, int BN, typename Src = double>
@@ -636,29 +666,140 @@ __device__ __forceinline__ void step1_tile(const Src *__restrict__ row, const in
     b3::Acc32<C::S::MI, C::S::NI> acc;
     acc.zero();
     b3::mainloop<BM, BN, 2, C::WGN>(la, lb, (nao + b3::BK - 1) / b3::BK, lds, acc);
-    // The split tile leaves through LDS one plane at a time (the mainloop's
-    // last barrier has freed it): each lane puts its MFMA results at their
-    // (row, column), then every thread writes whole 16-byte runs of 8
-    // columns.  ldr and k0 are multiples of 32, so a run lies entirely inside
-    // or outside ldr.
-    constexpr int P = BN + 8;                  // row pitch (u16), 16-byte multiple
-    constexpr int CH = BN / 8;                 // 16-byte runs per row
-    static_assert(BM * P <= C::S::LDS_ELEMS, "one output plane must fit the tile's LDS");
-    for (int plane = 0; plane < 2; plane++) {
-        u16 *R = plane ? Rlo : Rhi;
-        b3::epilogue<BM, BN, 2, C::WGN>(acc, [&](int r, int c, float v) {
-            u16 h, l;
-            b3::split(v, h, l);
-            lds[r * P + c] = plane ? l : h;
-        });
-        __syncthreads();
-        for (int u = threadIdx.x; u < BM * CH; u += C::THREADS) {
-            const int r = u / CH, c = (u % CH) * 8;
-            const int i = i0 + r, k = k0 + c;
-            if (i < nao && k < ldr)
-                *reinterpret_cast<uint4 *>(R + r_index(nao, i, k)) = *reinterpret_cast<const uint4 *>(lds + r * P + c);
+    put_split_tile<BN>(acc, Rhi, Rlo, nao, ldr, k0, lds, [&](int r, long &off) {
+        off = 0;
+        return i0 + r < nao ? i0 + r : -1;
+    });
+}
+
+// ---- step 1 on pair tiles (mdf_tiles.h): a K-step is 32 columns of the
+// group, two steps of its map.
+// A operand: a thread owns two neighbouring columns of one AO row and N of the
+// 8 aux rows, so its LDS stores are whole 4-byte pairs and 16 lanes read 32
+// consecutive columns.  As in tiles::ALoader every lane loads.
+template <int THREADS, typename Src>
+struct PairsA32 {
+    using reg_t = Src;
+    static constexpr int NLT = 2048 / THREADS;           // aux rows: 4 (512 threads) or 8 (256)
+    static constexpr int N = 2 * NLT;
+    const char *row[NLT];
+    const int *map;
+    int ii, jp, l0;
+    int2 pm;                  // the next step's map entries, read one call ahead
+    bool s0, s1;              // the loaded step's: stored
+    __device__ __forceinline__ void init(const Src *c, long ld, int nl, const int *gmap) {
+        const int t = threadIdx.x;
+        jp = t & 15;
+        ii = (t >> 4) & 15;
+        l0 = (__builtin_amdgcn_readfirstlane(t >> 6) >> 2) * NLT;
+#pragma unroll
+        for (int v = 0; v < NLT; v++) row[v] = (const char *)(c + (long)min(l0 + v, nl - 1) * ld);
+        map = gmap + (jp >> 3) * 256 + ii * 16 + (2 * jp & 15);
+        pm = *(const int2 *)map;
+    }
+    __device__ __forceinline__ void load(int kt, Src (&r)[N]) {
+        const unsigned o0 = (unsigned)max(pm.x, 0) * (unsigned)sizeof(Src);
+        const unsigned o1 = (unsigned)max(pm.y, 0) * (unsigned)sizeof(Src);
+#pragma unroll
+        for (int v = 0; v < NLT; v++) {
+            r[2 * v] = *(const Src *)(row[v] + o0);
+            r[2 * v + 1] = *(const Src *)(row[v] + o1);
         }
-        __syncthreads();
+        s0 = pm.x >= 0;
+        s1 = pm.y >= 0;
+        pm = *(const int2 *)(map + (kt + 1) * 512);
+    }
+    __device__ __forceinline__ void store(const Src (&r)[N], u16 *hi, u16 *lo) const {
+#pragma unroll
+        for (int v = 0; v < NLT; v++) {
+            unsigned h, m;
+            b3::split2(s0 ? (float)r[2 * v] : 0.f, s1 ? (float)r[2 * v + 1] : 0.f, h, m);
+            const int at = ((l0 + v) * tiles::RB + ii) * b3::PK + 2 * jp;
+            *(unsigned *)(hi + at) = h;
+            *(unsigned *)(lo + at) = m;
+        }
+    }
+};
+
+// B operand: eight factor rows (columns of the group, uniform over a
+// wavefront) at one occupied index per unit, each value hi << 16 | lo of the
+// packed factor; the octet leaves as 16 bytes of each plane.
+template <int BN, int THREADS>
+struct PairsB32 {
+    using reg_t = unsigned;
+    static constexpr int UNITS = 4 * BN, Q = (UNITS + THREADS - 1) / THREADS;
+    static constexpr int N = 8 * Q;
+    static_assert(BN % 64 == 0, "a wavefront stays in one octet");
+    const unsigned *base;     // packed factor at the tile's first column
+    const int *cols;
+    unsigned ldp;
+    int oct[Q], n[Q];         // this thread's units (the last repeated past the end)
+    __device__ __forceinline__ void init(const unsigned *fp, unsigned ldp_, int k0, const int *gcols) {
+        base = fp + k0;
+        cols = gcols;
+        ldp = ldp_;
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const int w = min(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + q * (THREADS / 64), UNITS / 64 - 1);
+            oct[q] = w / (BN / 64);
+            n[q] = w % (BN / 64) * 64 + (threadIdx.x & 63);
+        }
+    }
+    __device__ __forceinline__ void load(int kt, unsigned (&r)[N]) const {
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const int *c = cols + kt * b3::BK + oct[q] * 8;
+#pragma unroll
+            for (int e = 0; e < 8; e++) r[q * 8 + e] = (base + (unsigned long)((unsigned)c[e] * ldp))[n[q]];
+        }
+    }
+    __device__ __forceinline__ void store(const unsigned (&r)[N], u16 *hi, u16 *lo) const {
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            uint4 h, m;
+            unsigned *hs = (unsigned *)&h, *ms = (unsigned *)&m;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                hs[e] = __builtin_amdgcn_perm(r[q * 8 + 2 * e + 1], r[q * 8 + 2 * e], 0x07060302);
+                ms[e] = __builtin_amdgcn_perm(r[q * 8 + 2 * e + 1], r[q * 8 + 2 * e], 0x05040100);
+            }
+            *(uint4 *)(hi + n[q] * b3::PK + oct[q] * 8) = h;
+            *(uint4 *)(lo + n[q] * b3::PK + oct[q] * 8) = m;
+        }
+    }
+};
+
+// The step-1 tile of one group of pair tiles, as kcore::step1_pairs_tile;
+// strideL between the planes of aux rows.
+template <int BN, typename Src>
+__device__ __forceinline__ void step1_pairs_tile(const Src *__restrict__ c, long ld, int nl, const tiles::View &tv, int g,
+                                                 const unsigned *__restrict__ fp, unsigned ldp, u16 *Rhi, u16 *Rlo,
+                                                 long ldr, long strideL, int k0, u16 *lds) {
+    using C = Step1Cfg<BN>;
+    PairsA32<C::THREADS, Src> la;
+    PairsB32<BN, C::THREADS> lb;
+    la.init(c, ld, nl, tv.map + (long)g * tv.ccap * tiles::RB);
+    lb.init(fp, ldp, k0, tv.cols + (long)g * tv.ccap);
+    b3::Acc32<C::S::MI, C::S::NI> acc;
+    acc.zero();
+    b3::mainloop<BM, BN, 2, C::WGN>(la, lb, (tv.nstep[g] + 1) / 2, lds, acc);
+    const int *rows = tv.rows + g * tiles::RB;
+    put_split_tile<BN>(acc, Rhi, Rlo, tv.nao, ldr, k0, lds, [&](int r, long &off) {
+        const int l = r / tiles::RB;
+        off = l * strideL;
+        return l < nl ? rows[r % tiles::RB] : -1;
+    });
+}
+
+// Fp[j][k] = F[j][k] split, hi << 16 | lo; zero for k in nocc..ldp-1 and in
+// row nao.
+__device__ __forceinline__ void pack_split_range(const double *__restrict__ F, long ldf, int nao, int nocc, unsigned *fp,
+                                                 long ldp, long e0, long e1) {
+    for (long e = e0 + threadIdx.x; e < e1; e += blockDim.x) {
+        const int j = (int)(e / ldp), k = (int)(e - (long)j * ldp);
+        u16 h, l;
+        b3::split(j < nao && k < nocc ? (float)F[(long)j * ldf + k] : 0.f, h, l);
+        fp[e] = (unsigned)h << 16 | l;
     }
 }
 
@@ -739,33 +880,38 @@ __device__ __forceinline__ void split_ft_range(const double *__restrict__ F, lon
 // Workspace layout of one item (bytes from its base): step-2 partials, then
 // per factor side the FT planes and the R planes.
 struct Layout {
-    long ldr, ldft;
+    long ldr, ldft, ldp;
     size_t ft_elems, r_elems;        // per plane
-    size_t part_bytes, side_bytes, total;
+    size_t ft_bytes, part_bytes, side_bytes, total;
 };
 
-inline Layout layout(int nao, int nocc, long nL, int ksplit, bool two) {
+// pairs: the packed factor of the pair tiles (rows of ldp) in the place of
+// the FT planes
+inline Layout layout(int nao, int nocc, long nL, int ksplit, bool two, bool pairs) {
     Layout y;
     y.ldr = pad32(nocc);
     y.ldft = pad32(nao);
     y.ft_elems = (size_t)nocc * y.ldft;
     y.r_elems = (size_t)nL * nao * y.ldr;
+    const int bn = pick_bn(y.ldr);
+    y.ldp = (y.ldr + bn - 1) / bn * bn;
+    y.ft_bytes = align_up(pairs ? (size_t)(nao + 1) * y.ldp * sizeof(unsigned) : 2 * y.ft_elems * sizeof(u16), 256);
     y.part_bytes = align_up((size_t)ksplit * nao * nao * sizeof(double), 256);
-    y.side_bytes = align_up(2 * y.ft_elems * sizeof(u16), 256) + align_up(2 * y.r_elems * sizeof(u16), 256);
+    y.side_bytes = y.ft_bytes + align_up(2 * y.r_elems * sizeof(u16), 256);
     y.total = y.part_bytes + (two ? 2 : 1) * y.side_bytes;
     return y;
 }
 
 // pointers of one side (0 left, 1 right) inside an item's workspace
 struct Side {
-    u16 *fthi, *ftlo, *rhi, *rlo;
+    u16 *fthi, *ftlo, *rhi, *rlo;    // fthi: the packed factor with pair tiles
 };
 inline Side side_ptrs(char *base, const Layout &y, int side) {
     char *b = base + y.part_bytes + side * y.side_bytes;
     Side s;
     s.fthi = (u16 *)b;
     s.ftlo = s.fthi + y.ft_elems;
-    s.rhi = (u16 *)(b + align_up(2 * y.ft_elems * sizeof(u16), 256));
+    s.rhi = (u16 *)(b + y.ft_bytes);
     s.rlo = s.rhi + y.r_elems;
     return s;
 }

@@ -125,8 +125,8 @@ int mdf_get_k(const void *cderi, int cderi_dtype, long naux, long npairs, long l
  * groups, own-group pairs halved), for mdf_k_step1_tiles; order_of, another
  * buffer of the same map or NULL, gives the row order.
  * mdf_get_k_tiles is mdf_get_k with step 1 on the tiles (pair_tiles NULL:
- * mdf_get_k itself; MDF_PREC_BF16X3 uses the pair map either way); npairs <
- * 2^29.  Its workspace also holds the packed factors. */
+ * mdf_get_k itself); npairs < 2^29.  Its workspace also holds the packed
+ * factors. */
 size_t mdf_pair_tiles_bytes(int nao);
 int mdf_build_pair_tiles(const int *pair_map, int nao, int lower, const void *order_of, void *tiles,
                          size_t tiles_bytes, void *stream);

@@ -101,6 +101,21 @@ def test_k_tiles_types(storage, prec, nao, naux, nocc):
     assert rel(vk, exact_k(cderi, rows, cols, nao, fl, None)) < tol
 
 
+@pytest.mark.parametrize('storage', ['float32', 'float64'])
+@pytest.mark.parametrize('two', [False, True])
+@pytest.mark.parametrize('nao,naux,nocc', [(33, 9, 17), (64, 8, 128), (130, 12, 161), (97, 7, 256), (150, 5, 320)])
+def test_k_tiles_split_bf16(storage, two, nao, naux, nocc):
+    print(f'k tiles bf16x3 {storage} two {two} nao {nao} naux {naux} nocc {nocc}', flush=True)
+    cderi, rows, cols, addr, fl, fr = inputs(nao, naux, nocc, two, storage)
+    pmap, buf = make_tiles(addr, nao)
+    ref = exact_k(cderi, rows, cols, nao, fl, fr)
+    vk = get_k(cderi, pmap, buf, nao, fl, fr, 2)
+    # hi + lo holds 2^-17 of a value and the dropped lo lo term is below
+    # 2^-16 of a product, in each of two steps
+    assert rel(vk, ref) < 4 * 2. ** -16
+    assert rel(vk, ref) < 1.2 * rel(get_k(cderi, pmap, None, nao, fl, fr, 2), ref) + 1e-7
+
+
 def test_k_tiles_passes():
     """Passes of fewer aux rows than a block of 8, and of several blocks."""
     cderi, rows, cols, addr, fl, _ = inputs(60, 37, 20, False)
