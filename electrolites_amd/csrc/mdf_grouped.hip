@@ -61,10 +61,10 @@ struct GKItem {
     void *rl, *rr;          // transformed blocks (T), nL aux rows each
     double *part;           // ksplit x nao x nao
     long nL;                // aux rows per pass
-    int nao, nocc, ksplit, ntile;
+    int nao, nocc, ksplit, ntile, s2;
     // split-BF16 (prec 2): workspace offsets of [side][FT hi, FT lo, R hi, R lo]
     void *b3[2][4];
-    long ldr, ldft;         // R row stride (FP64/FP32: kcore::r_ld; split-BF16: a multiple of 32), FT row stride
+    long ldr, ldft;         // R row stride (split-BF16; FP64/FP32: 8 nocc), FT row stride
     int bn3;                // split-BF16 step-1 tile width (kb3::pick_bn(ldr))
     int bn1;                // FP64/FP32 step-1 tile width (the plan's bn, or kcore::pick_bn(nocc))
     const void *tiles;      // FP64/FP32: the pair map's tiles, or NULL
@@ -188,7 +188,8 @@ __global__ __launch_bounds__(kcore::Step1Shape<BN>::THREADS) void gk_step1(const
         const int ktile = e.c & 0xffff;
         const double *F = right ? it.fr : it.fl;
         const long lb = e.a % it.nL;        // row within the pass
-        T *R = (T *)(work + (size_t)(right ? it.rr : it.rl)) + lb * it.nao * it.ldr;
+        T *R = (T *)(work + (size_t)(right ? it.rr : it.rl)) + lb / kcore::RL * it.nao * it.ldr +
+               lb % kcore::RL * it.nocc;
         const Src *row = (const Src *)it.cderi + (long)e.a * it.ld;
         if (it.pmap)
             kcore::step1_tile<BN, true, T, Src>(row, it.pmap, it.nao, F, it.nocc, it.nocc, R, it.ldr, e.b * 128,
@@ -212,12 +213,12 @@ __global__ __launch_bounds__(kcore::Step1Shape<BN>::THREADS, 2) void gk_step1_pa
         const int side = e.c >> 16, ktile = e.c & 0xffff;
         const long lb = e.a % it.nL;        // row within the pass
         const long end = min(e.a - lb + it.nL, it.naux);
-        T *R = (T *)(work + (size_t)(side ? it.rr : it.rl)) + lb * it.nao * it.ldr;
+        T *R = (T *)(work + (size_t)(side ? it.rr : it.rl)) + lb / kcore::RL * it.nao * it.ldr;
         kcore::step1_pairs_tile<BN, T, Src, false>((const Src *)it.cderi + (long)e.a * it.ld, it.ld,
                                                    (int)min((long)tiles::NL, end - e.a),
                                                    tiles::view(it.tiles, it.nao), e.b,
                                                    (const T *)(work + (size_t)it.fp[side]), (unsigned)it.ldp, it.nocc,
-                                                   R, it.ldr, (long)it.nao * it.ldr, ktile * BN, lds);
+                                                   R, it.ldr, it.nocc, ktile * BN, lds);
         __syncthreads();
     }
 }
@@ -233,10 +234,10 @@ __global__ __launch_bounds__(256) void gk_pack_factor(const GKItem *items, const
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(G_THREADS, 2) void gk_step2(const GKItem *items, const Tile *tiles, long n,
+template <int B, typename T>
+__global__ __launch_bounds__(G_THREADS, B == 64 ? 4 : 2) void gk_step2(const GKItem *items, const Tile *tiles, long n,
                                                          char *work) {
-    __shared__ T lds[TileShape<kcore::S2_B, kcore::S2_B>::LDS_ELEMS];
+    __shared__ T lds[TileShape<B, B>::LDS_ELEMS];
     for (long t = blockIdx.x; t < n; t += gridDim.x) {
         const Tile e = tiles[t];            // (item, tile index, split, pass)
         const GKItem &it = items[e.item];
@@ -249,14 +250,13 @@ __global__ __launch_bounds__(G_THREADS, 2) void gk_step2(const GKItem *items, co
             ti = e.a / it.ntile;
             tj = e.a % it.ntile;
         }
-        const int kchunks = (it.nocc + G_BK - 1) / G_BK;
-        const long nsteps = nLb * kchunks;
+        const kcore::RShape y(nLb, it.nocc);
+        const long nsteps = y.steps();
         const long s0 = nsteps * e.b / it.ksplit, s1 = nsteps * (e.b + 1) / it.ksplit;
         const T *rl = (const T *)(work + (size_t)it.rl);
         const T *rr = it.fr ? (const T *)(work + (size_t)it.rr) : rl;
         double *o = (double *)(work + (size_t)it.part) + (long)e.b * it.nao * it.nao;
-        kcore::step2_tile<T>(rl, rr, it.nao, it.nocc, it.ldr, (long)it.nao * it.ldr, ti * kcore::S2_B,
-                             tj * kcore::S2_B, s0, s1, o, e.c > 0, lds);
+        kcore::step2_tile<B, T>(rl, rr, it.nao, y, ti * B, tj * B, s0, s1, o, e.c > 0, lds);
         __syncthreads();
     }
 }
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(256) void gk_finalize(const GKItem *items, const Ti
         const GKItem &it = items[e.item];
         const long nn = (long)it.nao * it.nao;
         const long e0 = (long)e.a * RED_CHUNK, e1 = min(e0 + RED_CHUNK, nn);
-        kcore::finalize_range((const double *)(work + (size_t)it.part), it.ksplit, nn, it.nao, it.fr == nullptr,
+        kcore::finalize_range((const double *)(work + (size_t)it.part), it.ksplit, nn, it.nao, it.fr ? 0 : it.s2,
                               it.vk, it.nao, 0, e0, e1);
     }
 }
@@ -381,8 +381,8 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
     MDF_CHECK_ARG(items && nitems >= 0 && out && work_bytes, "mdf_grouped_plan_create: null argument");
     MDF_CHECK_ARG(prec == MDF_PREC_FP64 || prec == MDF_PREC_FP32 || prec == MDF_PREC_BF16X3,
                   "mdf_grouped_plan_create: precision %d", prec);
-    MDF_CHECK_ARG(bn == 0 || bn == 64 || bn == 128 || bn == 160 || bn == 192 || bn == 256 || bn == 320,
-                  "mdf_grouped_plan_create: bn %d not in {0,64,128,160,192,256,320}", bn);
+    MDF_CHECK_ARG(bn == 0 || bn == 32 || bn == 64 || bn == 96 || bn == 128 || bn == 160 || bn == 192 || bn == 256 || bn == 320,
+                  "mdf_grouped_plan_create: bn %d not in {0,32,64,96,128,160,192,256,320}", bn);
     for (int m = 0; m < nitems; m++)
         MDF_CHECK_ARG(items[m].cderi_dtype == items[0].cderi_dtype &&
                           (items[m].cderi_dtype == MDF_DTYPE_F64 || items[m].cderi_dtype == MDF_DTYPE_F32),
@@ -446,14 +446,14 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
             const bool b3 = prec == MDF_PREC_BF16X3;
             const long nL = b3 ? kcore::block_rows(x.naux, x.nao, (int)kcore::kb3::pad32(x.nocc), two, 4)
                                : kcore::block_rows(x.naux, x.nao, x.nocc, two, elem);
-            kcore::KPlan kp = kcore::plan_k(x.naux, x.nao, x.nocc, two, nL, b3 ? sizeof(double) : elem);
+            kcore::KPlan kp = kcore::plan_k(x.naux, x.nao, x.nocc, two, nL, b3);
             for (int d = 0; d < x.n_dm; d++) {
                 GKItem g{};
                 g.cderi = x.cderi; g.ld = x.ld; g.naux = x.naux; g.pmap = x.pair_map;
                 g.fl = x.fl + (long)d * x.nao * x.nocc;
                 g.fr = two ? x.fr + (long)d * x.nao * x.nocc : nullptr;
                 g.vk = x.vk + (long)d * x.nao * x.nao;
-                g.nao = x.nao; g.nocc = x.nocc; g.ksplit = kp.ksplit; g.ntile = kp.ntile;
+                g.nao = x.nao; g.nocc = x.nocc; g.ksplit = kp.ksplit; g.ntile = kp.ntile; g.s2 = kp.s2;
                 g.nL = kp.nL;
                 g.bn1 = bn ? bn : kcore::pick_bn(x.nocc);
                 if (x.pair_tiles) {
@@ -477,7 +477,7 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
                     g.rl = (void *)0;
                     g.part = (double *)y.total;
                 } else {
-                    g.ldr = kcore::r_ld(x.nocc, elem);
+                    g.ldr = (long)kcore::RL * x.nocc;
                     g.rl = (void *)(align_up(kp.r_words * elem, 256));
                     g.part = (double *)(align_up(kp.part_words * sizeof(double), 256));
                 }
@@ -552,10 +552,10 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
           // one step-1 launch per tile width and per form of the pairs (0 the
           // full triangle, or for FP64/FP32 a pair map too; 1 a pair map
           // (split-BF16) or pair tiles; 2 pair tiles (split-BF16))
-          for (int cls = 0; cls < 12; cls++) {
+          for (int cls = 0; cls < (b3 ? 12 : 16); cls++) {
             static const int kBN3[4] = {128, 192, 256, 320};
-            static const int kBN1[6] = {64, 128, 160, 192, 256, 320};
-            const int mp = cls / (b3 ? 4 : 6), cbn = b3 ? kBN3[cls % 4] : kBN1[cls % 6];
+            static const int kBN1[8] = {32, 64, 96, 128, 160, 192, 256, 320};
+            const int mp = cls / (b3 ? 4 : 8), cbn = b3 ? kBN3[cls % 4] : kBN1[cls % 8];
             const long s1 = k1.size();
             for (size_t i = w0; i < w1; i++) {
                 const GKItem &g = p->hk[i];
@@ -587,10 +587,12 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
             });
             p->kphases.push_back({1, s1, (long)k1.size() - s1, cbn, mp});
           }
+            // one step-2 launch per output tile width
+            for (int width : {64, 128}) {
             const long s2 = k2.size();
             for (size_t i = w0; i < w1; i++) {
                 const GKItem &g = p->hk[i];
-                if (b * g.nL >= g.naux) continue;
+                if (b * g.nL >= g.naux || g.s2 != width) continue;
                 for (int s = 0; s < g.ksplit; s++)
                     for (int tl = 0; tl < kgrid[i]; tl++) k2.push_back({(int)i, tl, s, (int)b});
             }
@@ -599,12 +601,12 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
             auto s2cost = [&](const Tile &x) {
                 const GKItem &g = p->hk[x.item];
                 const long nLb = std::min(g.nL, g.naux - (long)x.c * g.nL);
-                const long kc = prec == MDF_PREC_BF16X3 ? g.ldr / b3::BK : cdiv((long)g.nocc, (long)G_BK);
-                return nLb * kc / g.ksplit;
+                return (prec == MDF_PREC_BF16X3 ? nLb * (g.ldr / b3::BK) : kcore::RShape(nLb, g.nocc).steps()) / g.ksplit;
             };
             std::stable_sort(k2.begin() + s2, k2.end(),
                              [&](const Tile &x, const Tile &y) { return s2cost(x) > s2cost(y); });
-            p->kphases.push_back({2, s2, (long)k2.size() - s2, 0, 0});
+            p->kphases.push_back({2, s2, (long)k2.size() - s2, width, 0});
+            }
         }
         const long sf = kf.size();
         for (size_t i = w0; i < w1; i++) {
@@ -733,6 +735,15 @@ static void launch_gk1(const mdf_grouped_plan *p, const Tile *tiles, long n, int
         launch_gk1_s<BN, double>(p, tiles, n, pairs, w, st);
 }
 
+template <int B>
+static void launch_gk2(const mdf_grouped_plan *p, const Tile *tab, long n, char *w, hipStream_t st) {
+    const dim3 g(persistent_grid(n, B == 64 ? 4 : 2)), b(G_THREADS);
+    if (p->prec == MDF_PREC_FP32)
+        hipLaunchKernelGGL((gk_step2<B, float>), g, b, 0, st, p->kitems, tab, n, w);
+    else
+        hipLaunchKernelGGL((gk_step2<B, double>), g, b, 0, st, p->kitems, tab, n, w);
+}
+
 template <bool MAPPED, int BN>
 static void launch_gk1_b3(const mdf_grouped_plan *p, const Tile *tiles, long n, char *w, hipStream_t st) {
     // one workgroup per CU (the 192-, 256- and 320-wide tiles hold 100-140 KB of LDS)
@@ -824,23 +835,15 @@ extern "C" int mdf_grouped_jk(const mdf_grouped_plan *p, void *work, size_t work
                 MDF_LAUNCHED("gk_step2_b3");
             } else if (ph.kind == 1) {
                 const Tile *t = p->k1 + ph.start;
-                switch (ph.bn) {
-                case 320: launch_gk1<320>(p, t, ph.count, ph.mapped, w, st); break;
-                case 256: launch_gk1<256>(p, t, ph.count, ph.mapped, w, st); break;
-                case 192: launch_gk1<192>(p, t, ph.count, ph.mapped, w, st); break;
-                case 160: launch_gk1<160>(p, t, ph.count, ph.mapped, w, st); break;
-                case 128: launch_gk1<128>(p, t, ph.count, ph.mapped, w, st); break;
-                default: launch_gk1<64>(p, t, ph.count, ph.mapped, w, st); break;
-                }
+                kcore::with_bn(ph.bn, [&](auto bw) {
+                    launch_gk1<decltype(bw)::value>(p, t, ph.count, ph.mapped, w, st);
+                });
                 MDF_LAUNCHED("gk_step1");
             } else if (ph.kind == 2) {
-                const int g2 = persistent_grid(ph.count, 2);
-                if (p->prec == MDF_PREC_FP32)
-                    hipLaunchKernelGGL(gk_step2<float>, dim3(g2), dim3(G_THREADS), 0, st, p->kitems,
-                                       p->k2 + ph.start, ph.count, w);
+                if (ph.bn == 64)
+                    launch_gk2<64>(p, p->k2 + ph.start, ph.count, w, st);
                 else
-                    hipLaunchKernelGGL(gk_step2<double>, dim3(g2), dim3(G_THREADS), 0, st, p->kitems,
-                                       p->k2 + ph.start, ph.count, w);
+                    launch_gk2<128>(p, p->k2 + ph.start, ph.count, w, st);
                 MDF_LAUNCHED("gk_step2");
             } else {
                 hipLaunchKernelGGL(gk_finalize, dim3(persistent_grid(ph.count, 4)), dim3(256), 0, st, p->kitems,

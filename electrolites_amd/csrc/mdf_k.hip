@@ -37,14 +37,14 @@ template <int BN, bool MAPPED, typename T, typename Src, bool TRI = false>
 __global__ __launch_bounds__(Step1Shape<BN>::THREADS) void k_step1(
     const Src *__restrict__ cderi, long ld, const int *__restrict__ pmap, int nao,
     const double *__restrict__ F, long ldf, int nocc, T *__restrict__ R, long ldr,
-    long strideL, int nkt, int nit, long ntiles) {
+    long strideL, long strideB, int nkt, int nit, long ntiles) {
     __shared__ T lds[Step1Shape<BN>::S::LDS_ELEMS];
     const long x = xcd_tile(blockIdx.x, gridDim.x);
     if (x >= ntiles) return;
     const int kt = (int)(x % nkt), it = (int)((x / nkt) % nit);
     const long L = x / ((long)nkt * nit);
-    step1_tile<BN, MAPPED, T, Src, TRI>(cderi + L * ld, pmap, nao, F, ldf, nocc, R + L * strideL, ldr, it * 128,
-                                        kt * BN, lds);
+    step1_tile<BN, MAPPED, T, Src, TRI>(cderi + L * ld, pmap, nao, F, ldf, nocc,
+                                        R + L / RL * strideB + L % RL * strideL, ldr, it * 128, kt * BN, lds);
 }
 
 // The pair-tile step 1: 1-D grid of round_xcd(nkt * ngroup * blocks of 8 aux
@@ -54,16 +54,16 @@ __global__ __launch_bounds__(Step1Shape<BN>::THREADS) void k_step1(
 template <int BN, typename T, typename Src, bool HALVES>
 __global__ __launch_bounds__(Step1Shape<BN>::THREADS, 2) void k_step1_pairs(
     const Src *__restrict__ cderi, long ld, int nL, tiles::View tv, const T *__restrict__ fp, unsigned ldp, int nocc,
-    T *__restrict__ R, long ldr, long strideL, int nkt, long ntiles) {
+    T *__restrict__ R, long ldr, long strideL, long strideB, int nkt, long ntiles) {
     __shared__ T lds[Step1Shape<BN>::S::LDS_ELEMS];
     const long x = xcd_tile(blockIdx.x, gridDim.x);
     if (x >= ntiles) return;
     const int kt = (int)(x % nkt);
     const long y = x / nkt;
     const int g = tv.ngroup - 1 - (int)(y % tv.ngroup);
-    const long L = y / tv.ngroup * tiles::NL;
+    const long b = y / tv.ngroup, L = b * tiles::NL;
     step1_pairs_tile<BN, T, Src, HALVES>(cderi + L * ld, ld, (int)min((long)tiles::NL, nL - L), tv, g, fp, ldp, nocc,
-                                         R + L * strideL, ldr, strideL, kt * BN, lds);
+                                         R + b * strideB, ldr, strideL, kt * BN, lds);
 }
 
 template <typename T>
@@ -74,12 +74,11 @@ __global__ __launch_bounds__(256) void k_pack_factor(const double *__restrict__ 
 }
 
 // 1-D grid of ntiles_grid * ksplit workgroups, (tile, split) by step2_coords.
-template <bool SYM, typename T>
-__global__ __launch_bounds__(G_THREADS, 2) void k_step2(
-    const T *__restrict__ Rl, const T *__restrict__ Rr, int nao, int nocc,
-    long ldr, long strideL, int nL, int ntile, int ntiles_grid, int ksplit, double *__restrict__ part,
-    long part_stride, int beta) {
-    __shared__ T lds[TileShape<S2_B, S2_B>::LDS_ELEMS];
+template <int B, bool SYM, typename T>
+__global__ __launch_bounds__(G_THREADS, B == 64 ? 4 : 2) void k_step2(
+    const T *__restrict__ Rl, const T *__restrict__ Rr, int nao, RShape y, int ntile, int ntiles_grid, int ksplit,
+    double *__restrict__ part, long part_stride, int beta) {
+    __shared__ T lds[TileShape<B, B>::LDS_ELEMS];
     int tile, split, ti, tj;
     step2_coords(blockIdx.x, ntiles_grid, tile, split);
     if (SYM) {
@@ -88,11 +87,9 @@ __global__ __launch_bounds__(G_THREADS, 2) void k_step2(
         ti = tile / ntile;
         tj = tile % ntile;
     }
-    const int kchunks = (nocc + G_BK - 1) / G_BK;
-    const long nsteps = (long)nL * kchunks;
+    const long nsteps = y.steps();
     const long s0 = nsteps * split / ksplit, s1 = nsteps * (split + 1) / ksplit;
-    step2_tile<T>(Rl, Rr, nao, nocc, ldr, strideL, ti * S2_B, tj * S2_B, s0, s1,
-                       part + (long)split * part_stride, beta, lds);
+    step2_tile<B, T>(Rl, Rr, nao, y, ti * B, tj * B, s0, s1, part + (long)split * part_stride, beta, lds);
 }
 
 __global__ __launch_bounds__(256) void k_finalize(
@@ -193,55 +190,46 @@ __global__ __launch_bounds__(G_THREADS, 2) void k_step2_b3(
 
 template <int BN, typename T, typename Src, bool TRI = false>
 void launch_step1(int nL, hipStream_t st, const Src *blk, long ld, const int *pmap, int nao,
-                  const double *f, long ldf, int nocc, T *r, long ldr, long strideL) {
+                  const double *f, long ldf, int nocc, T *r, long ldr, long strideL, long strideB) {
     const int nkt = (int)cdiv(nocc, BN), nit = (int)cdiv(nao, 128);
     const long ntiles = (long)nkt * nit * nL;
     const dim3 g((unsigned)round_xcd(ntiles)), b(Step1Shape<BN>::THREADS);
     if (pmap)
         hipLaunchKernelGGL((k_step1<BN, true, T, Src, TRI>), g, b, 0, st, blk, ld, pmap, nao, f, ldf,
-                           nocc, r, ldr, strideL, nkt, nit, ntiles);
+                           nocc, r, ldr, strideL, strideB, nkt, nit, ntiles);
     else
         hipLaunchKernelGGL((k_step1<BN, false, T, Src, TRI>), g, b, 0, st, blk, ld, pmap, nao, f, ldf,
-                           nocc, r, ldr, strideL, nkt, nit, ntiles);
+                           nocc, r, ldr, strideL, strideB, nkt, nit, ntiles);
 }
 
 template <typename T, typename Src, bool TRI = false>
 int step1(const KPlan &p, int nL, hipStream_t st, const Src *blk, long ld, const int *pmap, int nao,
-          const double *f, long ldf, int nocc, T *r, long ldr, long strideL) {
-    switch (p.bn) {
-    case 320: launch_step1<320, T, Src, TRI>(nL, st, blk, ld, pmap, nao, f, ldf, nocc, r, ldr, strideL); break;
-    case 256: launch_step1<256, T, Src, TRI>(nL, st, blk, ld, pmap, nao, f, ldf, nocc, r, ldr, strideL); break;
-    case 192: launch_step1<192, T, Src, TRI>(nL, st, blk, ld, pmap, nao, f, ldf, nocc, r, ldr, strideL); break;
-    case 160: launch_step1<160, T, Src, TRI>(nL, st, blk, ld, pmap, nao, f, ldf, nocc, r, ldr, strideL); break;
-    case 128: launch_step1<128, T, Src, TRI>(nL, st, blk, ld, pmap, nao, f, ldf, nocc, r, ldr, strideL); break;
-    default: launch_step1<64, T, Src, TRI>(nL, st, blk, ld, pmap, nao, f, ldf, nocc, r, ldr, strideL); break;
-    }
+          const double *f, long ldf, int nocc, T *r, long ldr, long strideL, long strideB) {
+    with_bn(p.bn, [&](auto w) {
+        launch_step1<decltype(w)::value, T, Src, TRI>(nL, st, blk, ld, pmap, nao, f, ldf, nocc, r, ldr, strideL,
+                                                      strideB);
+    });
     MDF_LAUNCHED("k_step1");
     return MDF_OK;
 }
 
 template <int BN, typename T, typename Src, bool HALVES>
 void launch_step1_pairs(int nL, hipStream_t st, const Src *blk, long ld, const tiles::View &tv, const T *fp,
-                        unsigned ldp, int nocc, T *r, long ldr, long strideL) {
+                        unsigned ldp, int nocc, T *r, long ldr, long strideL, long strideB) {
     const int nkt = (int)cdiv(nocc, BN);
     const long ntiles = (long)nkt * tv.ngroup * cdiv(nL, tiles::NL);
     hipLaunchKernelGGL((k_step1_pairs<BN, T, Src, HALVES>), dim3((unsigned)round_xcd(ntiles)),
-                       dim3(Step1Shape<BN>::THREADS), 0, st, blk, ld, nL, tv, fp, ldp, nocc, r, ldr, strideL, nkt,
-                       ntiles);
+                       dim3(Step1Shape<BN>::THREADS), 0, st, blk, ld, nL, tv, fp, ldp, nocc, r, ldr, strideL, strideB,
+                       nkt, ntiles);
 }
 
 template <typename T, typename Src, bool HALVES = false>
 int step1_pairs(const KPlan &p, int nL, hipStream_t st, const Src *blk, long ld, const tiles::View &tv, const T *fp,
-                int nocc, T *r, long ldr, long strideL) {
-    const unsigned ldp = pack_ld(p, nocc);
-    switch (p.bn) {
-    case 320: launch_step1_pairs<320, T, Src, HALVES>(nL, st, blk, ld, tv, fp, ldp, nocc, r, ldr, strideL); break;
-    case 256: launch_step1_pairs<256, T, Src, HALVES>(nL, st, blk, ld, tv, fp, ldp, nocc, r, ldr, strideL); break;
-    case 192: launch_step1_pairs<192, T, Src, HALVES>(nL, st, blk, ld, tv, fp, ldp, nocc, r, ldr, strideL); break;
-    case 160: launch_step1_pairs<160, T, Src, HALVES>(nL, st, blk, ld, tv, fp, ldp, nocc, r, ldr, strideL); break;
-    case 128: launch_step1_pairs<128, T, Src, HALVES>(nL, st, blk, ld, tv, fp, ldp, nocc, r, ldr, strideL); break;
-    default: launch_step1_pairs<64, T, Src, HALVES>(nL, st, blk, ld, tv, fp, ldp, nocc, r, ldr, strideL); break;
-    }
+                int nocc, T *r, long ldr, long strideL, long strideB) {
+    with_bn(p.bn, [&](auto w) {
+        launch_step1_pairs<decltype(w)::value, T, Src, HALVES>(nL, st, blk, ld, tv, fp, pack_ld(p, nocc), nocc, r, ldr,
+                                                               strideL, strideB);
+    });
     MDF_LAUNCHED("k_step1_pairs");
     return MDF_OK;
 }
@@ -255,16 +243,26 @@ int pack_factor(const KPlan &p, hipStream_t st, const double *f, long ldf, int n
     return MDF_OK;
 }
 
-template <typename T>
-int step2(const KPlan &p, int nL, bool two, hipStream_t st, const T *rl, const T *rr, int nao, int nocc,
-          long ldr, long strideL, double *part, long part_stride, int beta) {
+template <int B, typename T>
+void launch_step2(const KPlan &p, int nL, bool two, hipStream_t st, const T *rl, const T *rr, int nao, int nocc,
+                  double *part, long part_stride, int beta) {
     const dim3 g2((unsigned)((long)p.ntiles_grid * p.ksplit));
+    const RShape y(nL, nocc);
     if (two)
-        hipLaunchKernelGGL((k_step2<false, T>), g2, dim3(G_THREADS), 0, st, rl, rr, nao, nocc, ldr, strideL, nL,
-                           p.ntile, p.ntiles_grid, p.ksplit, part, part_stride, beta);
+        hipLaunchKernelGGL((k_step2<B, false, T>), g2, dim3(G_THREADS), 0, st, rl, rr, nao, y, p.ntile, p.ntiles_grid,
+                           p.ksplit, part, part_stride, beta);
     else
-        hipLaunchKernelGGL((k_step2<true, T>), g2, dim3(G_THREADS), 0, st, rl, rl, nao, nocc, ldr, strideL, nL,
-                           p.ntile, p.ntiles_grid, p.ksplit, part, part_stride, beta);
+        hipLaunchKernelGGL((k_step2<B, true, T>), g2, dim3(G_THREADS), 0, st, rl, rl, nao, y, p.ntile, p.ntiles_grid,
+                           p.ksplit, part, part_stride, beta);
+}
+
+template <typename T>
+int step2(const KPlan &p, int nL, bool two, hipStream_t st, const T *rl, const T *rr, int nao, int nocc, double *part,
+          long part_stride, int beta) {
+    if (p.s2 == 64)
+        launch_step2<64, T>(p, nL, two, st, rl, rr, nao, nocc, part, part_stride, beta);
+    else
+        launch_step2<128, T>(p, nL, two, st, rl, rr, nao, nocc, part, part_stride, beta);
     MDF_LAUNCHED("k_step2");
     return MDF_OK;
 }
@@ -286,7 +284,7 @@ int run_k(const KPlan &p, const Src *cderi, long naux, long ld, const int *pair_
     if (pair_tiles)
         for (int side = 0; side < (two ? 2 : 1); side++)
             if (int rc = pack_factor<T>(p, st, side ? fr : fl, ldf, nao, nocc, fp[side])) return rc;
-    const long ldr = r_ld(nocc, sizeof(T)), strideL = (long)nao * ldr;
+    const long ldr = (long)RL * nocc, strideB = (long)nao * ldr;
     const long part_stride = (long)nao * nao;
     for (long L0 = 0; L0 < naux; L0 += p.nL) {
         const int nL = (int)(naux - L0 < p.nL ? naux - L0 : p.nL);
@@ -295,17 +293,17 @@ int run_k(const KPlan &p, const Src *cderi, long naux, long ld, const int *pair_
         for (int side = 0; side < (two ? 2 : 1); side++) {
             T *r = side ? rr : rl;
             rc = pair_tiles ? step1_pairs<T, Src>(p, nL, st, blk, ld, tiles::view(pair_tiles, nao), fp[side], nocc, r,
-                                                  ldr, strideL)
+                                                  ldr, nocc, strideB)
                             : step1<T, Src>(p, nL, st, blk, ld, pair_map, nao, side ? fr : fl, ldf, nocc, r, ldr,
-                                            strideL);
+                                            nocc, strideB);
             if (rc) return rc;
         }
-        rc = step2<T>(p, nL, two, st, rl, rr, nao, nocc, ldr, strideL, part, part_stride, L0 > 0);
+        rc = step2<T>(p, nL, two, st, rl, rr, nao, nocc, part, part_stride, L0 > 0);
         if (rc) return rc;
     }
     long nt = (long)nao * nao;
     hipLaunchKernelGGL(k_finalize, dim3((unsigned)cdiv(nt, 256L)), dim3(256), 0, st,
-                       part, p.ksplit, part_stride, nao, two ? 0 : 1, vk, ldvk, accumulate);
+                       part, p.ksplit, part_stride, nao, two ? 0 : p.s2, vk, ldvk, accumulate);
     MDF_LAUNCHED("k_finalize");
     return MDF_OK;
 }
@@ -362,7 +360,7 @@ int run_k_b3(const KPlan &p, const Src *cderi, long naux, long ld, const int *pa
     }
     long nt = (long)nao * nao;
     hipLaunchKernelGGL(k_finalize, dim3((unsigned)cdiv(nt, 256L)), dim3(256), 0, st,
-                       part, p.ksplit, part_stride, nao, two ? 0 : 1, vk, ldvk, accumulate);
+                       part, p.ksplit, part_stride, nao, two ? 0 : p.s2, vk, ldvk, accumulate);
     MDF_LAUNCHED("k_finalize");
     return MDF_OK;
 }
@@ -380,7 +378,7 @@ static long k_rows_rule(long naux, int nao, int nocc, bool two, int prec) {
     return block_rows(naux, nao, nocc, two, prec == MDF_PREC_FP32 ? sizeof(float) : sizeof(double));
 }
 static size_t k_bytes(long naux, int nao, int nocc, bool two, int prec, long rows, bool pairs) {
-    KPlan p = plan_k(naux, nao, nocc, two, rows, prec == MDF_PREC_FP32 ? sizeof(float) : sizeof(double));
+    KPlan p = plan_k(naux, nao, nocc, two, rows, prec == MDF_PREC_BF16X3);
     if (prec == MDF_PREC_BF16X3) return kb3::layout(nao, nocc, p.nL, p.ksplit, two, pairs).total;
     return k_workspace(p, two, prec == MDF_PREC_FP32 ? sizeof(float) : sizeof(double),
                        pairs ? pack_words(p, nao, nocc) : 0);
@@ -452,7 +450,7 @@ extern "C" int mdf_get_k_tiles(const void *cderi, int cderi_dtype, long naux, lo
         }
         rows = lo;
     }
-    KPlan p = plan_k(naux, nao, nocc, two, rows, prec == MDF_PREC_FP32 ? sizeof(float) : sizeof(double));
+    KPlan p = plan_k(naux, nao, nocc, two, rows, prec == MDF_PREC_BF16X3);
     if (cderi_dtype == MDF_DTYPE_F32) {
         const float *c = (const float *)cderi;
         if (prec == MDF_PREC_BF16X3)
@@ -499,9 +497,9 @@ int k_step1_entry(const char *name, const void *cderi, int cderi_dtype, long nL,
     hipStream_t st = as_stream(stream);
     if (cderi_dtype == MDF_DTYPE_F32)
         return step1<double, float, TRI>(p, (int)nL, st, (const float *)cderi, ld, pair_map, nao, f, ldf, nocc, R,
-                                         ldr, strideL);
+                                         ldr, strideL, RL * strideL);
     return step1<double, double, TRI>(p, (int)nL, st, (const double *)cderi, ld, pair_map, nao, f, ldf, nocc, R,
-                                      ldr, strideL);
+                                         ldr, strideL, RL * strideL);
 }
 }  // namespace
 

@@ -207,54 +207,70 @@ __device__ __forceinline__ void step1_pairs_tile(const Src *__restrict__ c, long
 }
 
 // ---------------------------------------------------------------- step 2
-// Rows r0..r0+127 of R[L] (k contiguous); K-step kt of this split is
-// (L, kc) = divmod(s0 + kt, kchunks), columns kc*16 .. kc*16 + 15.  Rows of R
-// are whole 16-byte pieces (r_ld); the lanes of a row take its pieces, as in
-// RowsLoader.
-template <typename T>
+// The transformed blocks: the occupied columns of 8 aux rows side by side,
+// R[L / 8][i][(L % 8) nocc + k], row stride ldr = 8 nocc.  Step 2's reduction
+// runs over a block's 8 nocc columns in K-steps of 16 (one aux row at a time
+// it computed nocc rounded up to 16: 96 columns for 81, 64 for 50).
+constexpr int RL = tiles::NL;
+
+// Columns of a block's row that hold values: fewer in a pass's last block.
+struct RShape {
+    int nocc, ldr, kchunks, nfull, lastcols;
+    __host__ __device__ __forceinline__ RShape(long nL, int nocc_)
+        : nocc(nocc_), ldr(RL * nocc_), kchunks((RL * nocc_ + G_BK - 1) / G_BK), nfull((int)(nL / RL)),
+          lastcols((int)(nL % RL) * nocc_) {}
+    __host__ __device__ __forceinline__ long steps() const {
+        return (long)nfull * kchunks + (lastcols + G_BK - 1) / G_BK;
+    }
+};
+
+// Rows r0..r0+ROWS-1 of the blocks; K-step kt of this split is (block, kc) =
+// divmod(s0 + kt, kchunks), columns kc*16 .. kc*16 + 15.  The lanes of a row
+// take its 16-byte pieces, as in RowsLoader.
+template <typename T, int ROWS>
 struct TransformedLoader {
     using reg_t = T;
-    static constexpr int N = 128 * G_BK / G_THREADS;     // 8
+    static constexpr int N = ROWS * G_BK / G_THREADS;
     static constexpr int EPV = 16 / (int)sizeof(T);      // elements per 16-byte piece
     static constexpr int Q = N / EPV, LPR = G_BK / EPV, RPP = G_THREADS / LPR;
     static constexpr int SWZ = sizeof(T) == 8 ? 2 : 3;
+    static_assert(Q >= 1 && Q * RPP == ROWS, "TransformedLoader shape");
     const T *R;
-    long strideL;
-    int nocc, kchunks;
+    long strideB;
+    RShape y;
     unsigned off[Q];     // this thread's rows
     int last;            // its column in a row's last, ragged chunk
-    long L;              // current aux row of the next load()
-    int kc;              // current k chunk of the next load()
+    long b;              // block and
+    int kc;              // chunk of the next load()
     int left;            // columns in range of the loaded chunk
-    __device__ __forceinline__ TransformedLoader(const T *R_, long strideL_, long ldr, int r0, int nao, int nocc_,
-                                                 int kchunks_, long L_, int kc_)
-        : R(R_), strideL(strideL_), nocc(nocc_), kchunks(kchunks_), L(L_), kc(kc_) {
+    __device__ __forceinline__ TransformedLoader(const T *R_, long strideB_, const RShape &y_, int r0, int nao, long b_,
+                                                 int kc_)
+        : R(R_), strideB(strideB_), y(y_), b(b_), kc(kc_) {
         const int c = (int)(threadIdx.x % LPR) * EPV;
 #pragma unroll
         for (int q = 0; q < Q; q++)
-            off[q] = (unsigned)((long)min(r0 + (int)(threadIdx.x / LPR) + q * RPP, nao - 1) * ldr) + c;
-        last = min((kchunks - 1) * G_BK + c, (int)ldr - EPV) - c;
+            off[q] = (unsigned)min(r0 + (int)(threadIdx.x / LPR) + q * RPP, nao - 1) * (unsigned)y.ldr + c;
+        last = min((y.kchunks - 1) * G_BK + c, y.ldr - EPV) - c;
     }
     __device__ __forceinline__ void load(int, T (&r)[N]) {
-        // called for kt = 0, 1, 2, ... in order: advance (L, kc) in place
-        const bool ragged = (kc + 1) * G_BK > nocc;
-        const T *src = R + L * strideL + (ragged ? last : kc * G_BK);
+        // called for kt = 0, 1, 2, ... in order: advance (b, kc) in place
+        const T *src = R + b * strideB + ((kc + 1) * G_BK > y.ldr ? last : kc * G_BK);
 #pragma unroll
         for (int q = 0; q < Q; q++) {
             const Piece<T, EPV> x = *(const Piece<T, EPV> *)(src + off[q]);
 #pragma unroll
             for (int e = 0; e < EPV; e++) r[q * EPV + e] = x.v[e];
         }
-        left = nocc - kc * G_BK;
-        if (++kc == kchunks) {
+        left = (b < y.nfull ? y.ldr : y.lastcols) - kc * G_BK;
+        if (++kc == y.kchunks) {
             kc = 0;
-            ++L;
+            ++b;
         }
     }
     __device__ __forceinline__ void store(T (&r)[N], T *lds, int pitch) const {
         const int k = (int)(threadIdx.x % LPR) * EPV;
         if (left < G_BK) {
-            // columns nocc.. are not written: zero, whatever they hold
+            // columns past the last hold nothing: zero, whatever is there
 #pragma unroll
             for (int e = 0; e < N; e++)
                 if (k + e % EPV >= left) r[e] = (T)0;
@@ -265,24 +281,23 @@ struct TransformedLoader {
     }
 };
 
-constexpr int S2_B = 128;
+constexpr double S2_64_COST = 1.25;
+constexpr int S2_B = 128;              // split-BF16 step-2 tile; FP64/FP32: KPlan::s2 (64 or 128)
 // FP32 step 2 adds its MFMA accumulators into an FP64 shadow every S2_FLUSH
 // K-steps (S2_FLUSH * 16 products per element), so the rounding error of the
 // long (L, k) reduction grows with the flush length, not with naux * nocc.
 constexpr int S2_FLUSH = 32;
 
-// One 128 x 128 output tile (i0, j0) of step 2 over the K-steps [s0, s1) of
-// the (L, k-chunk) reduction; writes (beta = 0) or adds (beta = 1) into o.
-template <typename T>
-__device__ __forceinline__ void step2_tile(const T *__restrict__ Rl, const T *__restrict__ Rr, int nao, int nocc, long ldr,
-                                  long strideL, int i0, int j0, long s0, long s1, double *__restrict__ o, int beta,
-                                  T *lds) {
-    using S = TileShape<S2_B, S2_B>;
-    const int kchunks = (nocc + G_BK - 1) / G_BK;
-    const long Ls = s0 / kchunks;
-    const int kcs = (int)(s0 - Ls * kchunks);
-    TransformedLoader<T> la{Rl, strideL, ldr, i0, nao, nocc, kchunks, Ls, kcs};
-    TransformedLoader<T> lb{Rr, strideL, ldr, j0, nao, nocc, kchunks, Ls, kcs};
+// One B x B output tile (i0, j0) of step 2 over the K-steps [s0, s1) of the
+// (block, chunk) reduction; writes (beta = 0) or adds (beta = 1) into o.
+template <int B, typename T>
+__device__ __forceinline__ void step2_tile(const T *__restrict__ Rl, const T *__restrict__ Rr, int nao, const RShape &y,
+                                  int i0, int j0, long s0, long s1, double *__restrict__ o, int beta, T *lds) {
+    using S = TileShape<B, B>;
+    const long b0 = s0 / y.kchunks, strideB = (long)nao * y.ldr;
+    const int kc0 = (int)(s0 - b0 * y.kchunks);
+    TransformedLoader<T, B> la{Rl, strideB, y, i0, nao, b0, kc0};
+    TransformedLoader<T, B> lb{Rr, strideB, y, j0, nao, b0, kc0};
     Acc<S::MI, S::NI, T> acc;
     auto emit = [&](int r, int c, double v) {
         const int i = i0 + r, j = j0 + c;
@@ -293,16 +308,16 @@ __device__ __forceinline__ void step2_tile(const T *__restrict__ Rl, const T *__
     };
     if constexpr (sizeof(T) == 8) {
         acc.zero();
-        gemm_mainloop<S2_B, S2_B>(la, lb, (int)(s1 - s0), lds, acc);
-        gemm_epilogue<S2_B, S2_B, T>(acc, emit);
+        gemm_mainloop<B, B>(la, lb, (int)(s1 - s0), lds, acc);
+        gemm_epilogue<B, B, T>(acc, emit);
     } else {
         Acc<S::MI, S::NI, double> sum;
         sum.zero();
         for (long s = s0; s < s1; s += S2_FLUSH) {
             acc.zero();
-            // the loaders advance (L, k-chunk) in place, so consecutive calls
-            // continue the reduction where the previous one stopped
-            gemm_mainloop<S2_B, S2_B>(la, lb, (int)min((long)S2_FLUSH, s1 - s), lds, acc);
+            // the loaders advance in place, so consecutive calls continue the
+            // reduction where the previous one stopped
+            gemm_mainloop<B, B>(la, lb, (int)min((long)S2_FLUSH, s1 - s), lds, acc);
 #pragma unroll
             for (int a = 0; a < S::MI; a++)
 #pragma unroll
@@ -310,7 +325,7 @@ __device__ __forceinline__ void step2_tile(const T *__restrict__ Rl, const T *__
 #pragma unroll
                     for (int v = 0; v < 4; v++) sum.v[a][b][v] += (double)acc.v[a][b][v];
         }
-        gemm_epilogue_layout<S2_B, S2_B, T>(sum, emit);
+        gemm_epilogue_layout<B, B, T>(sum, emit);
     }
 }
 
@@ -322,27 +337,33 @@ __device__ __forceinline__ void tri_tile(int x, int &ti, int &tj) {
     tj = x - ti * (ti + 1) / 2;
 }
 
-// vk[i, j] (+)= sum_s part[s, I, J] for the flat range [e0, e1); SYM reads the
-// lower-tile copy for upper-tile entries.
+// vk[i, j] (+)= sum_s part[s, I, J] for the flat range [e0, e1); sym, the
+// step-2 tile width or 0, reads the lower-tile copy for upper-tile entries.
 __device__ __forceinline__ void finalize_range(const double *__restrict__ part, int ksplit, long part_stride, int nao,
                                       int sym, double *__restrict__ vk, long ldvk, int accumulate, long e0, long e1) {
     for (long t = e0 + threadIdx.x; t < e1; t += 256) {
         const int i = (int)(t / nao), j = (int)(t % nao);
         int I = i, J = j;
-        if (sym && (i / S2_B) < (j / S2_B)) { I = j; J = i; }
+        if (sym && (i / sym) < (j / sym)) { I = j; J = i; }
+        const double *src = part + (long)I * nao + J;
         double s = 0.;
-        for (int k = 0; k < ksplit; k++) s += part[k * part_stride + (long)I * nao + J];
+        for (int k = 0; k < ksplit; k += 8) {        // ksplit is a multiple of 8
+            double x[8];
+#pragma unroll
+            for (int v = 0; v < 8; v++) x[v] = src[(k + v) * part_stride];
+#pragma unroll
+            for (int v = 0; v < 8; v++) s += x[v];
+        }
         double *dst = vk + (long)i * ldvk + j;
         *dst = accumulate ? *dst + s : s;
     }
 }
 
-// step-1 N tile: the width in {64, 128, 160} that pads nocc least (ties: wider)
 // step-1 tile width: each k-tile re-reads the cderi tile (worth about 64
 // columns of MFMA work), so minimise nkt * (64 + BN) over the widths; ties
 // go to the wider tile
 inline int pick_bn(int nocc) {
-    const int cand[6] = {64, 128, 160, 192, 256, 320};
+    const int cand[8] = {32, 64, 96, 128, 160, 192, 256, 320};
     // MDF_K_STEP1_BN forces one of the widths (for tuning runs)
     if (const char *e = getenv("MDF_K_STEP1_BN")) {
         const int v = atoi(e);
@@ -358,41 +379,56 @@ inline int pick_bn(int nocc) {
     return best;
 }
 
+// f(integral constant of the step-1 tile width)
+template <class F>
+void with_bn(int bn, F &&f) {
+    switch (bn) {
+    case 320: f(std::integral_constant<int, 320>{}); break;
+    case 256: f(std::integral_constant<int, 256>{}); break;
+    case 192: f(std::integral_constant<int, 192>{}); break;
+    case 160: f(std::integral_constant<int, 160>{}); break;
+    case 128: f(std::integral_constant<int, 128>{}); break;
+    case 96: f(std::integral_constant<int, 96>{}); break;
+    case 64: f(std::integral_constant<int, 64>{}); break;
+    default: f(std::integral_constant<int, 32>{}); break;
+    }
+}
+
 struct KPlan {
     int ntile, ntiles_grid, ksplit, bn;
-    long nL;            // aux rows per block
+    int s2;             // step-2 tile width
+    long nL;            // aux rows per pass
     size_t r_words;     // one R buffer
     size_t part_words;
 };
 
-// Resident step-2 workgroups on this device: 2 per CU (LDS and registers).
-inline int resident_step2_wgs() {
+inline int cu_count() {
     static int cached[64] = {0};
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 512;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
     if (!cached[dev]) {
         int cu = 0;
         if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0)
             cu = 256;
-        cached[dev] = 2 * cu;
+        cached[dev] = cu;
     }
     return cached[dev];
 }
 
-// Split of the (L, k) reduction: a multiple of the XCD count, so that each
-// XCD takes whole splits (step2_coords) and the output tiles running on one
-// XCD at a time read the same R panels through its L2; among 8, 16, 24, 32
-// the one whose per-XCD share fills whole rounds of resident workgroups
-// best (ties: the larger split).
-inline int pick_ksplit(int ntiles_grid) {
-    const int slots = resident_step2_wgs() / N_XCD;
+// Split of the (L, k) reduction of nsteps K-steps: a multiple of the XCD
+// count, so that each XCD takes whole splits (step2_coords) and the output
+// tiles running on one XCD at a time read the same R panels through its L2.
+// Of the splits of at least 8 K-steps, the one of least estimated time: the
+// rounds of resident workgroups (slots per XCD) each over its K-steps and
+// about 6 more to start and end, plus the partials written and read again
+// (nao^2 words each, 1.5e-6 K-steps a word).
+inline int pick_ksplit(int ntiles_grid, long nsteps, int nao, int slots) {
     int best = N_XCD;
-    double best_eff = -1.;
-    for (int ks = N_XCD; ks <= 4 * N_XCD; ks += N_XCD) {
-        const long items = (long)ntiles_grid * ks / N_XCD;
-        const long rounds = (items + slots - 1) / slots;
-        const double eff = (double)items / (double)(rounds * slots);
-        if (eff >= best_eff - 1e-9) { best_eff = eff; best = ks; }
+    double best_t = 1e300;
+    for (int ks = N_XCD; ks <= 256 && (ks == N_XCD || nsteps >= 8L * ks); ks += N_XCD) {
+        const long rounds = ((long)ntiles_grid * ks / N_XCD + slots - 1) / slots;
+        const double t = rounds * ((double)nsteps / ks + 6.) + 1.5e-6 * ks * nao * nao;
+        if (t < best_t) { best_t = t; best = ks; }
     }
     return best;
 }
@@ -431,26 +467,31 @@ inline long block_rows(long naux, int nao, int nocc, bool two, size_t elem) {
     const size_t per_row = (size_t)nao * nocc * elem * (two ? 2 : 1);
     long r = per_row ? (long)(k_block_bytes() / per_row) : naux;
     if (r > naux) r = naux;
+    if (r > RL && r < naux) r = r / RL * RL;
     return r < 1 ? 1 : r;
 }
 
-// Row stride of a transformed block R[L][i][k]: nocc rounded up to whole
-// 16-byte vectors, so step 2 streams every row with vector loads whatever
-// the parity of nocc (columns nocc..ldr-1 are never written or read).
-inline long r_ld(int nocc, size_t elem) {
-    const long e = 16 / (long)elem;
-    return (nocc + e - 1) / e * e;
-}
+// Words of one factor's transformed blocks of a pass of nL aux rows.
+inline size_t r_words(long nL, int nao, int nocc) { return (size_t)((nL + RL - 1) / RL) * nao * RL * nocc; }
 
-inline KPlan plan_k(long naux, int nao, int nocc, bool two, long max_rows, size_t elem = 8) {
+// b3: the split-BF16 kernels' plan (128-wide step-2 tiles).
+inline KPlan plan_k(long naux, int nao, int nocc, bool two, long max_rows, bool b3) {
     KPlan p;
-    p.ntile = (nao + S2_B - 1) / S2_B;
-    p.ntiles_grid = two ? p.ntile * p.ntile : p.ntile * (p.ntile + 1) / 2;
-    p.ksplit = pick_ksplit(p.ntiles_grid);
-    p.bn = pick_bn(nocc);
     p.nL = max_rows < naux ? max_rows : naux;
     if (p.nL < 1) p.nL = 1;
-    p.r_words = (size_t)p.nL * nao * r_ld(nocc, elem);
+    auto tiles = [&](int b) {
+        const int n = (nao + b - 1) / b;
+        return two ? n * n : n * (n + 1) / 2;
+    };
+    // 64-wide tiles cover a small result with less padding, at S2_64_COST
+    // times the time of a 128-wide tile's product per element
+    p.s2 = !b3 && S2_64_COST * tiles(64) * 64 * 64 < (double)tiles(128) * 128 * 128 ? 64 : 128;
+    p.ntile = (nao + p.s2 - 1) / p.s2;
+    p.ntiles_grid = tiles(p.s2);
+    const long nsteps = b3 ? p.nL * ((nocc + 31) / 32) : RShape(p.nL, nocc).steps();
+    p.ksplit = pick_ksplit(p.ntiles_grid, nsteps, nao, (p.s2 == 64 ? 4 : 2) * cu_count() / N_XCD);
+    p.bn = pick_bn(nocc);
+    p.r_words = r_words(p.nL, nao, nocc);
     p.part_words = (size_t)p.ksplit * nao * nao;
     return p;
 }
