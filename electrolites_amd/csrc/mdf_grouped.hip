@@ -48,7 +48,7 @@ struct GJItem {
     double *rho, *vj;       // (ndm, naux), (ndm, npairs)
     double *part1, *part2;  // workspace
     long nchunk, ngroup, rows_per_group, ncblock;
-    int ndm, vec;
+    int ndm, vec, rb;
 };
 
 // Per-(molecule, density) K work on the device.
@@ -124,9 +124,11 @@ __global__ __launch_bounds__(jcore::J_THREADS) void gj_pass1(const GJItem *items
         double *part = (double *)(work + (size_t)it.part1);
         const S *L = (const S *)it.cderi;
         if (it.vec == W)
-            jcore::rho_partial_tile<NDM, W, S>(L, it.ld, it.naux, it.npairs, it.d, it.npairs, it.ndm, part, e.a, e.b);
+            jcore::rho_partial_tile<NDM, W, S>(L, it.ld, it.naux, it.npairs, it.d, it.npairs, it.ndm, part, e.a, e.b,
+                                              it.rb);
         else
-            jcore::rho_partial_tile<NDM, 1, S>(L, it.ld, it.naux, it.npairs, it.d, it.npairs, it.ndm, part, e.a, e.b);
+            jcore::rho_partial_tile<NDM, 1, S>(L, it.ld, it.naux, it.npairs, it.d, it.npairs, it.ndm, part, e.a, e.b,
+                                              it.rb);
     }
 }
 
@@ -424,6 +426,7 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
             g.vec = ((x.ld % wvec == 0) && ((uintptr_t)x.cderi % 16 == 0)) ? wvec : 1;
             jcore::JPlan pl = jcore::plan_j(x.naux, x.npairs, x.n_dm, g.vec);
             g.nchunk = pl.nchunk; g.ngroup = pl.ngroup; g.rows_per_group = pl.rows_per_group; g.ncblock = pl.ncblock;
+            g.rb = pl.rb;
             g.part1 = (double *)take(pl.part1_words * sizeof(double));
             g.part2 = (double *)take(pl.part2_words * sizeof(double));
             const int ji = (int)p->hj.size();

@@ -27,8 +27,8 @@ namespace {
 template <int NDM, int VEC, typename S>
 __global__ __launch_bounds__(J_THREADS) void j_rho_partial(const S *__restrict__ L, long ld, long naux,
                                                            long npairs, const double *__restrict__ d, long ldd,
-                                                           double *__restrict__ part) {
-    rho_partial_tile<NDM, VEC, S>(L, ld, naux, npairs, d, ldd, NDM, part, blockIdx.x, blockIdx.y);
+                                                           double *__restrict__ part, int rb) {
+    rho_partial_tile<NDM, VEC, S>(L, ld, naux, npairs, d, ldd, NDM, part, blockIdx.x, blockIdx.y, rb);
 }
 
 __global__ __launch_bounds__(J_THREADS) void j_rho_reduce(const double *__restrict__ part, long nchunk, int ndm,
@@ -63,8 +63,8 @@ __global__ __launch_bounds__(J_THREADS) void j_vj_reduce(const double *__restric
 template <int NDM, int VEC, typename S>
 __global__ __launch_bounds__(J_THREADS) void jh_rho_partial(const S *__restrict__ L, long ld, long naux,
                                                             long npairs, const double *__restrict__ d, long ldd,
-                                                            double *__restrict__ part) {
-    rho_partial_tile<NDM, VEC, S>(L, ld, naux, npairs, d, ldd, NDM, part, blockIdx.x, blockIdx.y);
+                                                            double *__restrict__ part, int rb) {
+    rho_partial_tile<NDM, VEC, S>(L, ld, naux, npairs, d, ldd, NDM, part, blockIdx.x, blockIdx.y, rb);
 }
 
 __global__ __launch_bounds__(J_THREADS) void jh_rho_reduce(const double *__restrict__ part, long nchunk, int ndm,
@@ -105,7 +105,8 @@ int run_j_group(const S *L, long ld, long naux, long npairs, const double *d, lo
     if (passes & 1) {
         dim3 g1((unsigned)pl.nchunk, (unsigned)pl.nrblock);
         auto rho_partial = halves ? jh_rho_partial<NDM, VEC, S> : j_rho_partial<NDM, VEC, S>;
-        hipLaunchKernelGGL(rho_partial, g1, dim3(J_THREADS), 0, st, L, ld, naux, npairs, d, ldd, part1);
+        hipLaunchKernelGGL(rho_partial, g1, dim3(J_THREADS), 0, st, L, ld, naux, npairs, d, ldd, part1,
+                           pl.rb);
         MDF_LAUNCHED("j_rho_partial");
         nt = (long)NDM * naux;
         auto rho_reduce = halves ? jh_rho_reduce : j_rho_reduce;

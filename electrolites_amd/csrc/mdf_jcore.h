@@ -12,7 +12,7 @@ namespace jcore {
 
 constexpr int J_THREADS = 256;
 constexpr int J_LANE = 8;     // cderi values per lane per row (pass 1)
-constexpr int J_RB = 32;      // rows per pass-1 tile
+constexpr int J_RB = 32;      // most rows per pass-1 tile (JPlan::rb)
 
 // The cderi is stored in S = double or float (the FP32 storage mode: every
 // value is widened to FP64 before arithmetic).  A lane loads VEC values at a
@@ -43,13 +43,13 @@ __device__ __forceinline__ double wave_sum(double v) {
 }
 
 // Pass-1 tile (chunk, rblock): the density slice of a chunk_cols() column
-// chunk is held in registers and reused for J_RB rows; each row's partial dot
+// chunk is held in registers and reused for rb (at most J_RB) rows; each row's partial dot
 // product is reduced across the wavefront and the four wavefronts.
 // part[(chunk * ndm + n) * naux + r]; ndm <= NDM densities are live.
 template <int NDM, int VEC, typename S = double>
 __device__ __forceinline__ void rho_partial_tile(const S *__restrict__ L, long ld, long naux, long npairs,
                                         const double *__restrict__ d, long ldd, int ndm,
-                                        double *__restrict__ part, long chunk, long rblock) {
+                                        double *__restrict__ part, long chunk, long rblock, int rb) {
     constexpr int J_U = J_LANE / VEC;
     constexpr int WCOLS = 64 * VEC * J_U;
     constexpr int GCOLS = 4 * WCOLS;
@@ -70,8 +70,8 @@ __device__ __forceinline__ void rho_partial_tile(const S *__restrict__ L, long l
             }
 
     __shared__ double red[4][NDM][J_RB];
-    const long r0 = rblock * J_RB;
-    const int nr = (int)min((long)J_RB, naux - r0);
+    const long r0 = rblock * rb;
+    const int nr = (int)min((long)rb, naux - r0);
 
     for (int rr = 0; rr < nr; rr++) {
         const S *row = L + (r0 + rr) * ld;
@@ -211,6 +211,7 @@ __device__ __forceinline__ void vj_reduce_range(const double *__restrict__ part,
 struct JPlan {
     long nchunk;          // pass-1 column chunks
     long nrblock;         // pass-1 row blocks
+    int rb;               // rows per block
     long ngroup;          // pass-2 row groups
     long rows_per_group;
     long ncblock;         // pass-2 column blocks
@@ -222,7 +223,13 @@ inline JPlan plan_j(long naux, long npairs, int ndm, int vec) {
     JPlan p;
     const long gc = chunk_cols();
     p.nchunk = (npairs + gc - 1) / gc;
-    p.nrblock = (naux + J_RB - 1) / J_RB;
+    // a tile's rows are dependent steps (a reduction over the workgroup each,
+    // about 0.6 us): few tiles of them take fewer rows each, down to 4 (3
+    // waters: 22 tiles of 32 rows, 20 us a pass, 168 of 4 rows 5 us).  A row's
+    // sum does not depend on its block.
+    p.rb = J_RB;
+    while (p.rb > 4 && p.nchunk * ((naux + p.rb - 1) / p.rb) < 1024) p.rb /= 2;
+    p.nrblock = (naux + p.rb - 1) / p.rb;
     p.ncblock = (npairs + (long)J_THREADS * vec - 1) / ((long)J_THREADS * vec);
     long ng = 1;
     while (p.ncblock * ng < 4096 && naux / (ng * 2) >= 64) ng *= 2;

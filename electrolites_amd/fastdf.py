@@ -386,14 +386,23 @@ def factorize_dm(dms, hermi):
     if mo_coeff is not None and mo_occ is not None:
         c = _dev.to_device(mo_coeff)
         c = c.reshape(-1, nao, c.shape[-1])
+        # the occupations decide the shape: read once (a boolean index on the
+        # device reads back its count for every density and use)
+        occ_h = np.asarray(_dev.to_host(mo_occ), dtype=np.float64).reshape(c.shape[0], -1)
         occ = _dev.to_device(mo_occ).reshape(c.shape[0], -1)
-        facs = []
-        nocc = int(max(int((occ[i] > 0).sum()) for i in range(c.shape[0])))
+        sel = occ_h > 0
+        num = sel.sum(axis=1)
+        nocc = int(num.max())
+        if (num == c.shape[-1]).all():
+            return (c * t.sqrt(occ)[:, None, :]).contiguous(), None
         out = t.zeros((c.shape[0], nao, nocc), dtype=t.float64, device=c.device)
         for i in range(c.shape[0]):
-            sel = occ[i] > 0
-            f = c[i][:, sel] * t.sqrt(occ[i][sel])
-            out[i, :, :f.shape[1]] = f
+            n = int(num[i])
+            if sel[i, :n].all():                       # the leading columns
+                out[i, :, :n] = c[i, :, :n] * t.sqrt(occ[i, :n])
+            else:
+                k = _dev.to_device(np.flatnonzero(sel[i]), dtype=t.int64)
+                out[i, :, :n] = c[i][:, k] * t.sqrt(occ[i][k])
         return out.contiguous(), None
     d = _dev.to_device(dms).reshape(-1, nao, nao)
     fls, frs = [], []
