@@ -10,7 +10,7 @@
 //                   place), 128-wide panels: one-workgroup diagonal block
 //                   factorisation + inverse, panel = A21 inv(L11)^T, trailing
 //                   SYRK on the engine.  A non-positive pivot sets *info.
-//   mdf_trtri       X = L^-1 by block rows from the diagonal inverses
+//   mdf_trtri       X = L^-1 from the diagonal inverses by doubling
 //   mdf_trmm        C = L^-1 B with the triangular A bound folded into the
 //                   K loop (the cderi = L^-1 (P|pq) product).
 #include <cmath>
@@ -35,8 +35,9 @@ __device__ __forceinline__ void lower_tile(int x, int &ti, int &tj) {
 }
 
 // TRI: 0 = A general; 1 = A lower triangular (row block m reads k < m0 + 128);
-// 2 = A upper triangular (row block m reads k >= m0).  blockIdx.z is the
-// batch index (operand strides sA, sB, sC).
+// 2 = A upper triangular (row block m reads k >= m0); 3 = B lower triangular
+// (column block n reads k >= n0).  blockIdx.z is the batch index (operand
+// strides sA, sB, sC).
 template <int BN, bool BT, int TRI, bool LOWER_C>
 __global__ __launch_bounds__(G_THREADS, 2) void gemm_f64_kernel(
     int M, int N, int K, double alpha, const double *__restrict__ A, long lda, long sA,
@@ -50,11 +51,13 @@ __global__ __launch_bounds__(G_THREADS, 2) void gemm_f64_kernel(
     if (LOWER_C) {
         lower_tile(blockIdx.x, ti, tj);
     } else {
-        ti = blockIdx.y;
+        // a lower triangular A's last row blocks have the longest sums: they
+        // start first, so the launch does not end on them
+        ti = TRI == 1 ? gridDim.y - 1 - blockIdx.y : blockIdx.y;
         tj = blockIdx.x;
     }
     const int m0 = ti * 128, n0 = tj * BN;
-    const int k0 = TRI == 2 ? min(K, m0) : 0;
+    const int k0 = TRI == 2 ? min(K, m0) : TRI == 3 ? min(K, n0) : 0;
     const int kmax = TRI == 1 ? min(K, m0 + 128) : K;
     RowsLoader<128> la{A, lda, m0, M, k0, kmax};
     Acc<S::MI, S::NI> acc;
@@ -412,71 +415,125 @@ int gemm_tri(int tri, int m, int n, int k, double alpha, const double *A, long l
 }
 
 // Cholesky of one diagonal block (n <= 128, lower, in place) by one
-// workgroup of 1024 threads, then its inverse into D (ldd = 128).  Both
-// triangles live in LDS, packed (i(i+1)/2 + j, 2 x 66 KB), so the 128
-// dependent steps of each phase touch LDS only.  A non-positive pivot
-// records (global index + 1) in *info and continues with pivot 1.
-constexpr int DIAG_THREADS = 1024;
-constexpr int DIAG_PARTS = DIAG_THREADS / LB;     // partial sums per inverse entry
+// workgroup of 8 wavefronts, then its inverse into D (ldd = 128).  The block
+// is cut into 16 x 16 ones in LDS: a diagonal one is factored and inverted in
+// one wavefront's registers (row i in lane i, broadcasts by readlane, no
+// barrier), the panel below and the trailing update are MFMA products, and
+// in the inverse each wavefront takes a block column on its own.  It is a
+// serial chain of 128 square roots and divisions either way; one column at a
+// time over 1024 threads, five barriers a column, it took 354 us.
+// A non-positive pivot records (global index + 1) in *info and continues with
+// pivot 1.  Rows past n are the identity's.
+constexpr int DIAG_THREADS = 512;
+constexpr int DP = LB + 2;        // LDS row pitch of the block
 
-__device__ __forceinline__ int ptri(int i) { return i * (i + 1) / 2; }
+__device__ __forceinline__ double lane_value(double x, int lane) {
+    const long long b = __double_as_longlong(x);
+    return __longlong_as_double((long long)__builtin_amdgcn_readlane((int)(b >> 32), lane) << 32 |
+                                (unsigned)__builtin_amdgcn_readlane((int)b, lane));
+}
 
-__global__ __launch_bounds__(DIAG_THREADS) void potrf_diag_kernel(double *A, long lda, int n, int k0,
-                                                                  double *D, int *info) {
-    __shared__ double Lp[LB * (LB + 1) / 2];
-    __shared__ double Xp[LB * (LB + 1) / 2];
-    __shared__ double red[DIAG_PARTS][LB];
-    const int t = threadIdx.x;
-    for (int e = t; e < n * n; e += DIAG_THREADS) {
-        const int i = e / n, j = e % n;
-        if (j <= i) Lp[ptri(i) + j] = A[(long)i * lda + j];
+__global__ __launch_bounds__(DIAG_THREADS) void potrf_diag_kernel(double *A, long lda, int n, int k0, double *D,
+                                                                  int *info) {
+    __shared__ double Ls[LB * DP];           // L below the diagonal blocks, the inverse transposed above
+    __shared__ double Xd[LB / 16][16][17];   // inverses of the diagonal blocks
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, l15 = lane & 15, q4 = lane >> 4;
+    for (int e = t; e < LB * LB; e += DIAG_THREADS) {
+        const int i = e / LB, j = e % LB;
+        Ls[i * DP + j] = i < n ? (j <= i ? A[(long)i * lda + j] : 0.) : i == j ? 1. : 0.;
     }
-    // right-looking factorisation
-    for (int k = 0; k < n; k++) {
-        __syncthreads();
-        const double d = Lp[ptri(k) + k];
-        const bool bad = !(d > 0.);
-        const double piv = bad ? 1. : sqrt(d);
-        __syncthreads();
-        if (t == 0) {
-            Lp[ptri(k) + k] = piv;
-            if (bad && info) atomicCAS(info, 0, k0 + k + 1);
+    __syncthreads();
+    for (int kb = 0; kb < LB / 16; kb++) {
+        if (wave == 0) {
+            double *B = Ls + kb * 16 * DP + kb * 16;
+            double a[16], x[16];
+#pragma unroll
+            for (int c = 0; c < 16; c++) a[c] = B[l15 * DP + c];
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                const double d = lane_value(a[k], k);
+                const bool bad = !(d > 0.);
+                const double piv = bad ? 1. : sqrt(d);
+                if (bad && lane == 0 && info) atomicCAS(info, 0, k0 + kb * 16 + k + 1);
+                a[k] = l15 == k ? piv : a[k] / piv;
+#pragma unroll
+                for (int j = k + 1; j < 16; j++) a[j] -= a[k] * lane_value(a[k], j);
+            }
+            // column l15 of the inverse by forward substitution
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                double s = 0.;
+#pragma unroll
+                for (int k = 0; k < i; k++) s += lane_value(a[k], i) * x[k];
+                x[i] = ((i == l15 ? 1. : 0.) - s) / lane_value(a[i], i);
+            }
+            if (lane < 16) {
+#pragma unroll
+                for (int c = 0; c < 16; c++) {
+                    if (c <= l15) B[l15 * DP + c] = a[c];
+                    Xd[kb][c][l15] = x[c];
+                }
+            }
         }
-        for (int i = k + 1 + t; i < n; i += DIAG_THREADS) Lp[ptri(i) + k] /= piv;
         __syncthreads();
-        const int m = n - k - 1;
-        for (int e = t; e < m * m; e += DIAG_THREADS) {
-            const int i = k + 1 + e / m, j = k + 1 + e % m;
-            if (j <= i) Lp[ptri(i) + j] -= Lp[ptri(i) + k] * Lp[ptri(j) + k];
+        // panel: L_ik = A_ik inv(L_kk)^T
+        for (int bi = kb + 1 + wave; bi < LB / 16; bi += DIAG_THREADS / 64) {
+            double4_t acc = {0., 0., 0., 0.};
+#pragma unroll
+            for (int kq = 0; kq < 4; kq++)
+                acc = mfma16(Ls[(bi * 16 + l15) * DP + kb * 16 + 4 * kq + q4], Xd[kb][l15][4 * kq + q4], acc);
+#pragma unroll
+            for (int v = 0; v < 4; v++) Ls[(bi * 16 + q4 + 4 * v) * DP + kb * 16 + l15] = acc[v];
+        }
+        __syncthreads();
+        // trailing blocks: A_ij -= L_ik L_jk^T, i >= j > k
+        const int m = LB / 16 - 1 - kb;
+        for (int p = wave; p < m * (m + 1) / 2; p += DIAG_THREADS / 64) {
+            int ti, tj;
+            lower_tile(p, ti, tj);
+            const int bi = kb + 1 + ti, bj = kb + 1 + tj;
+            double *C = Ls + bi * 16 * DP + bj * 16 + l15;
+            double4_t acc;
+#pragma unroll
+            for (int v = 0; v < 4; v++) acc[v] = C[(q4 + 4 * v) * DP];
+#pragma unroll
+            for (int kq = 0; kq < 4; kq++)
+                acc = mfma16(-Ls[(bi * 16 + l15) * DP + kb * 16 + 4 * kq + q4],
+                             Ls[(bj * 16 + l15) * DP + kb * 16 + 4 * kq + q4], acc);
+#pragma unroll
+            for (int v = 0; v < 4; v++) C[(q4 + 4 * v) * DP] = acc[v];
+        }
+        __syncthreads();
+    }
+    // inverse, block column j = wave: X_ij = -inv(L_ii) sum_{j <= k < i} L_ik
+    // X_kj, stored transposed at block (j, i); a product's result lies in the
+    // lanes as the next one's B operand
+    {
+        const int j = wave;
+        double *Xt = Ls + (j * 16 + l15) * DP;      // row l15 of the transposed blocks: column l15 of X
+        for (int i = j + 1; i < LB / 16; i++) {
+            double4_t s = {0., 0., 0., 0.}, x = {0., 0., 0., 0.};
+            for (int k = j; k < i; k++)
+#pragma unroll
+                for (int kq = 0; kq < 4; kq++) {
+                    const int kk = 4 * kq + q4;
+                    s = mfma16(Ls[(i * 16 + l15) * DP + k * 16 + kk], k == j ? Xd[j][kk][l15] : Xt[k * 16 + kk], s);
+                }
+#pragma unroll
+            for (int v = 0; v < 4; v++) x = mfma16(-Xd[i][l15][4 * v + q4], s[v], x);
+#pragma unroll
+            for (int v = 0; v < 4; v++) Xt[i * 16 + q4 + 4 * v] = x[v];
         }
     }
     __syncthreads();
-    // inverse by forward substitution, one row per step:
-    // X[i][j] = (delta_ij - sum_{j<=k<i} L[i][k] X[k][j]) / L[i][i], the sum
-    // split over DIAG_PARTS threads per column and added in a fixed order
-    const int j = t % LB, part = t / LB;
-    for (int i = 0; i < n; i++) {
-        double s = 0.;
-        if (j < i)
-            for (int k = j + part; k < i; k += DIAG_PARTS) s += Lp[ptri(i) + k] * Xp[ptri(k) + j];
-        red[part][j] = s;
-        __syncthreads();
-        if (part == 0 && j <= i) {
-            double acc = 0.;
-#pragma unroll
-            for (int q = 0; q < DIAG_PARTS; q++) acc += red[q][j];
-            Xp[ptri(i) + j] = ((i == j ? 1. : 0.) - acc) / Lp[ptri(i) + i];
-        }
-        __syncthreads();
-    }
     // the factor back (strict upper triangle of the block zeroed) and D
     for (int e = t; e < n * n; e += DIAG_THREADS) {
         const int i = e / n, c = e % n;
-        A[(long)i * lda + c] = c <= i ? Lp[ptri(i) + c] : 0.;
+        A[(long)i * lda + c] = c <= i ? Ls[i * DP + c] : 0.;
     }
     for (int e = t; e < LB * LB; e += DIAG_THREADS) {
         const int i = e / LB, c = e % LB;
-        D[(long)i * LB + c] = (i < n && c <= i) ? Xp[ptri(i) + c] : 0.;
+        D[(long)i * LB + c] = i >= n || c > i ? 0. : i / 16 == c / 16 ? Xd[i / 16][i % 16][c % 16] : Ls[c * DP + i];
     }
 }
 
@@ -645,34 +702,59 @@ extern "C" int mdf_potrf(double *A, long n, long lda, int *info, void *work, siz
     return MDF_OK;
 }
 
-extern "C" size_t mdf_trtri_workspace(long n) { return (size_t)LB * n * sizeof(double) + 256; }
+// half of the widest level's blocks
+extern "C" size_t mdf_trtri_workspace(long n) {
+    size_t most = 0;
+    for (long s = LB; s < n; s *= 2) {
+        const size_t w = (size_t)((n + 2 * s - 1) / (2 * s)) * s * s;
+        most = w > most ? w : most;
+    }
+    return most * sizeof(double) + 256;
+}
+
+namespace {
+// X = the diagonal block inverses D, zero elsewhere (every entry written).
+__global__ __launch_bounds__(256) void trtri_diag_kernel(const double *__restrict__ D, long n, double *X, long ldx) {
+    const long j = (long)blockIdx.x * 256 + threadIdx.x;
+    if (j >= ldx) return;
+    for (long i = blockIdx.y; i < n; i += gridDim.y)
+        X[i * ldx + j] = j <= i && j / LB == i / LB ? D[(i / LB) * LB * LB + (i % LB) * LB + j % LB] : 0.;
+}
+}  // namespace
 
 // X = L^-1 for the lower factor L left by mdf_potrf; D holds its diagonal
-// block inverses (mdf_potrf's workspace).  X must not alias L.
+// block inverses (mdf_potrf's workspace).  X must not alias L.  By doubling:
+// with the s x s diagonal blocks inverted, each pair of them gives the next
+// size by X21 = -X22 (L21 X11), all pairs of a level in one batched product
+// each (n^3 / 3 products in 2 log2(n / 128) launches; a block row at a time
+// took 54 pairs of dependent launches of at most 55 workgroups at n = 6976,
+// 29.6 ms).
 extern "C" int mdf_trtri(const double *L, long n, long ldl, const double *D, double *X, long ldx, void *work,
                          size_t work_bytes, void *stream) {
     MDF_CHECK_ARG(L && D && X && n >= 0 && ldl >= n && ldx >= n, "mdf_trtri: bad arguments");
     MDF_CHECK_ARG(work && work_bytes >= mdf_trtri_workspace(n), "mdf_trtri: workspace too small");
+    if (n == 0) return MDF_OK;
     hipStream_t st = as_stream(stream);
-    double *T = (double *)work;      // LB x n
-    // zero X, then place the diagonal inverses
-    {
-        const long tot = n * ldx;
-        MDF_HIP(hipMemsetAsync(X, 0, tot * sizeof(double), st));
-    }
-    for (long b0 = 0; b0 < n; b0 += LB) {
-        const int kb = (int)(n - b0 < LB ? n - b0 : LB);
-        const double *Db = D + (b0 / LB) * LB * LB;
-        MDF_HIP(hipMemcpy2DAsync(X + b0 * ldx + b0, ldx * sizeof(double), Db, LB * sizeof(double),
-                                 kb * sizeof(double), kb, hipMemcpyDeviceToDevice, st));
-        if (b0 == 0) continue;
-        // T = L[b, 0:b0] X[0:b0, 0:b0];  X[b, 0:b0] = -D_b T
-        int rc = launch_gemm<128, false, 0, false>(kb, (int)b0, (int)b0, 1., L + b0 * ldl, ldl, 0, X, ldx, 0, 0.,
-                                                   T, b0, 0, 1, st);
-        if (rc) return rc;
-        rc = launch_gemm<128, false, 0, false>(kb, (int)b0, kb, -1., Db, LB, 0, T, b0, 0, 0., X + b0 * ldx, ldx, 0,
-                                               1, st);
-        if (rc) return rc;
+    double *T = (double *)work;
+    hipLaunchKernelGGL(trtri_diag_kernel, dim3((unsigned)cdiv(ldx, 256L), (unsigned)(n < 4096 ? n : 4096)), dim3(256), 0,
+                       st, D, n, X, ldx);
+    MDF_LAUNCHED("trtri_diag_kernel");
+    for (long s = LB; s < n; s *= 2) {
+        const long whole = n / (2 * s), rest = n - whole * 2 * s - s;     // rest > 0: a last, smaller second block
+        for (int part = 0; part < 2; part++) {
+            const long m = part ? rest : s, batch = part ? (rest > 0) : whole, at = part ? whole * 2 * s : 0;
+            if (batch == 0 || m <= 0) continue;
+            const double *L21 = L + (at + s) * ldl + at;
+            double *X11 = X + at * ldx + at, *X21 = X11 + s * ldx, *X22 = X21 + s;
+            double *Tp = T + (part ? whole * s * s : 0);
+            // T = L21 X11 with X11 lower triangular; X21 = -X22 T
+            int rc = launch_gemm<128, false, 3, false>((int)m, (int)s, (int)s, 1., L21, ldl, 2 * s * (ldl + 1), X11, ldx,
+                                                       2 * s * (ldx + 1), 0., Tp, s, s * s, batch, st);
+            if (rc) return rc;
+            rc = launch_gemm<128, false, 1, false>((int)m, (int)s, (int)m, -1., X22, ldx, 2 * s * (ldx + 1), Tp, s,
+                                                   s * s, 0., X21, ldx, 2 * s * (ldx + 1), batch, st);
+            if (rc) return rc;
+        }
     }
     return MDF_OK;
 }
