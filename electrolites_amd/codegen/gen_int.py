@@ -104,7 +104,7 @@ def gen_class(la, lb, lc, two_c):
     w('        const double ea = ao.exps[oa + ia], da = ao.coefs[oa + ia];')
     if two_c:
         w('        {')
-        w('        const double p = ea, fab = da;')
+        w('        const double p = ea, ip_ = 1.0 / p, fab = da;')
         w('        const double Px = Ax, Py = Ay, Pz = Az;')
     else:
         w('        for (int ib = 0; ib < npb; ib++) {')
@@ -119,20 +119,23 @@ def gen_class(la, lb, lc, two_c):
     w('            const double rpc2 = PCx * PCx + PCy * PCy + PCz * PCz;')
     w('            for (int ic = 0; ic < npc; ic++) {')
     w('                const double q = aux.exps[oc + ic];')
-    w('                const double pq = p + q, ipq = 1.0 / pq;')
-    w('                const double x = p * q * ipq * rpc2;')
-    w('                const double pref = TWO_PI_2P5 / (p * q * sqrt(pq)) * fab * aux.coefs[oc + ic];')
+    # a division costs about as much as a dozen of the products around it:
+    # one reciprocal each of p, q and p + q serves every use
+    w('                const double ipq = 1.0 / (p + q), iq = 1.0 / q;')
+    w('                const double qr = q * ipq, pr = p * ipq;')
+    w('                const double x = p * qr * rpc2;')
+    w('                const double pref = TWO_PI_2P5 * ip_ * iq * sqrt(ipq) * fab * aux.coefs[oc + ic];')
     w(f'                double ru[{nroots}], rw[{nroots}];')
     w(f'                rys_roots<{nroots}>(x, ru, rw);')
     w('#pragma unroll')
     w(f'                for (int r = 0; r < {nroots}; r++) {{')
     w('                    const double u = ru[r];')
     w('                    const double B00 = 0.5 * u * ipq;')
+    w('                    const double qf = qr * u, pf = pr * u;')
     if lab >= 2:
-        w('                    const double B10 = 0.5 / p - 0.5 * q * u * ipq / p;')
+        w('                    const double B10 = 0.5 * ip_ - 0.5 * ip_ * qf;')
     if lc >= 2:
-        w('                    const double B01 = 0.5 / q - 0.5 * p * u * ipq / q;')
-    w('                    const double qf = q * u * ipq, pf = p * u * ipq;')
+        w('                    const double B01 = 0.5 * iq - 0.5 * iq * pf;')
     for d in 'xyz':
         w(f'                    const double C00{d} = PA{d} - qf * PC{d}, C0p{d} = pf * PC{d};')
     # VRR

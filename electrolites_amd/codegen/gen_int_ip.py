@@ -90,6 +90,7 @@ def _deriv(d, a, b, k, wrt):
 
 
 KCH = 4       # default aux shells one thread of a three-centre kernel loops over
+IP_THREADS = 131072   # threads of a three-centre launch below which it takes fewer aux shells each
 QCH = 16      # aux shells one thread of a two-centre kernel loops over
 LDS_MAX_ATOMS = 1024
 #: a three-centre class whose Cartesian weight block times the aux components
@@ -212,9 +213,10 @@ def gen3(la, lb, lc, m_fixed=None):
     w('            const double rpc2 = PCx * PCx + PCy * PCy + PCz * PCz;')
     w('            for (int ic = 0; ic < npc; ic++) {')
     w('                const double q = aux.exps[oc + ic];')
-    w('                const double pq = p + q, ipq = 1.0 / pq;')
-    w('                const double x = p * q * ipq * rpc2;')
-    w('                const double pref = TWO_PI_2P5 / (p * q * sqrt(pq)) * fab * aux.coefs[oc + ic];')
+    w('                const double ipq = 1.0 / (p + q), iq = 1.0 / q;')
+    w('                const double qr = q * ipq, pr = p * ipq;')
+    w('                const double x = p * qr * rpc2;')
+    w('                const double pref = TWO_PI_2P5 * ip_ * iq * sqrt(ipq) * fab * aux.coefs[oc + ic];')
     w(f'                double ru[{nroots}], rw[{nroots}];')
     w(f'                rys_roots<{nroots}>(x, ru, rw);')
     # the roots one at a time in the classes whose terms keep every Rys factor
@@ -222,11 +224,10 @@ def gen3(la, lb, lc, m_fixed=None):
     w('#pragma unroll' if am else '#pragma unroll 1')
     w(f'                for (int r = 0; r < {nroots}; r++) {{')
     w('                    const double u = ru[r];')
-    w('                    const double B00 = 0.5 * u * ipq;')
-    w('                    const double B10 = 0.5 / p - 0.5 * q * u * ipq / p;')
+    w('                    const double B00 = 0.5 * u * ipq, qf = qr * u, pf = pr * u;')
+    w('                    const double B10 = 0.5 * ip_ - 0.5 * ip_ * qf;')
     if lc >= 2:
-        w('                    const double B01 = 0.5 / q - 0.5 * p * u * ipq / q;')
-    w('                    const double qf = q * u * ipq, pf = p * u * ipq;')
+        w('                    const double B01 = 0.5 * iq - 0.5 * iq * pf;')
     for d in 'xyz':
         w(f'                    const double C00{d} = PA{d} - qf * PC{d}, C0p{d} = pf * PC{d};')
     ind = '                    '
@@ -311,25 +312,25 @@ def gen2(la, lc):
     w('    const int npc = aux.nprim[ksh], oc = aux.poff[ksh];')
     w('    for (int ia = 0; ia < npa; ia++) {')
     w('        const double ea = aux.exps[oa + ia], fab = aux.coefs[oa + ia];')
-    w('        const double p = ea;')
+    w('        const double p = ea, ip_ = 1.0 / p;')
     w('        const double PAx = 0., PAy = 0., PAz = 0.;')
     w('        const double PCx = Ax - Cx, PCy = Ay - Cy, PCz = Az - Cz;')
     w('        const double rpc2 = PCx * PCx + PCy * PCy + PCz * PCz;')
     w('        for (int ic = 0; ic < npc; ic++) {')
     w('            const double q = aux.exps[oc + ic];')
-    w('            const double pq = p + q, ipq = 1.0 / pq;')
-    w('            const double x = p * q * ipq * rpc2;')
-    w('            const double pref = TWO_PI_2P5 / (p * q * sqrt(pq)) * fab * aux.coefs[oc + ic];')
+    w('            const double ipq = 1.0 / (p + q), iq = 1.0 / q;')
+    w('            const double qr = q * ipq, pr = p * ipq;')
+    w('            const double x = p * qr * rpc2;')
+    w('            const double pref = TWO_PI_2P5 * ip_ * iq * sqrt(ipq) * fab * aux.coefs[oc + ic];')
     w(f'            double ru[{nroots}], rw[{nroots}];')
     w(f'            rys_roots<{nroots}>(x, ru, rw);')
     w('#pragma unroll')
     w(f'            for (int r = 0; r < {nroots}; r++) {{')
     w('                const double u = ru[r];')
-    w('                const double B00 = 0.5 * u * ipq;')
-    w('                const double B10 = 0.5 / p - 0.5 * q * u * ipq / p;')
+    w('                const double B00 = 0.5 * u * ipq, qf = qr * u, pf = pr * u;')
+    w('                const double B10 = 0.5 * ip_ - 0.5 * ip_ * qf;')
     if lc >= 2:
-        w('                const double B01 = 0.5 / q - 0.5 * p * u * ipq / q;')
-    w('                const double qf = q * u * ipq, pf = p * u * ipq;')
+        w('                const double B01 = 0.5 * iq - 0.5 * iq * pf;')
     for d in 'xyz':
         w(f'                const double C00{d} = PA{d} - qf * PC{d}, C0p{d} = pf * PC{d};')
     ind = '                '
@@ -381,16 +382,21 @@ def main():
              '    atomicAdd(d + 1, y);',
              '    atomicAdd(d + 2, z);',
              '}', '',
-             '// aux shells one thread of a three-centre kernel loops over (MDF_IP_KCH, default '
-             f'{KCH})',
-             'static int ip_kch() {',
+             '// aux shells one thread of a three-centre kernel loops over: MDF_IP_KCH, or '
+             f'{KCH},',
+             '// fewer where the launch would leave wavefront slots empty (a d pair with an l = 4',
+             '// shell: 8 workgroups at 32 waters, 481 us; 4 us of it is launch)',
+             'static int ip_kch(long np, long nk) {',
              '    static int v = 0;',
              '    if (!v) {',
              '        const char *e = getenv("MDF_IP_KCH");',
-             f'        const int x = e ? atoi(e) : {KCH};',
-             f'        v = x >= 1 && x <= 4096 ? x : {KCH};',
+             '        const int x = e ? atoi(e) : 0;',
+             '        v = x >= 1 && x <= 4096 ? x : -1;',
              '    }',
-             '    return v;',
+             '    if (v > 0) return v;',
+             f'    int k = {KCH};',
+             f'    while (k > 1 && np * ((nk + k - 1) / k) < {IP_THREADS}) k /= 2;',
+             '    return k;',
              '}', '']
     n3, n2 = {}, {}
     for la in range(LMAX_AO + 1):
@@ -413,8 +419,8 @@ def main():
             parts += [src, '']
     parts.append('int launch_int3c_ip(int la, int lb, int lc, const BasisDev &ao, const BasisDev &aux, '
                  'const int *pairs, int np, const int *kl, int nk, const double *W, long ldw, const int *cmap, '
-                 'const int *ao_atom, const int *aux_atom, int natm, double *grad, double *grad_aux, hipStream_t st) {')
-    parts.append('    const int kch = ip_kch();')
+                 'const int *ao_atom, const int *aux_atom, int natm, double *grad, double *grad_aux, ForkJoin &fj) {')
+    parts.append('    const int kch = ip_kch(np, nk);')
     parts.append('    const long nkc = (nk + kch - 1) / kch;')
     parts.append(f'    const int use_lds = natm <= {LDS_MAX_ATOMS};')
     parts.append('    const size_t shm = use_lds ? 6 * (size_t)natm * sizeof(double) : 0;')
@@ -426,7 +432,7 @@ def main():
         key = (la * (LMAX_AO + 1) + lb) * (LMAX_AUX + 1) + lc
         parts.append(f'    case {key}:')
         for n in names:
-            parts.append(f'        hipLaunchKernelGGL({n}, g, b, shm, st, ao, aux, pairs, np, kl, nk, W, ldw, '
+            parts.append(f'        hipLaunchKernelGGL({n}, g, b, shm, fj.next(), ao, aux, pairs, np, kl, nk, W, ldw, '
                          'cmap, ao_atom, aux_atom, natm, use_lds, kch, grad, grad_aux);')
         parts.append('        break;')
     parts.append('    default: set_error("int3c2e_ip: class (%d %d|%d) not generated", la, lb, lc); return MDF_EINVAL;')

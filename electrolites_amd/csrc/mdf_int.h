@@ -19,6 +19,30 @@ struct BasisDev {
     const double *xyz, *exps, *coefs;
 };
 
+// Spreads the launches of one call, one small kernel per angular class and
+// component, over the caller's stream and three of the library's own
+// (per device, default priority), so one kernel's last workgroups run under
+// the next ones: the own streams start after the caller's work queued so far
+// and the caller's stream goes on after all of them (join, also in the
+// destructor).  A capturing caller's launches stay on its stream.
+class ForkJoin {
+public:
+    explicit ForkJoin(hipStream_t st);
+    ~ForkJoin() { (void)join(); }
+    ForkJoin(const ForkJoin &) = delete;
+    ForkJoin &operator=(const ForkJoin &) = delete;
+    int status() const { return rc_; }
+    hipStream_t next();
+    int join();
+
+private:
+    static constexpr int SIDE = 3;
+    hipStream_t st_, side_[SIDE];
+    hipEvent_t ev_ = nullptr;
+    int n_ = 0, rc_ = MDF_OK, at_ = 0;
+    bool used_[SIDE] = {};
+};
+
 int launch_int3c(int la, int lb, int lc, const BasisDev &ao, const BasisDev &aux, const int *pairs, int np,
                  const int *kl, int nk, double *out, long ldo, long p0, const int *cmap, hipStream_t st);
 int launch_int1e(int la, int lb, const BasisDev &ao, const int *pairs, int np, int natm, const double *charges,
@@ -27,7 +51,7 @@ int launch_int2c(int la, int lc, const BasisDev &aux, const int *pl, int np, con
                  double *out, long ldo, hipStream_t st);
 int launch_int3c_ip(int la, int lb, int lc, const BasisDev &ao, const BasisDev &aux, const int *pairs, int np,
                     const int *kl, int nk, const double *W, long ldw, const int *cmap, const int *ao_atom,
-                    const int *aux_atom, int natm, double *grad, double *grad_aux, hipStream_t st);
+                    const int *aux_atom, int natm, double *grad, double *grad_aux, ForkJoin &fj);
 int launch_int2c_ip(int la, int lc, const BasisDev &aux, const int *pl, int np, const int *ql, int nq,
                     const double *Z, long ldz, const int *aux_atom, int natm, double *grad, hipStream_t st);
 

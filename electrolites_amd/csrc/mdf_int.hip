@@ -11,7 +11,75 @@
 #include "mdf_int.h"
 #include "../../include/mi355df.h"
 
+#include <mutex>
+
 using namespace mdf;
+
+// ------------------------------------------------------------ side streams
+namespace {
+constexpr int MAX_DEVICES = 64;
+std::mutex g_side_mu;
+hipStream_t g_side[MAX_DEVICES][3];
+bool g_side_made[MAX_DEVICES];
+}  // namespace
+
+mdf::ForkJoin::ForkJoin(hipStream_t st) : st_(st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    int dev = 0;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+        hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) {
+        (void)hipGetLastError();
+        return;                                      // everything on the caller's stream
+    }
+    {
+        std::lock_guard<std::mutex> lk(g_side_mu);
+        if (!g_side_made[dev]) {
+            for (hipStream_t &s : g_side[dev])
+                if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
+                    (void)hipGetLastError();
+                    return;
+                }
+            g_side_made[dev] = true;
+        }
+        for (int i = 0; i < SIDE; i++) side_[i] = g_side[dev][i];
+    }
+    if (hipEventCreateWithFlags(&ev_, hipEventDisableTiming) != hipSuccess || hipEventRecord(ev_, st_) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    n_ = SIDE;
+}
+
+hipStream_t mdf::ForkJoin::next() {
+    const int i = at_++ % (n_ + 1);
+    if (i == 0) return st_;
+    if (!used_[i - 1]) {
+        if (hipStreamWaitEvent(side_[i - 1], ev_, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            return st_;                              // not ordered after the caller's work: not used
+        }
+        used_[i - 1] = true;
+    }
+    return side_[i - 1];
+}
+
+int mdf::ForkJoin::join() {
+    for (int i = 0; i < n_; i++) {
+        if (!used_[i]) continue;
+        used_[i] = false;
+        hipError_t e = hipEventRecord(ev_, side_[i]);
+        if (e == hipSuccess) e = hipStreamWaitEvent(st_, ev_, 0);
+        if (e != hipSuccess) e = hipStreamSynchronize(side_[i]);
+        if (e != hipSuccess) {
+            set_error("joining a side stream failed: %s", hipGetErrorString(e));
+            rc_ = MDF_EHIP;
+        }
+    }
+    n_ = 0;
+    if (ev_) (void)hipEventDestroy(ev_);
+    ev_ = nullptr;
+    return rc_;
+}
 
 static BasisDev to_dev(const mdf_basis *b) {
     BasisDev d;
@@ -33,21 +101,23 @@ extern "C" int mdf_int3c2e(const mdf_basis *ao, const mdf_basis *aux, const int 
                   ao->lmax, LMAX_AO, aux->lmax, LMAX_AUX);
     hipStream_t st = as_stream(stream);
     const BasisDev a = to_dev(ao), x = to_dev(aux);
-    for (int la = 0; la <= LMAX_AO; la++)
-        for (int lb = 0; lb <= LMAX_AO; lb++) {
+    // the classes of high angular momentum, few and long, first
+    ForkJoin fj(st);
+    for (int la = LMAX_AO; la >= 0; la--)
+        for (int lb = LMAX_AO; lb >= 0; lb--) {
             const int cls = la * (LMAX_AO + 1) + lb;
             const long q0 = pair_class_off[cls], q1 = pair_class_off[cls + 1];
             if (q1 <= q0) continue;
             MDF_CHECK_ARG(q1 - q0 < (1L << 31), "mdf_int3c2e: too many pairs in one class");
-            for (int lc = 0; lc <= LMAX_AUX; lc++) {
+            for (int lc = LMAX_AUX; lc >= 0; lc--) {
                 const long k0 = aux_l_off[lc], k1 = aux_l_off[lc + 1];
                 if (k1 <= k0) continue;
                 int rc = launch_int3c(la, lb, lc, a, x, pairs + 2 * q0, (int)(q1 - q0), aux_sorted + k0,
-                                      (int)(k1 - k0), out, ldo, p0, col_map, st);
+                                      (int)(k1 - k0), out, ldo, p0, col_map, fj.next());
                 if (rc) return rc;
             }
         }
-    return MDF_OK;
+    return fj.join();
 }
 
 extern "C" int mdf_int2c2e(const mdf_basis *aux, const int *aux_sorted, const long *aux_l_off, double *out,
@@ -89,21 +159,22 @@ extern "C" int mdf_int3c2e_ip(const mdf_basis *ao, const mdf_basis *aux, const i
     MDF_CHECK_ARG(ldw > 0, "mdf_int3c2e_ip: ldw must be positive");
     hipStream_t st = as_stream(stream);
     const BasisDev a = to_dev(ao), x = to_dev(aux);
-    for (int la = 0; la <= LMAX_AO; la++)
-        for (int lb = 0; lb <= LMAX_AO; lb++) {
+    ForkJoin fj(st);
+    for (int la = LMAX_AO; la >= 0; la--)
+        for (int lb = LMAX_AO; lb >= 0; lb--) {
             const int cls = la * (LMAX_AO + 1) + lb;
             const long q0 = pair_class_off[cls], q1 = pair_class_off[cls + 1];
             if (q1 <= q0) continue;
             MDF_CHECK_ARG(q1 - q0 < (1L << 31), "mdf_int3c2e_ip: too many pairs in one class");
-            for (int lc = 0; lc <= LMAX_AUX; lc++) {
+            for (int lc = LMAX_AUX; lc >= 0; lc--) {
                 const long k0 = aux_l_off[lc], k1 = aux_l_off[lc + 1];
                 if (k1 <= k0) continue;
                 int rc = launch_int3c_ip(la, lb, lc, a, x, pairs + 2 * q0, (int)(q1 - q0), aux_sorted + k0,
-                                         (int)(k1 - k0), W, ldw, col_map, ao_atom, aux_atom, natm, grad, grad_aux, st);
+                                         (int)(k1 - k0), W, ldw, col_map, ao_atom, aux_atom, natm, grad, grad_aux, fj);
                 if (rc) return rc;
             }
         }
-    return MDF_OK;
+    return fj.join();
 }
 
 // Nuclear derivative of the metric term: grad[3 * atom + x] +=
