@@ -48,6 +48,8 @@ _SIGS = {
     'mdf_int3c2e': (I, [P, P, P, P, P, P, L, P, P, L, P]),
     'mdf_int2c2e': (I, [P, P, P, P, L, P]),
     'mdf_k_step1': (I, [P, I, L, L, L, P, I, P, L, I, P, L, L, P]),
+    'mdf_k_step1_tiles_workspace': (SZ, [I, I]),
+    'mdf_k_step1_tiles': (I, [P, I, L, L, L, P, I, I, P, L, I, P, L, L, P, SZ, P]),
     'mdf_k_step1_lower': (I, [P, I, L, L, L, P, I, P, L, I, P, L, L, P]),
     'mdf_int3c2e_ip': (I, [P, P, P, P, P, P, P, L, P, P, P, I, P, P, P]),
     'mdf_int2c2e_ip': (I, [P, P, P, P, L, P, I, P, P]),

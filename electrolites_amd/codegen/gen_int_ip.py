@@ -91,7 +91,7 @@ def _deriv(d, a, b, k, wrt):
 
 KCH = 4       # default aux shells one thread of a three-centre kernel loops over
 IP_THREADS = 131072   # threads of a three-centre launch below which it takes fewer aux shells each
-QCH = 16      # aux shells one thread of a two-centre kernel loops over
+QCH = 4       # aux shells one thread of a two-centre kernel loops over
 LDS_MAX_ATOMS = 1024
 #: a three-centre class whose Cartesian weight block times the aux components
 #: holds at most this many values computes every aux component m in one
@@ -442,7 +442,7 @@ def main():
     parts.append('}')
     parts.append('')
     parts.append('int launch_int2c_ip(int la, int lc, const BasisDev &aux, const int *pl, int np, const int *ql, '
-                 'int nq, const double *Z, long ldz, const int *aux_atom, int natm, double *grad, hipStream_t st) {')
+                 'int nq, const double *Z, long ldz, const int *aux_atom, int natm, double *grad, ForkJoin &fj) {')
     parts.append(f'    const long n = (long)np * ((nq + {QCH - 1}) / {QCH}) * (2 * lc + 1);')
     parts.append(f'    const int use_lds = natm <= {LDS_MAX_ATOMS};')
     parts.append('    const size_t shm = use_lds ? 3 * (size_t)natm * sizeof(double) : 0;')
@@ -450,7 +450,7 @@ def main():
     parts.append(f'    const dim3 g((unsigned)((n + {THREADS - 1}) / {THREADS})), b({THREADS});')
     parts.append(f'    switch (la * {LMAX_AUX + 1} + lc) {{')
     for (la, lc), n in n2.items():
-        parts.append(f'    case {la * (LMAX_AUX + 1) + lc}: hipLaunchKernelGGL({n}, g, b, shm, st, aux, pl, np, ql, nq, '
+        parts.append(f'    case {la * (LMAX_AUX + 1) + lc}: hipLaunchKernelGGL({n}, g, b, shm, fj.next(), aux, pl, np, ql, nq, '
                      'Z, ldz, aux_atom, natm, use_lds, grad); break;')
     parts.append('    default: set_error("int2c2e_ip: class (%d|%d) not generated", la, lc); return MDF_EINVAL;')
     parts.append('    }')

@@ -53,6 +53,6 @@ int launch_int3c_ip(int la, int lb, int lc, const BasisDev &ao, const BasisDev &
                     const int *kl, int nk, const double *W, long ldw, const int *cmap, const int *ao_atom,
                     const int *aux_atom, int natm, double *grad, double *grad_aux, ForkJoin &fj);
 int launch_int2c_ip(int la, int lc, const BasisDev &aux, const int *pl, int np, const int *ql, int nq,
-                    const double *Z, long ldz, const int *aux_atom, int natm, double *grad, hipStream_t st);
+                    const double *Z, long ldz, const int *aux_atom, int natm, double *grad, ForkJoin &fj);
 
 }  // namespace mdf

@@ -126,18 +126,19 @@ extern "C" int mdf_int2c2e(const mdf_basis *aux, const int *aux_sorted, const lo
     MDF_CHECK_ARG(aux->lmax <= LMAX_AUX, "mdf_int2c2e: aux angular momentum %d > %d", aux->lmax, LMAX_AUX);
     hipStream_t st = as_stream(stream);
     const BasisDev x = to_dev(aux);
-    for (int la = 0; la <= LMAX_AUX; la++) {
+    ForkJoin fj(st);
+    for (int la = LMAX_AUX; la >= 0; la--) {
         const long p0 = aux_l_off[la], p1 = aux_l_off[la + 1];
         if (p1 <= p0) continue;
-        for (int lc = 0; lc <= LMAX_AUX; lc++) {
+        for (int lc = LMAX_AUX; lc >= 0; lc--) {
             const long k0 = aux_l_off[lc], k1 = aux_l_off[lc + 1];
             if (k1 <= k0) continue;
             int rc = launch_int2c(la, lc, x, aux_sorted + p0, (int)(p1 - p0), aux_sorted + k0, (int)(k1 - k0),
-                                  out, ldo, st);
+                                  out, ldo, fj.next());
             if (rc) return rc;
         }
     }
-    return MDF_OK;
+    return fj.join();
 }
 
 // Nuclear derivative of the three-centre term of the DF gradient:
@@ -188,18 +189,19 @@ extern "C" int mdf_int2c2e_ip(const mdf_basis *aux, const int *aux_sorted, const
     MDF_CHECK_ARG(aux->lmax <= LMAX_AUX, "mdf_int2c2e_ip: aux angular momentum %d > %d", aux->lmax, LMAX_AUX);
     hipStream_t st = as_stream(stream);
     const BasisDev x = to_dev(aux);
-    for (int la = 0; la <= LMAX_AUX; la++) {
+    ForkJoin fj(st);
+    for (int la = LMAX_AUX; la >= 0; la--) {
         const long p0 = aux_l_off[la], p1 = aux_l_off[la + 1];
         if (p1 <= p0) continue;
-        for (int lc = 0; lc <= LMAX_AUX; lc++) {
+        for (int lc = LMAX_AUX; lc >= 0; lc--) {
             const long k0 = aux_l_off[lc], k1 = aux_l_off[lc + 1];
             if (k1 <= k0) continue;
             int rc = launch_int2c_ip(la, lc, x, aux_sorted + p0, (int)(p1 - p0), aux_sorted + k0,
-                                     (int)(k1 - k0), Z, ldz, aux_atom, natm, grad, st);
+                                     (int)(k1 - k0), Z, ldz, aux_atom, natm, grad, fj);
             if (rc) return rc;
         }
     }
-    return MDF_OK;
+    return fj.join();
 }
 
 // Overlap, kinetic and nuclear-attraction matrices over the listed shell

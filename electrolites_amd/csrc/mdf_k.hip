@@ -516,3 +516,43 @@ extern "C" int mdf_k_step1(const void *cderi, int cderi_dtype, long nL, long npa
     return k_step1_entry<false>("mdf_k_step1", cderi, cderi_dtype, nL, npairs, ld, pair_map, nao, f, ldf, nocc, R,
                                 ldr, strideL, stream);
 }
+
+extern "C" size_t mdf_k_step1_tiles_workspace(int nao, int nocc) {
+    KPlan p{};
+    p.bn = pick_bn(nocc);
+    return pack_words(p, nao, nocc) * sizeof(double);
+}
+
+extern "C" int mdf_k_step1_tiles(const void *cderi, int cderi_dtype, long nL, long npairs, long ld,
+                                 const void *pair_tiles, int lower, int nao, const double *f, long ldf, int nocc,
+                                 double *R, long ldr, long strideL, void *work, size_t work_bytes, void *stream) {
+    MDF_CHECK_ARG(nL >= 0 && nao >= 0 && nocc >= 0 && nL < (1L << 31), "mdf_k_step1_tiles: bad sizes");
+    MDF_CHECK_ARG(cderi && pair_tiles && f && R, "mdf_k_step1_tiles: null pointer");
+    MDF_CHECK_ARG(ld >= npairs && ldf >= nocc && ldr >= nocc && strideL >= (long)nao * ldr,
+                  "mdf_k_step1_tiles: leading dimension too small");
+    MDF_CHECK_ARG(cderi_dtype == MDF_DTYPE_F64 || cderi_dtype == MDF_DTYPE_F32, "mdf_k_step1_tiles: cderi dtype %d",
+                  cderi_dtype);
+    MDF_CHECK_ARG(nao <= tiles::MAX_NAO && npairs < (1L << 29),
+                  "mdf_k_step1_tiles: pair tiles hold up to %d functions and 2^29 pairs", tiles::MAX_NAO);
+    if (nL == 0 || nao == 0 || nocc == 0) return MDF_OK;
+    const size_t need = mdf_k_step1_tiles_workspace(nao, nocc);
+    if (!work || work_bytes < need) {
+        set_error("mdf_k_step1_tiles: workspace %zu bytes < %zu required", work ? work_bytes : (size_t)0, need);
+        return MDF_EWORKSPACE;
+    }
+    KPlan p{};
+    p.bn = pick_bn(nocc);
+    hipStream_t st = as_stream(stream);
+    double *fp = (double *)work;
+    if (int rc = pack_factor<double>(p, st, f, ldf, nao, nocc, fp)) return rc;
+    const tiles::View tv = tiles::view(pair_tiles, nao);
+    const long sB = RL * strideL;
+    if (cderi_dtype == MDF_DTYPE_F32) {
+        const float *c = (const float *)cderi;
+        return lower ? step1_pairs<double, float, true>(p, (int)nL, st, c, ld, tv, fp, nocc, R, ldr, strideL, sB)
+                     : step1_pairs<double, float, false>(p, (int)nL, st, c, ld, tv, fp, nocc, R, ldr, strideL, sB);
+    }
+    const double *c = (const double *)cderi;
+    return lower ? step1_pairs<double, double, true>(p, (int)nL, st, c, ld, tv, fp, nocc, R, ldr, strideL, sB)
+                 : step1_pairs<double, double, false>(p, (int)nL, st, c, ld, tv, fp, nocc, R, ldr, strideL, sB);
+}

@@ -553,6 +553,11 @@ extern "C" int mdf_gemm_batched(int transb, int tri_a, int lower_c, long M, long
     const int m = (int)M, n = (int)N, k = (int)K;
     if (!transb && tri_a == 0 && !lower_c && N > 256 && N <= 320)
         return launch_wide(m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch, st);
+    // N in (128, 160]: one 160-wide column tile instead of two of 128 (the
+    // gradient's F_r^T R_L at nocc 160: 2.4 -> 1.6 ms)
+    if (!transb && tri_a == 0 && !lower_c && N > 128 && N <= 160)
+        return launch_gemm<160, false, 0, false>(m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc,
+                                                 strideC, batch, st);
     if (lower_c)
         return transb ? gemm_tri<true, true>(tri_a, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc,
                                              strideC, batch, st)

@@ -137,8 +137,8 @@ __global__ __launch_bounds__(256) void tiles_groups_kernel(const int *__restrict
     if (n < nrows && rows[n] >= 0) grp[rows[n]] = n / RB;
 }
 
-// One workgroup per group: its columns (of groups up to its own with LOWER),
-// their count in steps and the map.
+// One workgroup per group: its columns (of its own and later groups with
+// LOWER), their count in steps and the map.
 template <bool LOWER>
 __global__ __launch_bounds__(256) void tiles_map_kernel(const int *__restrict__ pmap, int nao,
                                                         const int *__restrict__ grp, const int *__restrict__ rows,
@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void tiles_map_kernel(const int *__restrict__ 
     for (int j0 = 0; j0 < nao; j0 += 256) {
         const int j = j0 + t;
         bool in = false;
-        if (j < nao && (!LOWER || grp[j] <= g))
+        if (j < nao && (!LOWER || grp[j] >= g))
             for (int r = 0; r < RB; r++) in = in || (row[r] >= 0 && pmap[(long)row[r] * nao + j] >= 0);
         const u64 b = __ballot(in);
         if (lane == 0) wsum[wave] = __popcll(b);

@@ -223,7 +223,7 @@ class _PairLayout:
             if got is None:
                 got = self._tiles[lower] = PairTiles(
                     self.map, self.nao, self.npairs, lower,
-                    self._tiles[False].buf if lower and False in self._tiles else None)
+                    self._tiles[False].on_stream() if lower and False in self._tiles else None)
         return got.on_stream()
 
 

@@ -264,9 +264,9 @@ def _diag_positions(n):
 def _rhok(dfobj, fl, fr, nao, nrow):
     """``rhok[L] = F_r^T A_L F_l`` for every cderi row L, and whether it is
     packed.  With one factor (F_l = F_r = F) the form is symmetric: A_L =
-    T_L + T_L^T with T_L its lower triangle, diagonal halved, so rhok[L] =
-    G + G^T with G = F^T T_L F, and T_L F costs about half of A_L F
-    (``mdf_k_step1_lower``); rhok then comes back as ``(nrow, nocc (nocc +
+    T_L + T_L^T with T_L its lower triangle, diagonal halved, or another
+    such half, so rhok[L] = G + G^T with G = F^T T_L F, and T_L F costs about
+    half of A_L F (``mdf_k_step1_lower``, ``mdf_k_step1_tiles``); rhok then comes back as ``(nrow, nocc (nocc +
     1) / 2)`` packed upper triangles, off-diagonal entries times sqrt 2."""
     t = _dev.torch()
     nocc = fl.shape[1]
@@ -281,15 +281,25 @@ def _rhok(dfobj, fl, fr, nao, nrow):
         if cderi.shape[0] != nrow:
             raise ValueError(f'jk_energy_per_atom: the cderi has {cderi.shape[0]} rows, the metric factor {nrow}')
         lay = fastdf._layout(dfobj, cderi, nao)
+        # on the pair tiles T_L is any half of A_L, 22 % of nao^2 at 64 waters
+        # (its lower triangle by 128-row tiles 54 %)
+        tiles = lay.tiles(lower=sym)
+        work = None if tiles is None else \
+            t.empty(_lib.query('mdf_k_step1_tiles_workspace', nao, nocc), dtype=t.uint8, device=_dev.device())
         nb = max(1, min(nrow, RBLOCK_BYTES // max(8 * nao * nocc, 1)))
         R = t.empty((nb, nao, nocc), dtype=t.float64, device=_dev.device())
         G = t.empty((nb, nocc, nocc), dtype=t.float64, device=_dev.device()) if sym else None
         code = fastdf._dtype_code(cderi)
         for L0 in range(0, nrow, nb):
             nL = min(nb, nrow - L0)
-            _lib.call('mdf_k_step1_lower' if sym else 'mdf_k_step1', _dev.ptr(cderi[L0]), code, nL,
-                      cderi.shape[1], cderi.stride(0), _dev.ptr(lay.map), nao, _dev.ptr(fl), fl.stride(0), nocc,
-                      _dev.ptr(R), nocc, nao * nocc, _dev.stream_ptr())
+            if tiles is not None:
+                _lib.call('mdf_k_step1_tiles', _dev.ptr(cderi[L0]), code, nL, cderi.shape[1], cderi.stride(0),
+                          _dev.ptr(tiles), int(sym), nao, _dev.ptr(fl), fl.stride(0), nocc, _dev.ptr(R), nocc,
+                          nao * nocc, _dev.ptr(work), work.numel(), _dev.stream_ptr())
+            else:
+                _lib.call('mdf_k_step1_lower' if sym else 'mdf_k_step1', _dev.ptr(cderi[L0]), code, nL,
+                          cderi.shape[1], cderi.stride(0), _dev.ptr(lay.map), nao, _dev.ptr(fl), fl.stride(0), nocc,
+                          _dev.ptr(R), nocc, nao * nocc, _dev.stream_ptr())
             # F_r^T R_L, one batched product over the block's rows
             out = G if sym else rhok[L0]
             _gemm_batched(nocc, nocc, nao, frT.data_ptr(), nao, 0, R.data_ptr(), nocc, nao * nocc,

@@ -120,9 +120,9 @@ int mdf_get_k(const void *cderi, int cderi_dtype, long naux, long npairs, long l
  * a pair map into groups of 16 AO rows with compacted column lists (one device
  * buffer of mdf_pair_tiles_bytes(nao) bytes, 0 when nao is out of range; built
  * on the stream, nothing returns to the host).  It depends on the pair map
- * only and serves every later call over the same cderi.  lower != 0: the
- * triangular half T with A = T + T^T (columns of a row's own and earlier
- * groups, own-group pairs halved), for mdf_k_step1_tiles; order_of, another
+ * only and serves every later call over the same cderi.  lower != 0: a half
+ * T with A = T + T^T (columns of a row's own and later groups, own-group
+ * pairs halved: 22 % of nao^2 at 64 waters), for mdf_k_step1_tiles; order_of, another
  * buffer of the same map or NULL, gives the row order.
  * mdf_get_k_tiles is mdf_get_k with step 1 on the tiles (pair_tiles NULL:
  * mdf_get_k itself); npairs < 2^29.  Its workspace also holds the packed
@@ -136,6 +136,14 @@ int mdf_get_k_tiles(const void *cderi, int cderi_dtype, long naux, long npairs, 
                     const void *pair_tiles, int nao, const double *fl, const double *fr, int nocc, long ldf,
                     int prec, double *vk, long ldvk, int accumulate, void *work, size_t work_bytes,
                     void *stream);
+
+/* mdf_k_step1 on pair tiles: R[L] = A_L F, or T_L F with the lower tiles (R +
+ * its transpose then gives the symmetric form); the layout of mdf_k_step1.
+ * work: the packed factor, mdf_k_step1_tiles_workspace(nao, nocc) bytes. */
+size_t mdf_k_step1_tiles_workspace(int nao, int nocc);
+int mdf_k_step1_tiles(const void *cderi, int cderi_dtype, long nL, long npairs, long ld, const void *pair_tiles,
+                      int lower, int nao, const double *f, long ldf, int nocc, double *R, long ldr, long strideL,
+                      void *work, size_t work_bytes, void *stream);
 
 /* ---- grouped J/K over many (molecule, density) items -------------------
  * No counterpart in the reference (each get_jk call there contracts one

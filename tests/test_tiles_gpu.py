@@ -168,3 +168,31 @@ def test_tiles_hold_every_pair_once(nao):
         if which == 'lower':
             got = got + got.T
         assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize('storage', ['float64', 'float32'])
+@pytest.mark.parametrize('lower', [0, 1])
+@pytest.mark.parametrize('nao,nL,nocc', [(17, 9, 5), (47, 8, 33), (130, 11, 97), (150, 3, 321)])
+def test_step1_tiles(storage, lower, nao, nL, nocc):
+    """R = A F, and R = T F with T + T^T = A: F^T T F + its transpose."""
+    import torch
+    from electrolites_amd import _dev, _lib, fastdf
+    print(f'step1 tiles {storage} lower {lower} nao {nao} nL {nL} nocc {nocc}', flush=True)
+    cderi, rows, cols, addr, f, _ = inputs(nao, nL, nocc, False, storage, empty=(1,))
+    _, buf = make_tiles(addr, nao, lower)
+    nb = _lib.query('mdf_k_step1_tiles_workspace', nao, nocc)
+    work = torch.full((nb // 8,), float('nan'), dtype=torch.float64, device='cuda')
+    ldr = nocc + 3
+    R = torch.full((nL, nao, ldr), float('nan'), dtype=torch.float64, device='cuda')
+    _lib.call('mdf_k_step1_tiles', _dev.ptr(cderi), fastdf._dtype_code(cderi), nL, len(addr), cderi.stride(0),
+              _dev.ptr(buf), lower, nao, _dev.ptr(f), nocc, nocc, _dev.ptr(R), ldr, nao * ldr, _dev.ptr(work), nb,
+              _dev.stream_ptr())
+    a = torch.zeros((nL, nao, nao), dtype=torch.float64, device='cuda')
+    a[:, rows, cols] = cderi.double()
+    a[:, cols, rows] = cderi.double()
+    got, want = R[:, :, :nocc], a @ f
+    assert bool(R[:, :, nocc:].isnan().all())
+    if lower:
+        got = f.T @ got
+        got, want = got + got.transpose(1, 2), f.T @ want
+    assert rel(got, want) < 2.3e-16 * 4 * nao
