@@ -63,7 +63,7 @@ __global__ __launch_bounds__(G_THREADS, 2) void gemm_f64_kernel(
     Acc<S::MI, S::NI> acc;
     acc.zero();
     const int nk = (kmax - k0 + G_BK - 1) / G_BK;
-    if (BT) {
+    if constexpr (BT) {
         RowsLoader<BN> lb{B, ldb, n0, N, k0, kmax};
         gemm_mainloop<128, BN>(la, lb, nk, lds, acc);
     } else {
