@@ -385,7 +385,7 @@ def main():
              '// aux shells one thread of a three-centre kernel loops over: MDF_IP_KCH, or '
              f'{KCH},',
              '// fewer where the launch would leave wavefront slots empty (a d pair with an l = 4',
-             '// shell: 8 workgroups at 32 waters, 481 us; 4 us of it is launch)',
+             '// shell: 8 workgroups at 32 waters, 481 us)',
              'static int ip_kch(long np, long nk) {',
              '    static int v = 0;',
              '    if (!v) {',

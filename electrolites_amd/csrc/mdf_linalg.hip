@@ -17,6 +17,7 @@
 
 #include "mdf_common.h"
 #include "mdf_gemm.h"
+#include "mdf_tiles.h"
 #include "../../include/mi355df.h"
 
 using namespace mdf;
@@ -180,6 +181,112 @@ __global__ __launch_bounds__(G_THREADS, 2) void gemm_pairs_kernel(int n, int K, 
             for (int v = 0; v < 4; v++)
                 if (off[ni][v] != NONE) *(double *)(wb + off[ni][v]) = acc.v[mi][ni][v];
     }
+}
+
+// Rows of a matrix given by their addresses (RowsLoader's layout).
+template <int R>
+struct GatheredRows : RowsLoader<R> {
+    template <class F>
+    __device__ __forceinline__ GatheredRows(const double *base, int kmax, F &&row) : RowsLoader<R>(base, 0, 0, 1, 0, kmax) {
+#pragma unroll
+        for (int q = 0; q < RowsLoader<R>::Q; q++) this->p[q] = row((int)(threadIdx.x >> 3) + q * RowsLoader<R>::RPP);
+    }
+};
+
+// gemm_pairs_kernel<true> for symmetric P_z on lower pair tiles: a workgroup
+// takes the 16 rows of group g for 8 of the batch (128 tile rows) and the
+// group's compacted columns in tiles of 128, the last of 64 if that holds it.
+// At 32 waters the lower tiles hold 30 % of n^2 (the lower 128-tiles 58 %); the
+// columns of W are one table per 16 x 16 block, read once for the 8 batch
+// entries, where the other kernel looks each one up.  At 32 waters (nocc 160)
+// a term's four launches 10.1 -> 5.8 ms; the MFMAs take 59 % of that, 10
+// K-steps being few beside the 8-byte stores.
+template <int BN>
+__device__ __forceinline__ void pairs_tile(int nz, int K, double alpha, const double *__restrict__ A, long lda,
+                                           const double *__restrict__ B, long ldb, long sB, const tiles::View &tv, int g,
+                                           int c0, double *W, long ldw, const double *__restrict__ iscale,
+                                           const double *__restrict__ ivals, double *lds) {
+    using S = TileShape<128, BN>;
+    const int *rows = tv.rows + g * tiles::RB, *cols = tv.cols + (long)g * tv.ccap;
+    const int nstep = tv.nstep[g], ncol = nstep * 16;
+    GatheredRows<128> la(B, K, [&](int r) {
+        return B + (long)max(rows[r % tiles::RB], 0) * ldb + min(r / tiles::RB, nz - 1) * sB;
+    });
+    GatheredRows<BN> lb(A, K, [&](int r) {
+        return A + (long)min(cols[min(c0 + r, ncol - 1)], tv.nao - 1) * lda;
+    });
+    Acc<S::MI, S::NI> acc;
+    acc.zero();
+    gemm_mainloop<128, BN>(la, lb, (K + G_BK - 1) / G_BK, lds, acc);
+    constexpr unsigned NONE = ~0u;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = wave % 2, wn = wave / 2;
+    unsigned off[S::NI][4];
+    double base[S::NI][4];
+    int ri[4];
+#pragma unroll
+    for (int v = 0; v < 4; v++) ri[v] = rows[Mfma<double>::row(lane, v)];
+#pragma unroll
+    for (int ni = 0; ni < S::NI; ni++) {
+        const int s = (c0 + wn * S::WN) / 16 + ni;
+        if (s < nstep) {
+            const int *m = tv.map + ((long)g * tv.ccap + s * 16) * tiles::RB + (lane & 15);
+            const int j = cols[s * 16 + (lane & 15)];
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int p = m[16 * Mfma<double>::row(lane, v)];
+                // a pair of one group stands twice: its entry with i >= j
+                const bool put = p >= 0 && (!(p & tiles::HALF) || ri[v] >= j);
+                off[ni][v] = put ? (unsigned)(p & tiles::INDEX) * 8u : NONE;
+            }
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; v++) off[ni][v] = NONE;
+        }
+    }
+    if (iscale) {
+#pragma unroll
+        for (int ni = 0; ni < S::NI; ni++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                base[ni][v] = off[ni][v] != NONE ? *(const double *)((const char *)ivals + off[ni][v]) : 0.;
+    }
+#pragma unroll
+    for (int mi = 0; mi < S::MI; mi++) {
+        const int z = wm * S::MI + mi;            // 16 tile rows: one of the batch
+        if (z >= nz) continue;
+        char *wb = (char *)(W + z * ldw);
+        const double s = iscale ? iscale[z] : 1.;
+        if (!iscale) {
+#pragma unroll
+            for (int ni = 0; ni < S::NI; ni++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) base[ni][v] = off[ni][v] != NONE ? *(const double *)(wb + off[ni][v]) : 0.;
+        }
+#pragma unroll
+        for (int ni = 0; ni < S::NI; ni++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                if (off[ni][v] != NONE) *(double *)(wb + off[ni][v]) = s * base[ni][v] + alpha * acc.v[mi][ni][v];
+    }
+}
+
+__global__ __launch_bounds__(G_THREADS, 2) void gemm_pairs_tiles_kernel(
+    int nz, int K, double alpha, const double *__restrict__ A, long lda, const double *__restrict__ B, long ldb, long sB,
+    tiles::View tv, double *W, long ldw, const double *__restrict__ iscale, const double *__restrict__ ivals, long n) {
+    __shared__ double lds[TileShape<128, 128>::LDS_DOUBLES];
+    const long x = xcd_tile(blockIdx.x, gridDim.x);
+    if (x >= n) return;
+    const int g = (int)(x % tv.ngroup), z0 = (int)(x / tv.ngroup) * tiles::NL;
+    const int ncol = tv.nstep[g] * 16;
+    B += z0 * sB;
+    W += z0 * ldw;
+    if (iscale) iscale += z0;
+    const int m = min(tiles::NL, nz - z0);
+    int c0 = 0;
+    for (; ncol - c0 > 64; c0 += 128)
+        pairs_tile<128>(m, K, alpha, A, lda, B, ldb, sB, tv, g, c0, W, ldw, iscale, ivals, lds);
+    if (c0 < ncol) pairs_tile<64>(m, K, alpha, A, lda, B, ldb, sB, tv, g, c0, W, ldw, iscale, ivals, lds);
 }
 
 // Packed upper triangles (row-major over a <= b: the offset of (a, b) is
@@ -554,7 +661,8 @@ extern "C" int mdf_gemm_batched(int transb, int tri_a, int lower_c, long M, long
     if (!transb && tri_a == 0 && !lower_c && N > 256 && N <= 320)
         return launch_wide(m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch, st);
     // N in (128, 160]: one 160-wide column tile instead of two of 128 (the
-    // gradient's F_r^T R_L at nocc 160: 2.4 -> 1.6 ms)
+    // gradient's F_r^T R_L at nocc 160, 32 waters: the whole term 56.5 -> 54.3
+    // ms)
     if (!transb && tri_a == 0 && !lower_c && N > 128 && N <= 160)
         return launch_gemm<160, false, 0, false>(m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc,
                                                  strideC, batch, st);
@@ -596,6 +704,25 @@ extern "C" int mdf_gemm_pairs_batched(int transb, long n, long K, double alpha, 
                                ldw, isc, init_vals);
         MDF_LAUNCHED("gemm_pairs_kernel");
     }
+    return MDF_OK;
+}
+
+extern "C" int mdf_gemm_pairs_tiles(long n, long K, double alpha, const double *A, long lda, const double *B, long ldb,
+                                    long strideB, const void *pair_tiles, long npairs, double *W, long ldw,
+                                    const double *init_scale, const double *init_vals, long batch, void *stream) {
+    MDF_CHECK_ARG(n >= 0 && n <= tiles::MAX_NAO && K > 0 && K < (1L << 31) && npairs >= 0 && npairs < (1L << 29) &&
+                  batch >= 0 && batch < (1L << 31), "mdf_gemm_pairs_tiles: bad sizes");
+    if (n == 0 || batch == 0) return MDF_OK;
+    MDF_CHECK_ARG(A && B && pair_tiles && W, "mdf_gemm_pairs_tiles: null pointer");
+    MDF_CHECK_ARG(!init_scale == !init_vals, "mdf_gemm_pairs_tiles: init_scale and init_vals go together");
+    MDF_CHECK_ARG(lda >= K && ldb >= K && strideB >= 0 && (batch == 1 || ldw >= npairs),
+                  "mdf_gemm_pairs_tiles: leading dimension or stride");
+    const tiles::View tv = tiles::view(pair_tiles, (int)n);
+    const long nt = (batch + tiles::NL - 1) / tiles::NL * tv.ngroup;
+    MDF_CHECK_ARG(round_xcd(nt) < (1L << 31), "mdf_gemm_pairs_tiles: batch of %ld too large", batch);
+    hipLaunchKernelGGL(gemm_pairs_tiles_kernel, dim3((unsigned)round_xcd(nt)), dim3(G_THREADS), 0, as_stream(stream),
+                       (int)batch, (int)K, alpha, A, lda, B, ldb, strideB, tv, W, ldw, init_scale, init_vals, nt);
+    MDF_LAUNCHED("gemm_pairs_tiles_kernel");
     return MDF_OK;
 }
 

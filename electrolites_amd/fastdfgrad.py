@@ -36,7 +36,7 @@ packed rows read through the pair map) for a device-resident cderi, and from
 the unpacked blocks of :meth:`DF.loop` otherwise; the remaining contractions
 (F_r^T R_L, the triangular products, W's blocks and Z) run on the package's
 FP64 matrix-core GEMM (``mdf_gemm``, ``mdf_gemm_batched``,
-``mdf_gemm_pairs_batched``).  With one factor (F_l = F_r) every rhok_L and
+``mdf_gemm_pairs_batched``, ``mdf_gemm_pairs_tiles``).  With one factor (F_l = F_r) every rhok_L and
 dmoo_P is symmetric and is kept as its packed upper triangle
 (``mdf_sym_pack`` / ``mdf_sym_unpack``) with the off-diagonal entries times
 sqrt 2, so that the dot product of two packed rows is the full trace
@@ -416,6 +416,9 @@ def jk_energy_per_atom(dfobj, dm, j_factor=1., k_factor=1., hermi=1, auxbasis_re
     ncol = tabs['ncol']
     W = t.empty((naux, ncol), dtype=t.float64, device=_dev.device())
     Dflat = D.reshape(-1)[tabs['addr']].contiguous()
+    tiles = None
+    if _on_device(cderi) and k_factor != 0 and any(sym for _, sym in rhoks):
+        tiles = fastdf._layout(dfobj, cderi, nao).tiles(lower=True)
     jc = (j_factor * c).contiguous()
     if k_factor == 0:
         jb = max(1, min(naux, WBLOCK_BYTES // max(8 * ncol, 1)))
@@ -439,7 +442,8 @@ def jk_energy_per_atom(dfobj, dm, j_factor=1., k_factor=1., hermi=1, auxbasis_re
             # as H_P = F_r dmoo_P^T for a block of P (one product), then
             # the lower 128-tiles of F_l H_P^T per P put straight into the
             # cderi's compact columns (one batched product; no G_P is
-            # written), over the Coulomb part on the first factor set
+            # written), over the Coulomb part on the first factor set; a
+            # symmetric G_P on the pair tiles where there are any
             blk = max(1, min(naux, WBLOCK_BYTES // max(8 * nao * nocc, 1)))
             H = t.empty((nao, blk * nocc), dtype=t.float64, device=_dev.device())
             full = t.empty((blk, nocc * nocc), dtype=t.float64, device=_dev.device()) if sym else None
@@ -454,6 +458,11 @@ def jk_energy_per_atom(dfobj, dm, j_factor=1., k_factor=1., hermi=1, auxbasis_re
                     dm_blk = dmoo[P0:P1]
                 _gemm(fr, dm_blk.reshape(nP * nocc, nocc), Hb, transb=True)
                 init = (_dev.ptr(jc[P0:P1]), _dev.ptr(Dflat)) if si == 0 else (None, None)
+                if sym and tiles is not None and nocc > 0:
+                    _lib.call('mdf_gemm_pairs_tiles', nao, nocc, float(-2 * wk * k_factor), _dev.ptr(fl), nocc,
+                              _dev.ptr(Hb), Hb.stride(0), nocc, _dev.ptr(tiles), ncol, _dev.ptr(W[P0]), W.stride(0),
+                              init[0], init[1], nP, _dev.stream_ptr())
+                    continue
                 _lib.call('mdf_gemm_pairs_batched', 1, nao, nocc, float(-2 * wk * k_factor), ctypes.c_void_p(fl.data_ptr()),
                           nocc, 0, ctypes.c_void_p(Hb.data_ptr()), Hb.stride(0), nocc, _dev.ptr(tabs['cmap']),
                           _dev.ptr(W[P0]), W.stride(0), init[0], init[1], nP, _dev.stream_ptr())

@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define MDF_ABI_VERSION 13
+#define MDF_ABI_VERSION 14
 
 /* arithmetic precision of a contraction */
 #define MDF_PREC_FP64 0
@@ -365,6 +365,12 @@ int mdf_gemm_pairs_batched(int transb, long n, long K, double alpha, const doubl
                            long strideA, const double *B, long ldb, long strideB, const int *pair_col,
                            double *W, long ldw, const double *init_scale, const double *init_vals,
                            long batch, void *stream);
+/* mdf_gemm_pairs_tiles: mdf_gemm_pairs_batched with transb, one A for the
+ *   batch and symmetric P_z, on the lower pair tiles of the pair map
+ *   (mdf_build_pair_tiles): W's columns are the map's, npairs of them. */
+int mdf_gemm_pairs_tiles(long n, long K, double alpha, const double *A, long lda, const double *B, long ldb,
+                         long strideB, const void *pair_tiles, long npairs, double *W, long ldw,
+                         const double *init_scale, const double *init_vals, long batch, void *stream);
 /* mdf_sym_pack: for each z < batch, the packed upper triangle (row-major
  *   over a <= b; (a, b) at a n - a (a - 1) / 2 + b - a) of G_z + G_z^T,
  *   scaled by diag_scale on the diagonal and off_scale off it:

@@ -196,3 +196,49 @@ def test_step1_tiles(storage, lower, nao, nL, nocc):
         got = f.T @ got
         got, want = got + got.transpose(1, 2), f.T @ want
     assert rel(got, want) < 2.3e-16 * 4 * nao
+
+
+@pytest.mark.parametrize('nao,nocc,batch', [(16, 1, 1), (33, 5, 8), (120, 16, 9), (203, 17, 3), (300, 50, 17)])
+@pytest.mark.parametrize('init', [False, True])
+def test_gemm_pairs_tiles(nao, nocc, batch, init):
+    """A symmetric product's values at the stored pairs, from the lower tiles
+    and from the general entry (which reads its own lower triangle), against
+    a plain sum; every other entry of W keeps its value.  Two AOs have no
+    pair; the rows of W and of the factors are padded."""
+    import ctypes
+    import torch
+    from electrolites_amd import _dev, _lib
+    rng = np.random.default_rng(nao + nocc + batch)
+    rows, cols = pair_list(rng, nao, .4, (0, nao - 1))
+    npairs = len(rows)
+    addr = torch.from_numpy((rows * nao + cols).astype(np.int32)).cuda()
+    _, tiles = make_tiles(addr, nao, 1)
+    f = torch.zeros((nao, nocc + 3), dtype=torch.float64, device='cuda')
+    f[:, :nocc] = torch.from_numpy(rng.standard_normal((nao, nocc))).cuda()
+    m = torch.from_numpy(rng.standard_normal((batch, nocc, nocc))).cuda()
+    m = m + m.transpose(1, 2)
+    h = torch.zeros((nao, batch * nocc + 1), dtype=torch.float64, device='cuda')
+    h[:, :batch * nocc] = torch.matmul(f[:, :nocc], m).transpose(0, 1).reshape(nao, -1)
+    w = torch.from_numpy(rng.standard_normal((batch, npairs + 5))).cuda()
+    sc, vals = (torch.from_numpy(rng.standard_normal(n)).cuda() for n in (batch, npairs))
+    p = torch.matmul(torch.matmul(f[:, :nocc], m), f[:, :nocc].T)
+    r, c = torch.from_numpy(rows).cuda(), torch.from_numpy(cols).cuda()
+    base = sc[:, None] * vals if init else w[:, :npairs]
+    base = base.clone()
+    ref = torch.cat([base - .6 * p[:, r, c], w[:, npairs:]], dim=1)
+    if init:
+        w[:, :npairs] = float('nan')
+    g = w.clone()
+    isc = (_dev.ptr(sc), _dev.ptr(vals)) if init else (None, None)
+    _lib.call('mdf_gemm_pairs_tiles', nao, nocc, ctypes.c_double(-.6), _dev.ptr(f), nocc + 3, _dev.ptr(h),
+              h.shape[1], nocc, _dev.ptr(tiles), npairs, _dev.ptr(w), npairs + 5, *isc, batch, _dev.stream_ptr())
+    cmap = torch.full((nao * (nao + 1) // 2,), -1, dtype=torch.int32, device='cuda')
+    cmap[r * (r + 1) // 2 + c] = torch.arange(npairs, dtype=torch.int32, device='cuda')
+    _lib.call('mdf_gemm_pairs_batched', 1, nao, nocc, ctypes.c_double(-.6), _dev.ptr(f), nocc + 3, 0, _dev.ptr(h),
+              h.shape[1], nocc, _dev.ptr(cmap), _dev.ptr(g), npairs + 5, *isc, batch, _dev.stream_ptr())
+    # two products of nocc terms each, both sides rounding every one:
+    # 4 nocc eps sum |f| |m| |f|, and the sum with the base
+    bound = 4 * 2.3e-16 * (nocc * float(f.abs().max()) ** 2 * float(m.abs().sum(dim=(1, 2)).max()) +
+                           float(base.abs().max()))
+    assert float((w - ref).abs().max()) < bound
+    assert float((w - g).abs().max()) < bound
