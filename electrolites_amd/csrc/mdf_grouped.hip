@@ -368,6 +368,23 @@ __global__ __launch_bounds__(256) void gk_finalize(const GKItem *items, const Ti
     }
 }
 
+// Reorders a step-1 table from s on so that each XCD's contiguous run holds an
+// eighth of every item, in the items' order: a run of whole items gave one XCD
+// the long tiles of the large items and another the short ones (12 molecules of
+// 3 to 32 waters, FP64: 36.6 -> 31.9 ms a run; 15 of 3 to 27, split BF16: 19.9 ->
+// 13.8).
+void spread_xcd(std::vector<Tile> &tab, size_t s) {
+    std::vector<Tile> run[N_XCD];
+    for (size_t a = s, b; a < tab.size(); a = b) {
+        for (b = a + 1; b < tab.size() && tab[b].item == tab[a].item;) b++;
+        for (size_t t = a; t < b; t++) run[(t - a) * N_XCD / (b - a)].push_back(tab[t]);
+    }
+    for (const auto &r : run) {
+        std::copy(r.begin(), r.end(), tab.begin() + s);
+        s += r.size();
+    }
+}
+
 int persistent_grid(long ntiles, int per_cu) {
     int dev = 0, cu = 256;
     if (hipGetDevice(&dev) == hipSuccess) hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev);
@@ -588,6 +605,7 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
             std::stable_sort(k1.begin() + s1, k1.end(), [&](const Tile &x, const Tile &y) {
                 return p->hk[x.item].nao > p->hk[y.item].nao;
             });
+            spread_xcd(k1, s1);
             p->kphases.push_back({1, s1, (long)k1.size() - s1, cbn, mp});
           }
             // one step-2 launch per output tile width

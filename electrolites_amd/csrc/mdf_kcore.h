@@ -421,13 +421,14 @@ inline int cu_count() {
 // Of the splits of at least 8 K-steps, the one of least estimated time: the
 // rounds of resident workgroups (slots per XCD) each over its K-steps and
 // about 6 more to start and end, plus the partials written and read again
-// (nao^2 words each, 1.5e-6 K-steps a word).
-inline int pick_ksplit(int ntiles_grid, long nsteps, int nao, int slots) {
+// (nao^2 words each, 1.5e-6 K-steps a word; 3e-6 of split BF16's, which take
+// half the time).
+inline int pick_ksplit(int ntiles_grid, long nsteps, int nao, int slots, double word) {
     int best = N_XCD;
     double best_t = 1e300;
     for (int ks = N_XCD; ks <= 256 && (ks == N_XCD || nsteps >= 8L * ks); ks += N_XCD) {
         const long rounds = ((long)ntiles_grid * ks / N_XCD + slots - 1) / slots;
-        const double t = rounds * ((double)nsteps / ks + 6.) + 1.5e-6 * ks * nao * nao;
+        const double t = rounds * ((double)nsteps / ks + 6.) + word * ks * nao * nao;
         if (t < best_t) { best_t = t; best = ks; }
     }
     return best;
@@ -489,7 +490,8 @@ inline KPlan plan_k(long naux, int nao, int nocc, bool two, long max_rows, bool 
     p.ntile = (nao + p.s2 - 1) / p.s2;
     p.ntiles_grid = tiles(p.s2);
     const long nsteps = b3 ? p.nL * ((nocc + 31) / 32) : RShape(p.nL, nocc).steps();
-    p.ksplit = pick_ksplit(p.ntiles_grid, nsteps, nao, (p.s2 == 64 ? 4 : 2) * cu_count() / N_XCD);
+    p.ksplit = pick_ksplit(p.ntiles_grid, nsteps, nao, (p.s2 == 64 ? 4 : 2) * cu_count() / N_XCD,
+                           b3 ? 3e-6 : 1.5e-6);
     p.bn = pick_bn(nocc);
     p.r_words = r_words(p.nL, nao, nocc);
     p.part_words = (size_t)p.ksplit * nao * nao;
