@@ -59,8 +59,9 @@ class Entry:
         self.vk = t.empty((n_dm, nao, nao), dtype=t.float64, device=dev)
 
     def tiles(self):
-        """The pair map's tiles, given or made here: the same ones a single
-        call's layout makes, so an item's K is the same alone."""
+        """The pair map's tiles, given or made here (complete on return, so a
+        plan may run on any stream): the same ones a single call's layout
+        makes, so an item's K is the same alone."""
         if self.pair_tiles is None and self.pair_map is not None:
             self.pair_tiles = fastdf.PairTiles(self.pair_map, self.nao, self.npairs).buf
         return self.pair_tiles
@@ -105,6 +106,7 @@ class GroupedJK:
         self.work = None if work_pool is not None else \
             _dev.torch().empty(max(self.work_bytes, 256), dtype=_dev.torch().uint8, device=_dev.device())
         self.graph = None
+        self._streams = set()           # that the entries' tiles are kept for
 
     def _create(self, bn):
         plan = P()
@@ -147,6 +149,12 @@ class GroupedJK:
 
     def run(self):
         """Launch the batch on the current stream (or replay its graph)."""
+        cur = _dev.torch().cuda.current_stream()
+        if cur.cuda_stream not in self._streams:
+            self._streams.add(cur.cuda_stream)
+            for e in self.entries:
+                if e.pair_tiles is not None:
+                    e.pair_tiles.record_stream(cur)
         if self.graph is not None:
             self.graph.replay()
             return

@@ -214,8 +214,7 @@ class _PairLayout:
     def tiles(self, lower=False):
         """The pair tiles of this layout's map (K's step 1 skips the pairs
         not stored), built at the first exchange; None for a full triangle
-        or sizes they do not hold.  ``lower``: the triangular half's.  Another
-        stream than the building one waits for it."""
+        or sizes they do not hold.  ``lower``: the triangular half's."""
         if self.map is None:
             return None
         with self._tiles_lock:
@@ -234,8 +233,10 @@ TILES_MIN_NAO = 112
 
 
 class PairTiles:
-    """``mdf_build_pair_tiles`` of a pair map, with the stream it was built
-    on (``buf`` None: sizes the tiles do not hold or do not help)."""
+    """``mdf_build_pair_tiles`` of a pair map (``buf`` None: sizes the tiles do
+    not hold or do not help).  The host waits for the build, once per map: a
+    kernel takes offsets and row numbers from the tiles as they are, so no
+    stream, plan or graph may meet them half built."""
 
     def __init__(self, pair_map, nao, npairs, lower=False, order_of=None):
         t = _dev.torch()
@@ -247,18 +248,14 @@ class PairTiles:
         _lib.call('mdf_build_pair_tiles', _dev.ptr(pair_map), nao, int(lower), _dev.ptr(order_of),
                   _dev.ptr(self.buf), nbytes, _dev.stream_ptr())
         self.stream = t.cuda.current_stream()
-        self.done = t.cuda.Event()
-        self.done.record(self.stream)
+        self.stream.synchronize()
 
     def on_stream(self):
-        """The buffer, ordered before the current stream's next work and kept
-        for it."""
+        """The buffer, kept for the current stream's next work."""
         if self.buf is None:
             return None
         cur = _dev.torch().cuda.current_stream()
         if cur != self.stream:
-            if not self.done.query():
-                cur.wait_event(self.done)
             self.buf.record_stream(cur)
         return self.buf
 

@@ -165,3 +165,44 @@ def test_grouped_fp32_storage(precision):
         rj, rk = fastdf.get_jk(df, dm, hermi=1)
         assert np.array_equal(vj.cpu().numpy(), rj)
         assert np.array_equal(vk.cpu().numpy(), rk)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('precision', ['fp64', 'bf16x3'])
+def test_plan_runs_on_another_stream(precision):
+    """A plan whose entries' pair tiles are built on one stream, behind work
+    already queued there, and which then runs on another (two plans sharing
+    the entry), gives the single call's K."""
+    import torch
+    from electrolites_amd import batch, fastdf
+    nao, naux, nocc = 150, 61, 20
+    rng = np.random.default_rng(9)
+    pa, _ = O.pair_addresses(nao)
+    rows, cols = np.divmod(pa, nao)
+    pa = pa[(rng.random(len(pa)) > .5) | (rows == cols)]
+    df = FakeDF(rng.standard_normal((naux, len(pa))), pa, nao)
+    c = np.linalg.qr(rng.standard_normal((nao, nocc)))[0]
+    dm = fastdf.tag_array(2 * c @ c.T, mo_coeff=c, mo_occ=np.full(nocc, 2.))
+    df.k_precision = precision
+    ref = torch.from_numpy(fastdf.get_jk(df, dm, hermi=1)[1]).cuda()
+    entry, = _entries([df], [dm])
+    big = torch.randn(4096, 4096, device='cuda', dtype=torch.float64)
+    torch.cuda.synchronize()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(a):
+        for _ in range(4):
+            big @ big
+        g = batch.GroupedJK([entry], precision=precision, tune=False)
+    assert entry.tiles() is not None
+    with torch.cuda.stream(b):
+        g.run()
+        got = entry.vk[0].clone()
+        g2 = batch.GroupedJK([entry], precision=precision, tune=False)
+    with torch.cuda.stream(a):
+        a.wait_stream(b)
+        entry.vk.zero_()
+        g2.run()
+    torch.cuda.synchronize()
+    assert torch.equal(got, ref) and torch.equal(entry.vk[0], ref)
+    g.close()
+    g2.close()

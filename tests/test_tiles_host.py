@@ -1,0 +1,68 @@
+"""Host side of the pair tiles on the CPU, with the library and the streams
+replaced: when tiles are built, when they may be used, what is kept."""
+import types
+
+import pytest
+
+
+class FakeStream:
+    cuda_stream = 7
+
+    def __init__(self, log):
+        self.log = log
+
+    def synchronize(self):
+        self.log.append('sync')
+
+
+class FakeEvent:
+    def __init__(self, *a, **k):
+        pass
+
+    def record(self, *a):
+        pass
+
+    def query(self):
+        return False
+
+
+@pytest.fixture
+def fake(monkeypatch):
+    """The library's calls and the stream's waits, in order; ``capturing``
+    says whether the current stream is being captured."""
+    import torch
+    from electrolites_amd import _dev, _lib
+    f = types.SimpleNamespace(log=[], capturing=False)
+    stream = FakeStream(f.log)
+    monkeypatch.setattr(_lib, 'query', lambda name, *a: f.log.append(name) or 4096)
+    monkeypatch.setattr(_lib, 'call', lambda name, *a: f.log.append(name))
+    monkeypatch.setattr(_dev, 'stream_ptr', lambda: None)
+    monkeypatch.setattr(_dev, 'device', lambda: torch.device('cpu'))
+    monkeypatch.setattr(torch.cuda, 'current_stream', lambda *a: stream)
+    monkeypatch.setattr(torch.cuda, 'is_current_stream_capturing', lambda: f.capturing)
+    monkeypatch.setattr(torch.cuda, 'Event', FakeEvent)
+    return f
+
+
+def layout(nao=120):
+    """A screened layout: the last pair of the triangle is not stored."""
+    import numpy as np
+    from electrolites_amd import fastdf
+    rows, cols = np.tril_indices(nao)
+    addr = (rows * nao + cols).astype(np.int32)[:-1]
+    return fastdf._PairLayout(addr, nao, len(addr))
+
+
+@pytest.mark.parametrize('via', ['entry', 'layout', 'lower'])
+def test_tiles_are_complete_when_handed_out(fake, via):
+    """Whoever gets the tiles may run on any stream: the host has waited for
+    the build by then."""
+    import torch
+    from electrolites_amd import batch
+    lay = layout()
+    if via == 'entry':
+        buf = batch.Entry(torch.zeros(3, lay.npairs, dtype=torch.float64), 120, 1, 2, pair_map=lay.map).tiles()
+    else:
+        buf = lay.tiles(lower=via == 'lower')
+    assert buf is not None
+    assert 'sync' in fake.log[fake.log.index('mdf_build_pair_tiles'):]
