@@ -214,12 +214,17 @@ class _PairLayout:
     def tiles(self, lower=False):
         """The pair tiles of this layout's map (K's step 1 skips the pairs
         not stored), built at the first exchange; None for a full triangle
-        or sizes they do not hold.  ``lower``: the triangular half's."""
+        or sizes they do not hold.  ``lower``: the triangular half's.  None too
+        where they would have to be built on a stream that is being captured:
+        the caller's graph goes through the pair map, and the tiles wait for a
+        call whose launches run."""
         if self.map is None:
             return None
         with self._tiles_lock:
             got = self._tiles.get(lower)
             if got is None:
+                if _dev.torch().cuda.is_current_stream_capturing():
+                    return None
                 got = self._tiles[lower] = PairTiles(
                     self.map, self.nao, self.npairs, lower,
                     self._tiles[False].on_stream() if lower and False in self._tiles else None)

@@ -242,3 +242,39 @@ def test_gemm_pairs_tiles(nao, nocc, batch, init):
                            float(base.abs().max()))
     assert float((w - ref).abs().max()) < bound
     assert float((w - g).abs().max()) < bound
+
+
+@pytest.mark.parametrize('built', [False, True])
+def test_captured_call(built):
+    """get_jk of response densities (no value goes to the host) captured with
+    the tiles not built yet, or built: each replay, with eager calls between,
+    gives the eager result, and the eager calls stay right afterwards."""
+    import torch
+    from electrolites_amd import fastdf
+    nao, naux, nocc = 150, 40, 20
+    cderi, rows, cols, addr, fl, fr = inputs(nao, naux, nocc, True)
+    print(f'captured get_jk, tiles built {built}', flush=True)
+
+    class DF:
+        def __init__(self):
+            self._cderi, self._cderi_idx = {0: cderi}, (addr, None)
+    x = fl @ (2. * fr).T
+    dm = fastdf.tag_array(x + x.T, mo1=fl, occ_coeff=fr, symmetrize=1)
+    refs = [t.clone() for t in fastdf.get_jk(DF(), dm, hermi=1)]     # sizes the shared workspace
+    df = DF()
+    fastdf.get_jk(df, dm, hermi=1, with_k=built)
+    assert bool(df._mdf_layout[2]._tiles) == built
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        vj, vk = fastdf.get_jk(df, dm, hermi=1)
+    for rep in range(3):
+        vj.zero_()
+        vk.zero_()
+        eager = fastdf.get_jk(df, dm, hermi=1)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        for got in ((vj, vk), eager):
+            assert torch.equal(got[0], refs[0])
+            assert rel(got[1], refs[1]) < 2.3e-16 * 2 * (nao + naux * nocc)

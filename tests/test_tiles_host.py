@@ -66,3 +66,19 @@ def test_tiles_are_complete_when_handed_out(fake, via):
         buf = lay.tiles(lower=via == 'lower')
     assert buf is not None
     assert 'sync' in fake.log[fake.log.index('mdf_build_pair_tiles'):]
+
+
+def test_a_captured_call_builds_no_tiles(fake):
+    """Tiles built inside a capture would hold nothing until the graph runs,
+    and lie in its memory: the captured call goes without, and a later call
+    builds them; once built, a captured call takes them."""
+    lay = layout()
+    fake.capturing = True
+    n = len(fake.log)
+    assert lay.tiles() is None and lay.tiles(lower=True) is None
+    assert fake.log[n:] == []
+    fake.capturing = False
+    buf = lay.tiles()
+    assert buf is not None
+    fake.capturing = True
+    assert lay.tiles() is buf and lay.tiles(lower=True) is None
