@@ -209,7 +209,11 @@ class _PairLayout:
             _lib.call('mdf_build_pair_map', _dev.ptr(addr), npairs, nao,
                       _dev.ptr(self.map), _dev.stream_ptr())
         self._tiles = {}
-        self._tiles_lock = threading.Lock()
+
+    def __getstate__(self):
+        """A copy builds tiles of its own: those kept here belong to this
+        layout's map and stream."""
+        return dict(self.__dict__, _tiles={})
 
     def tiles(self, lower=False):
         """The pair tiles of this layout's map (K's step 1 skips the pairs
@@ -220,17 +224,22 @@ class _PairLayout:
         call whose launches run."""
         if self.map is None:
             return None
-        with self._tiles_lock:
-            got = self._tiles.get(lower)
-            if got is None:
-                if _dev.torch().cuda.is_current_stream_capturing():
-                    return None
-                got = self._tiles[lower] = PairTiles(
-                    self.map, self.nao, self.npairs, lower,
-                    self._tiles[False].on_stream() if lower and False in self._tiles else None)
+        got = self._tiles.get(lower)
+        if got is None:
+            if _dev.torch().cuda.is_current_stream_capturing():
+                return None
+            with _TILES_LOCK:
+                got = self._tiles.get(lower)
+                if got is None:
+                    got = self._tiles[lower] = PairTiles(
+                        self.map, self.nao, self.npairs, lower,
+                        self._tiles[False].on_stream() if lower and False in self._tiles else None)
         return got.on_stream()
 
 
+#: held while a layout's tiles are built (not a member of the layout, which
+#: is copied with the DF object that keeps it)
+_TILES_LOCK = threading.Lock()
 #: K's step 1 runs on pair tiles from this many functions: below it they
 #: gain nothing (a whole get_jk at nao 72: 257 us with them, 253 without; at
 #: 120: 342 and 352; at 192: 534 and 607) and the first call pays for them

@@ -82,3 +82,20 @@ def test_a_captured_call_builds_no_tiles(fake):
     assert buf is not None
     fake.capturing = True
     assert lay.tiles() is buf and lay.tiles(lower=True) is None
+
+
+@pytest.mark.parametrize('built', [False, True])
+@pytest.mark.parametrize('how', ['deepcopy', 'pickle'])
+def test_a_layout_can_be_copied(fake, how, built):
+    """As a DF object that keeps one is: the copy has the pair tables and no
+    tiles, and the original keeps its own."""
+    import copy
+    import pickle
+    from electrolites_amd import fastdf
+    for lay in (layout(), fastdf._PairLayout(None, 4, 10)):
+        tiles = lay.tiles() if built else None
+        got = copy.deepcopy(lay) if how == 'deepcopy' else pickle.loads(pickle.dumps(lay))
+        assert (got.nao, got.npairs, got.full) == (lay.nao, lay.npairs, lay.full)
+        assert (got.map is None) == (lay.map is None) and got._tiles == {}
+        if tiles is not None:
+            assert lay.tiles() is tiles and got.tiles() is not tiles
