@@ -72,6 +72,7 @@ class _State:
             self.tasks.append(tk)
         widest = max([tk.c1 - tk.c0 for tk in self.tasks] + [1])
         self.buf = t.empty(self.naux * widest, dtype=t.float64, device=_dev.device())
+        self.held = None          # what the buffer holds: see _sweep
 
 
 def _state(dfobj, chunk_bytes=None):
@@ -87,20 +88,24 @@ def _state(dfobj, chunk_bytes=None):
 
 def _sweep(st, fn, held=None):
     """Evaluate each chunk of (P|ij) over its kept pairs into the buffer
-    (every column written) and hand it to fn, the ``held`` one, whose
-    integrals the buffer has already, first and as it is; returns the chunk
-    the buffer then holds.  A molecule of one chunk (up to ``CHUNK_BYTES`` of
-    integrals, about 30 waters) so evaluates its integrals once per call
-    instead of once per sweep: 12.4 -> 7.0 ms at 24 waters."""
-    for tk in ([held] if held is not None else []) + [tk for tk in st.tasks if tk is not held]:
+    (every column written) and hand it to fn, first and as it is the chunk of
+    ``held``, a call's mark of what it left in the buffer; returns the mark of
+    the last one (another call on the same molecule that comes between two
+    sweeps replaces it, and the chunk is evaluated again).  A molecule of one
+    chunk (up to ``CHUNK_BYTES`` of integrals, about 30 waters) so evaluates
+    its integrals once per call instead of once per sweep: 12.4 -> 7.0 ms at
+    24 waters."""
+    first = None if held is None else held[0]
+    for tk in ([first] if first is not None else []) + [tk for tk in st.tasks if tk is not first]:
         width = tk.c1 - tk.c0
         blk = st.buf[:st.naux * width]
-        if tk is not held:
+        mark = held
+        if tk is not first or st.held is not held:
+            st.held = mark = (tk,)
             ints.int3c2e_chunk(st.ao, st.aux, tk, blk, width, col_map=tk.cmap)
         fn(tk, blk, width)
         STATS['chunks'] += 1
-        last = tk
-    return last
+    return mark
 
 
 def get_j(dfobj, dm, hermi=1):
