@@ -457,8 +457,8 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
             p->hj.push_back(g);
         }
         if (with_k && x.nocc > 0 && x.naux > 0) {
-            if (!x.fl || !x.vk) {
-                set_error("mdf_grouped_plan_create: item %d lacks K buffers", m);
+            if (!x.fl || !x.vk || x.nocc > kcore::max_cols(x.nao)) {
+                set_error("mdf_grouped_plan_create: item %d lacks K buffers, or nocc %d is too large", m, x.nocc);
                 delete p;
                 return MDF_EINVAL;
             }

@@ -433,6 +433,16 @@ extern "C" int mdf_get_k_tiles(const void *cderi, int cderi_dtype, long naux, lo
             for (int i = 0; i < nao; i++) MDF_HIP(hipMemsetAsync(vk + (long)i * ldvk, 0, nao * sizeof(double), st));
         return MDF_OK;
     }
+    const long most = max_cols(nao);
+    if (nocc > most) {
+        // the sum over the columns in parts
+        for (long k0 = 0; k0 < nocc; k0 += most)
+            if (int rc = mdf_get_k_tiles(cderi, cderi_dtype, naux, npairs, ld, pair_map, pair_tiles, nao, fl + k0,
+                                         two ? fr + k0 : nullptr, (int)(nocc - k0 < most ? nocc - k0 : most), ldf, prec,
+                                         vk, ldvk, accumulate || k0 > 0, work, work_bytes, stream))
+                return rc;
+        return MDF_OK;
+    }
     MDF_CHECK_ARG(work != nullptr, "mdf_get_k: workspace is null");
     size_t need1 = k_bytes(naux, nao, nocc, two, prec, 1, pairs);
     if (work_bytes < need1) {
@@ -534,6 +544,7 @@ extern "C" int mdf_k_step1_tiles(const void *cderi, int cderi_dtype, long nL, lo
                   cderi_dtype);
     MDF_CHECK_ARG(nao <= tiles::MAX_NAO && npairs < (1L << 29),
                   "mdf_k_step1_tiles: pair tiles hold up to %d functions and 2^29 pairs", tiles::MAX_NAO);
+    MDF_CHECK_ARG(nocc <= max_cols(nao), "mdf_k_step1_tiles: nocc %d > %ld", nocc, max_cols(nao));
     if (nL == 0 || nao == 0 || nocc == 0) return MDF_OK;
     const size_t need = mdf_k_step1_tiles_workspace(nao, nocc);
     if (!work || work_bytes < need) {

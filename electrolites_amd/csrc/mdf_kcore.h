@@ -213,6 +213,14 @@ __device__ __forceinline__ void step1_pairs_tile(const Src *__restrict__ c, long
 // it computed nocc rounded up to 16: 96 columns for 81, 64 for 50).
 constexpr int RL = tiles::NL;
 
+// Columns a factor may have in one contraction: TransformedLoader's and the
+// packed factor's 32-bit offsets reach that far (at least 92,000 columns
+// at the functions that int32 pair addresses hold).
+inline long max_cols(int nao) {
+    const long packed = (1L << 32) / (nao + 1L) - 320;
+    return packed < 1L << 22 ? packed : 1L << 22;
+}
+
 // Columns of a block's row that hold values: fewer in a pass's last block.
 struct RShape {
     int nocc, ldr, kchunks, nfull, lastcols;
@@ -235,21 +243,24 @@ struct TransformedLoader {
     static constexpr int Q = N / EPV, LPR = G_BK / EPV, RPP = G_THREADS / LPR;
     static constexpr int SWZ = sizeof(T) == 8 ? 2 : 3;
     static_assert(Q >= 1 && Q * RPP == ROWS, "TransformedLoader shape");
-    const T *R;
+    const T *R;          // row r0 of block 0
     long strideB;
     RShape y;
-    unsigned off[Q];     // this thread's rows
+    // this thread's rows, from row r0: 32 bits hold the 127 rows of a tile up
+    // to max_cols columns, where a row's place in the whole block outgrows
+    // them from nao nocc = 2^29
+    unsigned off[Q];
     int last;            // its column in a row's last, ragged chunk
     long b;              // block and
     int kc;              // chunk of the next load()
     int left;            // columns in range of the loaded chunk
     __device__ __forceinline__ TransformedLoader(const T *R_, long strideB_, const RShape &y_, int r0, int nao, long b_,
                                                  int kc_)
-        : R(R_), strideB(strideB_), y(y_), b(b_), kc(kc_) {
+        : R(R_ + (long)r0 * y_.ldr), strideB(strideB_), y(y_), b(b_), kc(kc_) {
         const int c = (int)(threadIdx.x % LPR) * EPV;
 #pragma unroll
         for (int q = 0; q < Q; q++)
-            off[q] = (unsigned)min(r0 + (int)(threadIdx.x / LPR) + q * RPP, nao - 1) * (unsigned)y.ldr + c;
+            off[q] = (unsigned)min((int)(threadIdx.x / LPR) + q * RPP, nao - 1 - r0) * (unsigned)y.ldr + c;
         last = min((y.kchunks - 1) * G_BK + c, y.ldr - EPV) - c;
     }
     __device__ __forceinline__ void load(int, T (&r)[N]) {

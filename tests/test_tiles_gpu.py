@@ -278,3 +278,30 @@ def test_captured_call(built):
         for got in ((vj, vk), eager):
             assert torch.equal(got[0], refs[0])
             assert rel(got[1], refs[1]) < 2.3e-16 * 2 * (nao + naux * nocc)
+
+
+@pytest.mark.parametrize('tiled', [False, True])
+@pytest.mark.parametrize('two', [False, True])
+@pytest.mark.parametrize('nocc', [(1 << 22) - 3, (1 << 22) + 5])
+def test_k_rows_beyond_32_bits(monkeypatch, tiled, two, nocc):
+    """The transformed blocks of 130 functions and 2^22 columns span more
+    than 2^32 values (step 2's row offsets); a factor of more columns than
+    one contraction takes is summed in parts."""
+    import torch
+    monkeypatch.setenv('MDF_K_BLOCK_BYTES', str(80 << 30))
+    nao, naux = 130, 8
+    print(f'k rows nao {nao} nocc {nocc} tiled {tiled} two {two}', flush=True)
+    cderi, rows, cols, addr, _, _ = inputs(nao, naux, 1, False)
+    pmap, buf = make_tiles(addr, nao)
+    g = torch.Generator(device='cuda').manual_seed(nocc)
+    fl = torch.randn((nao, nocc), generator=g, dtype=torch.float64, device='cuda')
+    fr = torch.randn((nao, nocc), generator=g, dtype=torch.float64, device='cuda') if two else None
+    vk = get_k(cderi, pmap, buf if tiled else None, nao, fl, fr, 0)
+    a = torch.zeros((naux, nao, nao), dtype=torch.float64, device='cuda')
+    a[:, rows, cols] = cderi
+    a[:, cols, rows] = cderi
+    m = fl @ (fl if fr is None else fr).T
+    ref = sum(x @ m @ x for x in a)
+    # naux nocc products a sum in any order; random signs, so their number
+    # counts by its root
+    assert rel(vk, ref) < 2.3e-16 * 4 * (naux * nocc) ** .5
