@@ -64,7 +64,7 @@ struct GKItem {
     int nao, nocc, ksplit, ntile, s2;
     // split-BF16 (prec 2): workspace offsets of [side][FT hi, FT lo, R hi, R lo]
     void *b3[2][4];
-    long ldr, ldft;         // R row stride (split-BF16; FP64/FP32: 8 nocc), FT row stride
+    long ldr, ldft;         // R row stride (split-BF16; FP64/FP32: kcore::block_ld), FT row stride
     int bn3;                // split-BF16 step-1 tile width (kb3::pick_bn(ldr))
     int bn1;                // FP64/FP32 step-1 tile width (the plan's bn, or kcore::pick_bn(nocc))
     const void *tiles;      // FP64/FP32: the pair map's tiles, or NULL
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(G_THREADS, B == 64 ? 4 : 2) void gk_step2(const GKI
             ti = e.a / it.ntile;
             tj = e.a % it.ntile;
         }
-        const kcore::RShape y(nLb, it.nocc);
+        const kcore::RShape y(nLb, it.nocc, kcore::block_of(it.nL));
         const long nsteps = y.steps();
         const long s0 = nsteps * e.b / it.ksplit, s1 = nsteps * (e.b + 1) / it.ksplit;
         const T *rl = (const T *)(work + (size_t)it.rl);
@@ -464,8 +464,8 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
             }
             const bool two = x.fr != nullptr;
             const bool b3 = prec == MDF_PREC_BF16X3;
-            const long nL = b3 ? kcore::block_rows(x.naux, x.nao, (int)kcore::kb3::pad32(x.nocc), two, 4)
-                               : kcore::block_rows(x.naux, x.nao, x.nocc, two, elem);
+            const long nL = b3 ? kcore::block_rows(x.naux, x.nao, (int)kcore::kb3::pad32(x.nocc), two, true, 4)
+                               : kcore::block_rows(x.naux, x.nao, x.nocc, two, false, elem);
             kcore::KPlan kp = kcore::plan_k(x.naux, x.nao, x.nocc, two, nL, b3);
             for (int d = 0; d < x.n_dm; d++) {
                 GKItem g{};
@@ -497,7 +497,7 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
                     g.rl = (void *)0;
                     g.part = (double *)y.total;
                 } else {
-                    g.ldr = (long)kcore::RL * x.nocc;
+                    g.ldr = kcore::block_ld(kcore::block_of(kp.nL), x.nocc);
                     g.rl = (void *)(align_up(kp.r_words * elem, 256));
                     g.part = (double *)(align_up(kp.part_words * sizeof(double), 256));
                 }
@@ -622,7 +622,8 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
             auto s2cost = [&](const Tile &x) {
                 const GKItem &g = p->hk[x.item];
                 const long nLb = std::min(g.nL, g.naux - (long)x.c * g.nL);
-                return (prec == MDF_PREC_BF16X3 ? nLb * (g.ldr / b3::BK) : kcore::RShape(nLb, g.nocc).steps()) / g.ksplit;
+                return (prec == MDF_PREC_BF16X3 ? nLb * (g.ldr / b3::BK)
+                                                : kcore::RShape(nLb, g.nocc, kcore::block_of(g.nL)).steps()) / g.ksplit;
             };
             std::stable_sort(k2.begin() + s2, k2.end(),
                              [&](const Tile &x, const Tile &y) { return s2cost(x) > s2cost(y); });

@@ -20,6 +20,8 @@
 // packed cderi and the factors to FP32 on the way into LDS, runs both steps
 // on FP32 MFMA with FP32 accumulation and stores R in FP32 (the mixed-
 // precision SCF cycles); the cross-split sum and the output stay FP64.
+#include <algorithm>
+
 #include "mdf_common.h"
 #include "mdf_gemm.h"
 #include "mdf_kcore.h"
@@ -247,7 +249,7 @@ template <int B, typename T>
 void launch_step2(const KPlan &p, int nL, bool two, hipStream_t st, const T *rl, const T *rr, int nao, int nocc,
                   double *part, long part_stride, int beta) {
     const dim3 g2((unsigned)((long)p.ntiles_grid * p.ksplit));
-    const RShape y(nL, nocc);
+    const RShape y(nL, nocc, block_of(p.nL));
     if (two)
         hipLaunchKernelGGL((k_step2<B, false, T>), g2, dim3(G_THREADS), 0, st, rl, rr, nao, y, p.ntile, p.ntiles_grid,
                            p.ksplit, part, part_stride, beta);
@@ -284,7 +286,7 @@ int run_k(const KPlan &p, const Src *cderi, long naux, long ld, const int *pair_
     if (pair_tiles)
         for (int side = 0; side < (two ? 2 : 1); side++)
             if (int rc = pack_factor<T>(p, st, side ? fr : fl, ldf, nao, nocc, fp[side])) return rc;
-    const long ldr = (long)RL * nocc, strideB = (long)nao * ldr;
+    const long ldr = block_ld(block_of(p.nL), nocc), strideB = (long)nao * ldr;
     const long part_stride = (long)nao * nao;
     for (long L0 = 0; L0 < naux; L0 += p.nL) {
         const int nL = (int)(naux - L0 < p.nL ? naux - L0 : p.nL);
@@ -374,8 +376,8 @@ static size_t k_workspace(const KPlan &p, bool two, size_t elem, size_t pack) {
 
 // Aux rows per pass and workspace of one call for any precision.
 static long k_rows_rule(long naux, int nao, int nocc, bool two, int prec) {
-    if (prec == MDF_PREC_BF16X3) return block_rows(naux, nao, (int)kb3::pad32(nocc), two, 4);
-    return block_rows(naux, nao, nocc, two, prec == MDF_PREC_FP32 ? sizeof(float) : sizeof(double));
+    if (prec == MDF_PREC_BF16X3) return block_rows(naux, nao, (int)kb3::pad32(nocc), two, true, 4);
+    return block_rows(naux, nao, nocc, two, false, prec == MDF_PREC_FP32 ? sizeof(float) : sizeof(double));
 }
 static size_t k_bytes(long naux, int nao, int nocc, bool two, int prec, long rows, bool pairs) {
     KPlan p = plan_k(naux, nao, nocc, two, rows, prec == MDF_PREC_BF16X3);
@@ -386,7 +388,7 @@ static size_t k_bytes(long naux, int nao, int nocc, bool two, int prec, long row
 
 static size_t k_workspace_rule(long naux, int nao, int nocc, bool two, int prec, long max_block_rows, bool pairs) {
     long rows = k_rows_rule(naux, nao, nocc, two, prec);
-    if (max_block_rows > 0 && max_block_rows < rows) rows = max_block_rows;
+    if (max_block_rows > 0) rows = std::min(rows, rows_within(naux, max_block_rows, prec == MDF_PREC_BF16X3));
     return k_bytes(naux, nao, nocc, two, prec, rows, pairs);
 }
 

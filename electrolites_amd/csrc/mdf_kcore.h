@@ -208,7 +208,8 @@ __device__ __forceinline__ void step1_pairs_tile(const Src *__restrict__ c, long
 
 // ---------------------------------------------------------------- step 2
 // The transformed blocks: the occupied columns of 8 aux rows side by side,
-// R[L / 8][i][(L % 8) nocc + k], row stride ldr = 8 nocc.  Step 2's reduction
+// R[L / 8][i][(L % 8) nocc + k], row stride ldr = 8 nocc (of a pass of fewer
+// rows, one block as wide as those).  Step 2's reduction
 // runs over a block's 8 nocc columns in K-steps of 16 (one aux row at a time
 // it computed nocc rounded up to 16: 96 columns for 81, 64 for 50).
 constexpr int RL = tiles::NL;
@@ -221,12 +222,19 @@ inline long max_cols(int nao) {
     return packed < 1L << 22 ? packed : 1L << 22;
 }
 
-// Columns of a block's row that hold values: fewer in a pass's last block.
+// Aux rows a block holds in passes of nL rows, and its row stride (whole 16-byte
+// pieces of float).
+__host__ __device__ __forceinline__ int block_of(long nL) { return nL < RL ? (int)nL : RL; }
+__host__ __device__ __forceinline__ long block_ld(int rl, int nocc) { return ((long)rl * nocc + 3) / 4 * 4; }
+
+// A pass of nL aux rows in blocks of rl (block_of the plan's passes, in the
+// last, shorter one too): columns of a block's row that hold values, fewer in
+// the last block.
 struct RShape {
-    int nocc, ldr, kchunks, nfull, lastcols;
-    __host__ __device__ __forceinline__ RShape(long nL, int nocc_)
-        : nocc(nocc_), ldr(RL * nocc_), kchunks((RL * nocc_ + G_BK - 1) / G_BK), nfull((int)(nL / RL)),
-          lastcols((int)(nL % RL) * nocc_) {}
+    int ldr, cols, kchunks, nfull, lastcols;
+    __host__ __device__ __forceinline__ RShape(long nL, int nocc, int rl)
+        : ldr((int)block_ld(rl, nocc)), cols(rl * nocc), kchunks((cols + G_BK - 1) / G_BK), nfull((int)(nL / rl)),
+          lastcols((int)(nL % rl) * nocc) {}
     __host__ __device__ __forceinline__ long steps() const {
         return (long)nfull * kchunks + (lastcols + G_BK - 1) / G_BK;
     }
@@ -272,7 +280,7 @@ struct TransformedLoader {
 #pragma unroll
             for (int e = 0; e < EPV; e++) r[q * EPV + e] = x.v[e];
         }
-        left = (b < y.nfull ? y.ldr : y.lastcols) - kc * G_BK;
+        left = (b < y.nfull ? y.cols : y.lastcols) - kc * G_BK;
         if (++kc == y.kchunks) {
             kc = 0;
             ++b;
@@ -475,16 +483,25 @@ inline size_t k_block_bytes() {
     return K_BLOCK_BYTES;
 }
 
-inline long block_rows(long naux, int nao, int nocc, bool two, size_t elem) {
-    const size_t per_row = (size_t)nao * nocc * elem * (two ? 2 : 1);
-    long r = per_row ? (long)(k_block_bytes() / per_row) : naux;
-    if (r > naux) r = naux;
-    if (r > RL && r < naux) r = r / RL * RL;
+// The most of naux aux rows whose transformed blocks take no more than cap rows'
+// space: all of them, whole blocks, or one block of fewer rows (at least one).
+// Split BF16's rows stand alone (b3): no space goes to a last block's missing ones.
+inline long rows_within(long naux, long cap, bool b3) {
+    const long all = b3 || naux < RL ? naux : (naux + RL - 1) / RL * RL;
+    const long r = cap >= all ? naux : cap >= RL ? cap / RL * RL : cap;
     return r < 1 ? 1 : r;
 }
 
+inline long block_rows(long naux, int nao, int nocc, bool two, bool b3, size_t elem) {
+    const size_t per_row = (size_t)nao * nocc * elem * (two ? 2 : 1);
+    return rows_within(naux, per_row ? (long)(k_block_bytes() / per_row) : naux + RL, b3);
+}
+
 // Words of one factor's transformed blocks of a pass of nL aux rows.
-inline size_t r_words(long nL, int nao, int nocc) { return (size_t)((nL + RL - 1) / RL) * nao * RL * nocc; }
+inline size_t r_words(long nL, int nao, int nocc) {
+    const int rl = block_of(nL);
+    return (size_t)((nL + rl - 1) / rl) * nao * block_ld(rl, nocc);
+}
 
 // b3: the split-BF16 kernels' plan (128-wide step-2 tiles).
 inline KPlan plan_k(long naux, int nao, int nocc, bool two, long max_rows, bool b3) {
@@ -500,7 +517,7 @@ inline KPlan plan_k(long naux, int nao, int nocc, bool two, long max_rows, bool 
     p.s2 = !b3 && S2_64_COST * tiles(64) * 64 * 64 < (double)tiles(128) * 128 * 128 ? 64 : 128;
     p.ntile = (nao + p.s2 - 1) / p.s2;
     p.ntiles_grid = tiles(p.s2);
-    const long nsteps = b3 ? p.nL * ((nocc + 31) / 32) : RShape(p.nL, nocc).steps();
+    const long nsteps = b3 ? p.nL * ((nocc + 31) / 32) : RShape(p.nL, nocc, block_of(p.nL)).steps();
     p.ksplit = pick_ksplit(p.ntiles_grid, nsteps, nao, (p.s2 == 64 ? 4 : 2) * cu_count() / N_XCD,
                            b3 ? 3e-6 : 1.5e-6);
     p.bn = pick_bn(nocc);

@@ -502,7 +502,7 @@ def _vk(cderi, lay, fl, fr, precision='fp64'):
     two = fr is not None
     elem = 8 if prec == 0 else 4
     per_row = nao * nocc * elem * (2 if two else 1)
-    rows = max(1, min(naux, K_WORKSPACE_BYTES // max(per_row, 1)))
+    rows = max(1, K_WORKSPACE_BYTES // max(per_row, 1))
     # the library cuts naux into passes by shape (the grouped launch cuts the
     # same way); K_WORKSPACE_BYTES can only shorten them
     tiles = lay.tiles()
@@ -543,7 +543,7 @@ def _jk_blocked(dfobj, cderi, lay, dms3, hermi, with_j, fl, fr, precision, block
         tiles = lay.tiles()
         nocc, two = fl.shape[-1], fr is not None
         per_row = nao * nocc * (8 if prec == 0 else 4) * (2 if two else 1)
-        rows = max(1, min(blk_rows, K_WORKSPACE_BYTES // max(per_row, 1)))
+        rows = max(1, K_WORKSPACE_BYTES // max(per_row, 1))
         kbytes = _lib.query(_k_workspace(tiles), blk_rows, nao, nocc, int(two), prec, rows)
     nbytes = max(jbytes, kbytes)
     if blocks is None:

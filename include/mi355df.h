@@ -103,9 +103,10 @@ int mdf_j_vj(const void *B, int dtype, long naux, long width, long ld, const dou
  *   only narrow mode is FP32 *storage* widened before arithmetic
  *   (electrolites/_dffp32.py:166-196).
  * The aux rows are transformed in passes of at most 8 GiB of transformed
- * blocks (a function of naux, nao, nocc, the factor count and prec only);
- * max_block_rows > 0 lowers that bound for the workspace query, and a
- * smaller workspace makes mdf_get_k use shorter passes.
+ * blocks (a function of naux, nao, nocc, the factor count and prec only; one
+ * aux row at least, whole blocks of 8 from 8 on); max_block_rows > 0 lowers
+ * that bound to so many rows' space for the workspace query, and a smaller
+ * workspace makes mdf_get_k use shorter passes.
  */
 size_t mdf_get_k_workspace(long naux, int nao, int nocc, int two_factors, int prec,
                            long max_block_rows);

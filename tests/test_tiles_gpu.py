@@ -305,3 +305,20 @@ def test_k_rows_beyond_32_bits(monkeypatch, tiled, two, nocc):
     # naux nocc products a sum in any order; random signs, so their number
     # counts by its root
     assert rel(vk, ref) < 2.3e-16 * 4 * (naux * nocc) ** .5
+
+
+@pytest.mark.parametrize('prec', [0, 1])
+@pytest.mark.parametrize('two', [False, True])
+@pytest.mark.parametrize('nocc', [1, 3, 5, 18])
+def test_k_short_blocks(prec, two, nocc):
+    """Passes of one block of fewer than 8 aux rows, the last pass shorter
+    still, with rows of every remainder by the 16-byte pieces."""
+    nao, naux = 37, 17
+    cderi, rows, cols, addr, fl, fr = inputs(nao, naux, nocc, two)
+    pmap, buf = make_tiles(addr, nao)
+    ref = exact_k(cderi, rows, cols, nao, fl, fr)
+    tol = 2.3e-16 * (nao + naux * nocc) if prec == 0 else 1.2e-7 * (nao + naux * nocc) ** .5
+    for nrow in (1, 2, 3, 5, 7, 8, 9):
+        for tiles in (None, buf):
+            print(f'k short blocks prec {prec} two {two} nocc {nocc} rows {nrow} tiled {tiles is not None}', flush=True)
+            assert rel(get_k(cderi, pmap, tiles, nao, fl, fr, prec, nrow), ref) < tol
