@@ -227,14 +227,24 @@ inline long max_cols(int nao) {
 __host__ __device__ __forceinline__ int block_of(long nL) { return nL < RL ? (int)nL : RL; }
 __host__ __device__ __forceinline__ long block_ld(int rl, int nocc) { return ((long)rl * nocc + 3) / 4 * 4; }
 
+// FP32 step 2 adds its MFMA accumulators into an FP64 shadow every S2_FLUSH
+// K-steps of one aux row's columns rounded up to 16 (at nocc = 81, 32 steps of
+// 13.5 products on average), so the rounding error of the long (L, k) reduction
+// grows with the flush length, not with naux * nocc.
+constexpr int S2_FLUSH = 32;
+
 // A pass of nL aux rows in blocks of rl (block_of the plan's passes, in the
 // last, shorter one too): columns of a block's row that hold values, fewer in
-// the last block.
+// the last block; and the K-steps, of 16 products each here, between two
+// flushes.
 struct RShape {
-    int ldr, cols, kchunks, nfull, lastcols;
+    int ldr, cols, kchunks, nfull, lastcols, flush;
     __host__ __device__ __forceinline__ RShape(long nL, int nocc, int rl)
         : ldr((int)block_ld(rl, nocc)), cols(rl * nocc), kchunks((cols + G_BK - 1) / G_BK), nfull((int)(nL / rl)),
-          lastcols((int)(nL % rl) * nocc) {}
+          lastcols((int)(nL % rl) * nocc) {
+        const long f = (long)S2_FLUSH * nocc / ((nocc + G_BK - 1L) / G_BK * G_BK);
+        flush = f > 1 ? (int)f : 1;
+    }
     __host__ __device__ __forceinline__ long steps() const {
         return (long)nfull * kchunks + (lastcols + G_BK - 1) / G_BK;
     }
@@ -302,10 +312,6 @@ struct TransformedLoader {
 
 constexpr double S2_64_COST = 1.25;
 constexpr int S2_B = 128;              // split-BF16 step-2 tile; FP64/FP32: KPlan::s2 (64 or 128)
-// FP32 step 2 adds its MFMA accumulators into an FP64 shadow every S2_FLUSH
-// K-steps (S2_FLUSH * 16 products per element), so the rounding error of the
-// long (L, k) reduction grows with the flush length, not with naux * nocc.
-constexpr int S2_FLUSH = 32;
 
 // One B x B output tile (i0, j0) of step 2 over the K-steps [s0, s1) of the
 // (block, chunk) reduction; writes (beta = 0) or adds (beta = 1) into o.
@@ -332,11 +338,11 @@ __device__ __forceinline__ void step2_tile(const T *__restrict__ Rl, const T *__
     } else {
         Acc<S::MI, S::NI, double> sum;
         sum.zero();
-        for (long s = s0; s < s1; s += S2_FLUSH) {
+        for (long s = s0; s < s1; s += y.flush) {
             acc.zero();
             // the loaders advance in place, so consecutive calls continue the
             // reduction where the previous one stopped
-            gemm_mainloop<B, B>(la, lb, (int)min((long)S2_FLUSH, s1 - s), lds, acc);
+            gemm_mainloop<B, B>(la, lb, (int)min((long)y.flush, s1 - s), lds, acc);
 #pragma unroll
             for (int a = 0; a < S::MI; a++)
 #pragma unroll

@@ -310,3 +310,39 @@ def test_ri_j_without_cderi(chunk_bytes):
     vj0 = dfj.get_j(ns, hermi=0)
     rj0, _ = fastdf.get_jk(df, ns, hermi=0, with_k=False)
     assert rel(vj0, rj0) < 1e-12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('nocc', [1, 5, 9])
+def test_fp32_step2_flush_length(nocc):
+    """FP32 step 2 keeps at most the products of 32 K-steps of one aux row
+    (32 nocc for nocc <= 16) in one FP32 sum: over positive values the error
+    is that of such sums added in FP64, taken here on the CPU one product
+    after the other, which rounds more often than the matrix instruction."""
+    import torch
+    from electrolites_amd import _dev, _lib
+    nao, naux = 48, 120000
+    rng = np.random.default_rng(nocc)
+    a = (rng.random((naux, nao)) + .5).astype(np.float32)
+    cderi = torch.from_numpy(a.astype(np.float64)).cuda()        # diagonal pairs only: R = a exactly
+    addr = torch.arange(nao, dtype=torch.int32, device='cuda') * (nao + 1)
+    pmap = torch.empty(nao * nao, dtype=torch.int32, device='cuda')
+    _lib.call('mdf_build_pair_map', _dev.ptr(addr), nao, nao, _dev.ptr(pmap), _dev.stream_ptr())
+    f = torch.ones((nao, nocc), dtype=torch.float64, device='cuda')
+    vk = torch.empty((nao, nao), dtype=torch.float64, device='cuda')
+    nb = _lib.query('mdf_get_k_workspace', naux, nao, nocc, 0, 1, 0)
+    work = torch.empty(nb, dtype=torch.uint8, device='cuda')
+    print(f'fp32 flush nocc {nocc}', flush=True)
+    _lib.call('mdf_get_k', _dev.ptr(cderi), 0, naux, nao, nao, _dev.ptr(pmap), nao, _dev.ptr(f), None, nocc, nocc, 1,
+              _dev.ptr(vk), nao, 0, _dev.ptr(work), nb, _dev.stream_ptr())
+    low = np.tril_indices(nao)
+    exact = nocc * (a.T.astype(np.float64) @ a.astype(np.float64))[low]
+    p = (a[:, low[0]].astype(np.float64) * a[:, low[1]]).reshape(-1, 32, len(low[0]))      # 32 aux rows a flush
+    s = np.zeros((p.shape[0], len(low[0])), dtype=np.float32)
+    for r in range(32):
+        for _ in range(nocc):
+            s = (s + p[:, r]).astype(np.float32)                  # a fused multiply-add rounds once
+    want = np.sqrt(np.mean((s.sum(axis=0, dtype=np.float64) / exact - 1) ** 2))
+    got = np.sqrt(np.mean((vk.cpu().numpy()[low] / exact - 1) ** 2))
+    print(f'  rms relative error {got:.2e}, of FP32 sums of {32 * nocc} products {want:.2e}')
+    assert got < 1.2 * want
