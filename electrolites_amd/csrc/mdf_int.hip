@@ -18,30 +18,47 @@ using namespace mdf;
 // ------------------------------------------------------------ side streams
 namespace {
 constexpr int MAX_DEVICES = 64;
+constexpr int SIDE_SETS = 8;       // callers' streams per device with side streams of their own
+struct SideSet {
+    hipStream_t caller, side[3];
+    bool made;
+    unsigned long used;            // when last taken
+};
 std::mutex g_side_mu;
-hipStream_t g_side[MAX_DEVICES][3];
-bool g_side_made[MAX_DEVICES];
+SideSet g_side[MAX_DEVICES][SIDE_SETS];
+unsigned long g_side_clock;
+
+// The side streams of a caller's stream: its own, or a set not used yet, or
+// the one unused for longest (the callers of a set wait for each other's
+// launches, so only more than SIDE_SETS of them at a time do).
+bool side_streams(int dev, hipStream_t st, hipStream_t (&out)[3]) {
+    std::lock_guard<std::mutex> lk(g_side_mu);
+    SideSet *set = nullptr;
+    for (SideSet &x : g_side[dev])
+        if (x.made && x.caller == st) set = &x;
+    if (!set) {
+        set = g_side[dev];
+        for (SideSet &x : g_side[dev])
+            if (x.used < set->used) set = &x;
+    }
+    if (!set->made)
+        for (hipStream_t &s : set->side)
+            if (!s && hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return false;
+    set->made = true;
+    set->caller = st;
+    set->used = ++g_side_clock;
+    for (int i = 0; i < 3; i++) out[i] = set->side[i];
+    return true;
+}
 }  // namespace
 
 mdf::ForkJoin::ForkJoin(hipStream_t st) : st_(st) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     int dev = 0;
     if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
-        hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) {
+        hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES || !side_streams(dev, st, side_)) {
         (void)hipGetLastError();
         return;                                      // everything on the caller's stream
-    }
-    {
-        std::lock_guard<std::mutex> lk(g_side_mu);
-        if (!g_side_made[dev]) {
-            for (hipStream_t &s : g_side[dev])
-                if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) {
-                    (void)hipGetLastError();
-                    return;
-                }
-            g_side_made[dev] = true;
-        }
-        for (int i = 0; i < SIDE; i++) side_[i] = g_side[dev][i];
     }
     if (hipEventCreateWithFlags(&ev_, hipEventDisableTiming) != hipSuccess || hipEventRecord(ev_, st_) != hipSuccess) {
         (void)hipGetLastError();

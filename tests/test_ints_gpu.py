@@ -47,3 +47,81 @@ def test_int3c2e(mol, nchunk):
     rows, cols = np.tril_indices(nao)
     ref = j3c[rows, cols, :].T
     assert rel(got, ref) < 1e-13
+
+
+def _metric_and_chunk(mol):
+    """A call that evaluates both integral tensors into buffers of its own on
+    the current stream, and those buffers."""
+    import torch
+    from electrolites_amd import ints
+    ao, aux = ints.DeviceBasis(mol.ao), ints.DeviceBasis(mol.aux)
+    t = ints.PairTasks(mol.ao, 0, mol.ao.nbas)
+    t.dev
+
+    def buffers():
+        return (torch.zeros((mol.naux, mol.naux), dtype=torch.float64, device='cuda'),
+                torch.zeros((mol.naux, t.p1 - t.p0), dtype=torch.float64, device='cuda'))
+
+    def run(out):
+        ints.int2c2e(aux, out[0])
+        ints.int3c2e_chunk(ao, aux, t, out[1], out[1].stride(0))
+        return out
+    return buffers, run
+
+
+@pytest.mark.gpu
+def test_callers_on_streams_of_their_own(mol):
+    """The integral classes spread over side streams of the caller's: more
+    callers' streams than there are sets of them, two threads at a time, each
+    behind work on its own stream and read by it afterwards, give the null
+    stream's values."""
+    import threading
+    import torch
+    buffers, run = _metric_and_chunk(mol)
+    ref = run(buffers())
+    torch.cuda.synchronize()
+    bad = []
+
+    def caller(streams):
+        x = torch.randn(1024, 1024, dtype=torch.float64, device='cuda')
+        for s in streams:
+            with torch.cuda.stream(s):
+                for _ in range(2):
+                    out = buffers()
+                    for b in out:
+                        b.fill_(float('nan'))
+                    x @ x
+                    for b in out:
+                        b.zero_()
+                    run(out)
+                    if not all(bool(torch.equal(a, b)) for a, b in zip(out, ref)):
+                        bad.append(s)
+    threads = [threading.Thread(target=caller, args=([torch.cuda.Stream() for _ in range(7)],)) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
+@pytest.mark.gpu
+def test_capturing_caller(mol):
+    """A captured call stays on its stream: every replay, with eager calls on
+    the same buffers between, gives the eager values."""
+    import torch
+    buffers, run = _metric_and_chunk(mol)
+    ref = run(buffers())
+    out = run(buffers())
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        run(out)
+    for rep in range(3):
+        for b in out:
+            b.fill_(float('nan'))
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, ref)), rep
+        run(out)
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, ref)), rep
