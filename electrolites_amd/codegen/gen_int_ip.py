@@ -216,7 +216,7 @@ def gen3(la, lb, lc, m_fixed=None):
     w('                const double ipq = 1.0 / (p + q), iq = 1.0 / q;')
     w('                const double qr = q * ipq, pr = p * ipq;')
     w('                const double x = p * qr * rpc2;')
-    w('                const double pref = TWO_PI_2P5 * ip_ * iq * sqrt(ipq) * fab * aux.coefs[oc + ic];')
+    w('                const double pref = TWO_PI_2P5 / (p * q * sqrt(p + q)) * fab * aux.coefs[oc + ic];')
     w(f'                double ru[{nroots}], rw[{nroots}];')
     w(f'                rys_roots<{nroots}>(x, ru, rw);')
     # the roots one at a time in the classes whose terms keep every Rys factor
@@ -321,7 +321,7 @@ def gen2(la, lc):
     w('            const double ipq = 1.0 / (p + q), iq = 1.0 / q;')
     w('            const double qr = q * ipq, pr = p * ipq;')
     w('            const double x = p * qr * rpc2;')
-    w('            const double pref = TWO_PI_2P5 * ip_ * iq * sqrt(ipq) * fab * aux.coefs[oc + ic];')
+    w('            const double pref = TWO_PI_2P5 / (p * q * sqrt(p + q)) * fab * aux.coefs[oc + ic];')
     w(f'            double ru[{nroots}], rw[{nroots}];')
     w(f'            rys_roots<{nroots}>(x, ru, rw);')
     w('#pragma unroll')
