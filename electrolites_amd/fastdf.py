@@ -399,7 +399,10 @@ def factorize_dm(dms, hermi):
         c = c.reshape(-1, nao, c.shape[-1])
         # the occupations decide the shape: read once (a boolean index on the
         # device reads back its count for every density and use)
-        occ_h = np.asarray(_dev.to_host(mo_occ), dtype=np.float64).reshape(c.shape[0], -1)
+        mo_occ = _dev.as_torch(mo_occ)
+        occ_h = mo_occ.detach().to('cpu', t.float64).numpy() if isinstance(mo_occ, t.Tensor) else \
+            np.asarray(mo_occ, dtype=np.float64)
+        occ_h = occ_h.reshape(c.shape[0], -1)
         occ = _dev.to_device(mo_occ).reshape(c.shape[0], -1)
         sel = occ_h > 0
         num = sel.sum(axis=1)
