@@ -400,8 +400,8 @@ extern "C" int mdf_grouped_plan_create(const mdf_jk_item *items, int nitems, int
     MDF_CHECK_ARG(items && nitems >= 0 && out && work_bytes, "mdf_grouped_plan_create: null argument");
     MDF_CHECK_ARG(prec == MDF_PREC_FP64 || prec == MDF_PREC_FP32 || prec == MDF_PREC_BF16X3,
                   "mdf_grouped_plan_create: precision %d", prec);
-    MDF_CHECK_ARG(bn == 0 || bn == 32 || bn == 64 || bn == 96 || bn == 128 || bn == 160 || bn == 192 || bn == 256 || bn == 320,
-                  "mdf_grouped_plan_create: bn %d not in {0,32,64,96,128,160,192,256,320}", bn);
+    MDF_CHECK_ARG(bn == 0 || bn == 64 || bn == 128 || bn == 160 || bn == 192 || bn == 256 || bn == 320,
+                  "mdf_grouped_plan_create: bn %d not in {0,64,128,160,192,256,320}", bn);
     for (int m = 0; m < nitems; m++)
         MDF_CHECK_ARG(items[m].cderi_dtype == items[0].cderi_dtype &&
                           (items[m].cderi_dtype == MDF_DTYPE_F64 || items[m].cderi_dtype == MDF_DTYPE_F32),
