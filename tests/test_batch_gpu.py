@@ -15,13 +15,18 @@ class FakeDF:
         self._cderi_idx = (pa.astype(np.int32), np.where(rows == cols)[0])
 
 
+#: items whose step 1 runs on pair tiles (a pair map and nao >= 112): AO
+#: counts off the groups of 16, aux rows off the blocks of 8, one and two factors
+TILED = [(150, 77, 21, 1, True, True), (133, 61, 100, 1, False, True), (250, 45, 33, 2, True, True)]
+
+
 def make_batch(seed=0):
     from electrolites_amd import fastdf
     rng = np.random.default_rng(seed)
     dfs, dms = [], []
     # (nao, naux, nocc, n_dm, tagged, screened)
     spec = [(37, 60, 5, 1, True, False), (72, 330, 15, 2, True, False), (129, 500, 40, 3, False, False),
-            (90, 150, 12, 1, True, True), (161, 610, 45, 1, True, False), (210, 260, 170, 1, True, False)]
+            (90, 150, 12, 1, True, True), (161, 610, 45, 1, True, False), (210, 260, 170, 1, True, False)] + TILED
     for nao, naux, nocc, n_dm, tagged, screened in spec:
         pa, _ = O.pair_addresses(nao)
         if screened:
@@ -36,6 +41,15 @@ def make_batch(seed=0):
             d = fastdf.tag_array(d, mo_coeff=np.array(cs), mo_occ=np.full((n_dm, nocc), 2.))
         dms.append(d)
     return dfs, dms
+
+
+@pytest.mark.gpu
+def test_batch_holds_tiled_items():
+    """What the tests below rely on: the last items of the batch have tiles,
+    the first ones none."""
+    dfs, dms = make_batch(0)
+    tiled = [e.tiles() is not None for e in _entries(dfs, dms)]
+    assert tiled == [False] * (len(dfs) - len(TILED)) + [True] * len(TILED)
 
 
 @pytest.mark.gpu
