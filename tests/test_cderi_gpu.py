@@ -242,6 +242,33 @@ def test_gemm_batched(transb, tri_a, lower_c):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize('M,K', [(1, 1), (160, 768), (131, 37), (300, 16)])
+@pytest.mark.parametrize('N', [127, 128, 129, 145, 159, 160, 161, 256, 257, 320, 321])
+def test_gemm_batched_widths(N, M, K):
+    """The column tiles that N picks (160 wide for 129 to 160, 320 for 257 to
+    320, else 128) at their edges, against numpy: padded rows of every
+    operand, A of its own, B shared, C read and not read."""
+    import torch
+    from electrolites_amd import _dev, _lib
+    rng = np.random.default_rng(N + M)
+    nb = 3
+    a, b = rng.standard_normal((nb, M, K + 3)), rng.standard_normal((K, N + 2))
+    c = rng.standard_normal((nb, M, N + 1))
+    A, B = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    for beta in (0., -1.5):
+        print(f'gemm_batched M {M} N {N} K {K} beta {beta}', flush=True)
+        C = torch.from_numpy(c.copy()).cuda()
+        if beta == 0.:
+            C[:, :, :N] = float('nan')
+        _lib.call('mdf_gemm_batched', 0, 0, 0, M, N, K, ctypes.c_double(.7), _dev.ptr(A), K + 3, M * (K + 3),
+                  _dev.ptr(B), N + 2, 0, ctypes.c_double(beta), _dev.ptr(C), N + 1, M * (N + 1), nb, None)
+        got = C.cpu().numpy()
+        ref = .7 * a[:, :, :K] @ b[:, :N] + (beta * c[:, :, :N] if beta else 0.)
+        assert rel(got[:, :, :N], ref) < 1e-13
+        assert np.array_equal(got[:, :, N:], c[:, :, N:])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize('transb', [0, 1])
 @pytest.mark.parametrize('init', [False, True])
 def test_gemm_pairs_batched(transb, init):

@@ -291,3 +291,48 @@ def test_packed_diagonal_positions(n):
     x, y = x + x.T, y + y.T
     w = np.where(a == b, 1., SQRT2)
     assert abs((w * x[a, b]) @ (w * y[a, b]) - (x * y).sum()) < 1e-12 * n * n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('dens', ['restricted', 'spin', 'spin-one-factor'])
+@pytest.mark.parametrize('storage', ['float64', 'float32'])
+def test_gradient_on_pair_tiles(monkeypatch, dens, storage):
+    """The gradient of a molecule whose exchange runs on pair tiles, in
+    several ragged blocks of aux rows and of weights, equals the one through
+    the pair map: the same sums in another order."""
+    import torch
+    from electrolites_amd import _lib, fastdf, fastdfgrad
+    from electrolites_amd.df import DF
+    from electrolites_amd.gto import water_cluster
+    mol = water_cluster(6, seed=2, li=True)
+    rng = np.random.default_rng(4)
+    nspin, nocc = (1, 31) if dens == 'restricted' else (2, 17)
+    c = np.stack([np.linalg.qr(rng.standard_normal((mol.nao, nocc)))[0] for _ in range(nspin)])
+    occ = np.full((nspin, nocc), 2. / nspin)
+    if dens == 'spin-one-factor':
+        occ[1, 9:] = 0.                       # fewer columns in the second spin
+    d = np.einsum('sik,sk,sjk->sij', c, occ, c)
+    dm = fastdf.tag_array(d[0] if nspin == 1 else d, mo_coeff=c[0] if nspin == 1 else c,
+                          mo_occ=occ[0] if nspin == 1 else occ)
+    assert mol.nao >= fastdf.TILES_MIN_NAO
+    row = 8 * mol.nao * nocc
+    monkeypatch.setattr(fastdfgrad, 'RBLOCK_BYTES', 101 * row)
+    monkeypatch.setattr(fastdfgrad, 'WBLOCK_BYTES', 75 * row)
+    names = []
+    call = _lib.call
+    monkeypatch.setattr(_lib, 'call', lambda name, *a: names.append(name) or call(name, *a))
+    got = []
+    for least in (fastdf.TILES_MIN_NAO, 10 ** 9):
+        monkeypatch.setattr(fastdf, 'TILES_MIN_NAO', least)
+        df = DF(mol)
+        df.build()
+        if storage == 'float32':
+            df._cderi = {k: v.float() for k, v in df._cderi.items()}
+        del names[:]
+        got.append(fastdfgrad.jk_energy_per_atom(df, dm, .7, .6))
+        tiled = least < 10 ** 9
+        assert ('mdf_k_step1_tiles' in names) == tiled and ('mdf_gemm_pairs_tiles' in names) == tiled
+        assert ('mdf_k_step1_lower' in names) != tiled and ('mdf_gemm_pairs_batched' in names) != tiled
+    # the terms of an atom's gradient cancel to about 1e-2 of their sizes, and
+    # atomic adds order the sums differently from run to run
+    assert rel(got[0], got[1]) < 1e-11
