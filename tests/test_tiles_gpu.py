@@ -322,3 +322,78 @@ def test_k_short_blocks(prec, two, nocc):
         for tiles in (None, buf):
             print(f'k short blocks prec {prec} two {two} nocc {nocc} rows {nrow} tiled {tiles is not None}', flush=True)
             assert rel(get_k(cderi, pmap, tiles, nao, fl, fr, prec, nrow), ref) < tol
+
+
+@pytest.mark.parametrize('prec', [0, 1, 2])
+@pytest.mark.parametrize('two', [False, True])
+def test_one_function(prec, two):
+    """nao 1: one pair, one group of one row and one column."""
+    import torch
+    print(f'one function prec {prec} two {two}', flush=True)
+    rng = np.random.default_rng(prec)
+    cderi = torch.from_numpy(rng.standard_normal((9, 1))).cuda()
+    addr = torch.zeros(1, dtype=torch.int32, device='cuda')
+    fl, fr = (torch.from_numpy(rng.standard_normal((1, 3))).cuda() for _ in range(2))
+    pmap, buf = make_tiles(addr, 1)
+    got = get_k(cderi, pmap, buf, 1, fl, fr if two else None, prec)
+    ref = (cderi ** 2).sum() * (fl * (fr if two else fl)).sum()
+    assert float((got - ref).abs()) < (1e-14, 1e-5, 1e-3)[prec] * float((cderi ** 2).sum() * (fl * fl).sum().sqrt() *
+                                                                        (fr * fr + fl * fl).sum().sqrt())
+
+
+def test_tiles_of_many_functions():
+    """The row order's widest form (from 8193 functions on): a permutation
+    of the rows, and in the map each pair once, at its row and column."""
+    import torch
+    nao = 8250
+    print(f'tiles nao {nao}', flush=True)
+    g = torch.Generator(device='cuda').manual_seed(1)
+    near = torch.randint(0, nao, (nao, 12), generator=g, device='cuda')
+    rows = torch.arange(nao, device='cuda').repeat_interleave(12)
+    near = near.reshape(-1)
+    pair = torch.unique(torch.cat([torch.maximum(rows, near) * nao + torch.minimum(rows, near),
+                                   torch.arange(nao, device='cuda') * (nao + 1)]))
+    _, buf = make_tiles(pair.to(torch.int32), nao)
+    w = buf[:buf.numel() // 4 * 4].view(torch.int32)
+    G, C = (nao + 15) // 16, (nao + 31) // 32 * 32 + 32
+    r = w[:16 * G]
+    assert torch.equal(torch.sort(r[:nao])[0], torch.arange(nao, dtype=torch.int32, device='cuda'))
+    assert bool((r[nao:] == -1).all())
+    o = (17 * G + 63) // 64 * 64
+    cols = w[o:o + G * C].reshape(G, C)
+    o = (o + G * C + 63) // 64 * 64
+    m = w[o:o + G * C * 16].reshape(G, C // 16, 16, 16).transpose(1, 2).reshape(G, 16, C)
+    gi, ii, kk = torch.nonzero(m >= 0, as_tuple=True)
+    i, j, p = r.reshape(G, 16)[gi, ii].long(), cols[gi, kk].long(), m[gi, ii, kk].long()
+    assert torch.equal(pair[p], torch.maximum(i, j) * nao + torch.minimum(i, j))
+    # every off-diagonal pair in both orders
+    assert torch.unique(i * nao + j).numel() == i.numel() == 2 * pair.numel() - nao
+
+
+def test_layout_tiles_on_another_stream():
+    """Tiles built on one stream behind queued work, used by a call on
+    another: the single-stream result."""
+    import torch
+    from electrolites_amd import fastdf
+    nao, naux, nocc = 150, 40, 20
+    cderi, rows, cols, addr, f, _ = inputs(nao, naux, nocc, False)
+    print('layout tiles on another stream', flush=True)
+
+    class DF:
+        def __init__(self):
+            self._cderi, self._cderi_idx = {0: cderi}, (addr, None)
+    dm = fastdf.tag_array(f @ f.T, mo_coeff=f, mo_occ=torch.ones(nocc, dtype=torch.float64, device='cuda'))
+    ref = fastdf.get_jk(DF(), dm, hermi=1)[1].clone()
+    df = DF()
+    lay = fastdf._layout(df, cderi, nao)
+    big = torch.randn(4096, 4096, device='cuda', dtype=torch.float64)
+    torch.cuda.synchronize()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(a):
+        for _ in range(4):
+            big @ big
+        assert lay.tiles() is not None
+    with torch.cuda.stream(b):
+        vk = fastdf.get_jk(df, dm, hermi=1)[1]
+    torch.cuda.synchronize()
+    assert torch.equal(vk, ref)

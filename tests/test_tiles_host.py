@@ -99,3 +99,23 @@ def test_a_layout_can_be_copied(fake, how, built):
         assert (got.map is None) == (lay.map is None) and got._tiles == {}
         if tiles is not None:
             assert lay.tiles() is tiles and got.tiles() is not tiles
+
+
+def test_sizes_the_tiles_do_not_hold(fake):
+    """From 2^29 pairs on no tiles are built."""
+    from electrolites_amd import fastdf
+    pmap = layout().map
+    assert fastdf.PairTiles(pmap, 32768, 1 << 29).buf is None
+    assert fastdf.PairTiles(pmap, 111, 6000).buf is None
+    assert 'mdf_build_pair_tiles' not in fake.log
+
+
+@pytest.mark.parametrize('nao,npairs', [(32768, 1 << 29), (32769, 100)])
+def test_the_library_refuses_them(nao, npairs):
+    """Checked before any device call."""
+    from electrolites_amd import _lib
+    p = 256                                   # a pointer that is not read
+    with pytest.raises(Exception, match='pair tiles hold up to'):
+        _lib.call('mdf_get_k_tiles', p, 0, 1, npairs, npairs, p, p, nao, p, None, 1, 1, 0, p, nao, 0, p, 1 << 40, None)
+    with pytest.raises(Exception, match='pair tiles hold up to'):
+        _lib.call('mdf_k_step1_tiles', p, 0, 1, npairs, npairs, p, 0, nao, p, 1, 1, p, 1, nao, p, 1 << 40, None)
