@@ -18,7 +18,7 @@ group) against FP64 MFMA peak; ``roofline_j`` is the J build against HBM
 bandwidth.  Per-call durations come from HIP events recorded on the stream
 the library launches on (torch's current stream).
 
-``serving`` (skipped with ``--no-serve``) is the north-star workload at one
+``serving`` (skipped with ``--no-serve``) is the serving workload at one
 rate: 48 DF-RHF energy requests over the molecule mix ((H2O)3-40, Li+ on
 half), Poisson arrivals at 8 req/s, served by the continuous-batching loop in
 mixed precision (split-BF16 K until the DIIS error is below 1e-5, FP64

@@ -447,7 +447,12 @@ inline int cu_count() {
 // rounds of resident workgroups (slots per XCD) each over its K-steps and
 // about 6 more to start and end, plus the partials written and read again
 // (nao^2 words each, 1.5e-6 K-steps a word; 3e-6 of split BF16's, which take
-// half the time).
+// half the time).  Against the best of 8, 16, 24, 32, 48, 64, 96, 128, 192 and
+// 256 splits, whole K at 48 to 768 functions: FP64 within 9 % (nao 192: 189 us
+// for 173; 768: 13.94 ms for 13.96), two factors within 4 % of the chosen
+// width's best, FP32 within 18 % (192: 143 us for 123; from 288 on 5 %), split
+// BF16 within 7 % (from 192 on 5 %); a fixed 32 loses up to 36 % (48 functions)
+// and 21 % (768).
 inline int pick_ksplit(int ntiles_grid, long nsteps, int nao, int slots, double word) {
     int best = N_XCD;
     double best_t = 1e300;
@@ -519,7 +524,11 @@ inline KPlan plan_k(long naux, int nao, int nocc, bool two, long max_rows, bool 
         return two ? n * n : n * (n + 1) / 2;
     };
     // 64-wide tiles cover a small result with less padding, at S2_64_COST
-    // times the time of a 128-wide tile's product per element
+    // times the time of a 128-wide tile's product per element: a whole FP64 K,
+    // one factor, 64 against 128 wide, each at its best split, at nao 72 29/37
+    // us, 96 42/47, 144 78/92, 192 173/206, 288 522/637, 384 1304/1319, 489
+    // 3293/3213, 576 5120/5330, 768 14972/13935; the rule takes 128 at 144,
+    // 249, 384, 489 and 768
     p.s2 = !b3 && S2_64_COST * tiles(64) * 64 * 64 < (double)tiles(128) * 128 * 128 ? 64 : 128;
     p.ntile = (nao + p.s2 - 1) / p.s2;
     p.ntiles_grid = tiles(p.s2);

@@ -43,7 +43,7 @@ __device__ __forceinline__ u64 wave_min63(u64 k) {
 // fewest partners and takes, until it holds 16, the row that adds the fewest
 // columns to the group's (ties: the most columns in common, then the lowest
 // index), and with it the AOs that follow it and add none (the rest of its
-// shell).  About one step per shell, each three barriers and two reads of the
+// shell).  About one step per shell, each four barriers and two reads of the
 // bit rows long, once per molecule.  A thread keeps its rows' counts in
 // registers.
 template <int GT, int ROWS>
