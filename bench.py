@@ -429,7 +429,9 @@ def bench_batch(args):
     fk = 0.
     for e in entries:
         two = 2 if e.fr is not None else 1
-        fk += e.n_dm * (2. * two * e.naux * e.nao * e.nao * e.nocc +
+        # step 1 over the stored pairs (each off-diagonal one twice), as the
+        # getjk workload counts it
+        fk += e.n_dm * (2. * two * e.naux * (2 * e.npairs - e.nao) * e.nocc +
                         (1. if two == 2 else .5) * 2 * e.naux * e.nocc * e.nao * e.nao)
     ndens = sum(e.n_dm for e in entries)
     out = {
