@@ -240,9 +240,13 @@ class _PairLayout:
 #: held while a layout's tiles are built (not a member of the layout, which
 #: is copied with the DF object that keeps it)
 _TILES_LOCK = threading.Lock()
-#: K's step 1 runs on pair tiles from this many functions: below it they
-#: gain nothing (a whole get_jk at nao 72: 257 us with them, 253 without; at
-#: 120: 342 and 352; at 192: 534 and 607) and the first call pays for them
+#: K's step 1 runs on pair tiles from this many functions.  Below it they gain
+#: nothing (a get_jk at nao 72: 131 us with them, 125 without; at 96: 139 and
+#: 135) and a layout's first call builds them (about 100 us).  From 112 to 128
+#: a single call is even (120: 159 and 158) and a grouped run gains (24 items of
+#: nao 120: 1.35 and 1.55 ms FP64, 1.06 and 1.33 split BF16); from 129, where
+#: the pair map's rows take a second tile, both do (129: 167 and 200; 192: 286
+#: and 353)
 TILES_MIN_NAO = 112
 
 
