@@ -662,7 +662,7 @@ extern "C" int mdf_gemm_batched(int transb, int tri_a, int lower_c, long M, long
         return launch_wide(m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch, st);
     // N in (128, 160]: one 160-wide column tile instead of two of 128 (the
     // gradient's F_r^T R_L at nocc 160, 32 waters: the whole term 56.5 -> 54.3
-    // ms)
+    // ms); up to 128 one tile of 128 does, and two of them cover (160, 256]
     if (!transb && tri_a == 0 && !lower_c && N > 128 && N <= 160)
         return launch_gemm<160, false, 0, false>(m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc,
                                                  strideC, batch, st);
