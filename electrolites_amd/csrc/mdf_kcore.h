@@ -219,7 +219,7 @@ constexpr int RL = tiles::NL;
 // at the functions that int32 pair addresses hold).
 inline long max_cols(int nao) {
     const long packed = (1L << 32) / (nao + 1L) - 320;
-    return packed < 1L << 22 ? packed : 1L << 22;
+    return packed < 1 ? 1 : packed < 1L << 22 ? packed : 1L << 22;
 }
 
 // Aux rows a block holds in passes of nL rows, and its row stride (whole 16-byte
